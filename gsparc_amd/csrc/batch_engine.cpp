@@ -180,7 +180,6 @@ sptc_status BatchEngine::plan(int B, const sptc_coo* X, const sptc_coo* Y, const
   bad_.reset(1);
   digest_.reset(2);
   scratch_.reset(4);
-  vsum_.reset(1);
   tmp_.reset(scan_tmp_count(n1) + 1);
   slices_.assign(B, {});
   sptc_status st = run(s, true);
@@ -506,7 +505,6 @@ sptc_status BatchEngine::run(hipStream_t s, bool P) {
     da.d.yvals = yv;
     da.d.row_cnt = c.row_cnt.get();
     da.d.out_off = c.out_off.get();
-    da.d.vsum = vsum_.get();
     da.grp_rows = c.grp_rows.get();
     da.grp_row0 = c.grp_row0.get();
     da.grp_inst = c.grp_inst.get();

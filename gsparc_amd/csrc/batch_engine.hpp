@@ -116,7 +116,6 @@ class BatchEngine {
   DevBuf<uint32_t> act_row_, dup_, bad_;
   DevBuf<U2> tmp_;
   DevBuf<uint64_t> digest_, scratch_;
-  DevBuf<double> vsum_;
   std::vector<uint64_t> iP_, iA_, iR_, ytoff_h_;
   std::vector<int> kyf_h_, acc_;
   std::vector<DenseClass> dense_;

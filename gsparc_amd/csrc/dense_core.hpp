@@ -193,8 +193,9 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
       ++o;
     }
   }
+  if (!a.vsum) return;  // batches sum their outputs instead
   for (int off = kWave / 2; off > 0; off >>= 1) vsum += __shfl_xor(vsum, off, kWave);
-  if (lane_id() == 0 && vsum != 0.0) atomicAdd(a.vsum, vsum);
+  if (lane_id() == 0 && vsum != 0.0) slot_add(a.vsum, vsum);
 }
 
 }  // namespace sptc

@@ -509,8 +509,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   // Dense applies when the column space (ranks of Y's free keys) fits an LDS
   // row and Y has no duplicate coordinates; automatically chosen when rows
   // are dense enough for the LDS row to pay off.
-  DevBuf<double> vsum(1);
-  fill_u64(reinterpret_cast<uint64_t*>(vsum.get()), 0, 1, s_);
+  DevBuf<double> vsum(kSumSlots);
+  fill_u64(reinterpret_cast<uint64_t*>(vsum.get()), 0, kSumSlots, s_);
   bool use_dense = false;
   if (o_.dense_accumulator >= 0 && ir && kyf <= kDenseMaxBits) {
     DevBuf<uint32_t> flag(1);
@@ -891,6 +891,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   } else {
     record(4);
   }
+  launch_fold_sums(vsum.get(), s_);
   SPTC_HIP(hipMemcpyAsync(&info.value_sum, vsum.get(), sizeof(double), hipMemcpyDeviceToHost,
                           s_));
   SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));

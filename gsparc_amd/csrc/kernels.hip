@@ -585,7 +585,7 @@ __global__ __launch_bounds__(kBlock) void k_expand(ExpandArgs a) {
   if (threadIdx.x == 0) {
     double t = 0;
     for (int w = 0; w < kBlock / kWave; ++w) t += s_sum[w];
-    atomicAdd(a.vsum, t);
+    slot_add(a.vsum, t);
   }
 }
 
@@ -963,6 +963,24 @@ void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t
       default: hipLaunchKernelGGL((k_dense_numeric<13, false>), g, b, 0, s, a); break;
     }
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_fold_sums(double* slots) {
+  __shared__ double red[kBlock / kWave];
+  double t = 0.0;
+  for (uint32_t i = threadIdx.x; i < kSumSlots; i += kBlock) t += slots[i];
+  for (int off = kWave / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, kWave);
+  if (lane_id() == 0) red[threadIdx.x / kWave] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double u = 0.0;
+    for (int w = 0; w < kBlock / kWave; ++w) u += red[w];
+    slots[0] = u;
+  }
+}
+
+void launch_fold_sums(double* slots, hipStream_t s) {
+  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kBlock), 0, s, slots);
 }
 
 // Any two equal adjacent keys in a sorted array (duplicate coordinates).

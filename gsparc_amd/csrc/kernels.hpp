@@ -76,7 +76,7 @@ struct ExpandArgs {
   const uint32_t* ycol;
   uint64_t* hist;
   int passes;
-  double* vsum;
+  double* vsum;  // [kSumSlots]
   uint32_t remap;  // XCD-contiguous tile order (set by launch_expand)
   // big-row tiles count the first pass's digits at this column shift
   // (set by launch_expand_items from the plan)
@@ -98,7 +98,7 @@ struct DenseArgs {
   uint32_t* out_row;
   uint64_t* out_col;
   float* out_val;
-  double* vsum;
+  double* vsum;                // [kSumSlots] sum of the products (may be NULL)
 };
 
 constexpr int kDenseMaxBits = 13;  // dense LDS rows up to 8192 slots
@@ -126,6 +126,8 @@ inline bool dense_pays(uint64_t ir, uint64_t rows, uint64_t active, uint64_t slo
 bool dense_ordered();
 void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
 void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
+// slots[0] = sum of the kSumSlots slots, added in a fixed order.
+void launch_fold_sums(double* slots, hipStream_t s);
 void launch_any_dup(const uint64_t* keys, uint64_t n, uint32_t* flag, hipStream_t s);
 void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s);
 

@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kBlock) void k_expand_items(ExpandArgs a,
   if (threadIdx.x == 0) {
     double t = 0;
     for (int w = 0; w < kBlock / kWave; ++w) t += s_sum[w];
-    atomicAdd(a.vsum, t);
+    slot_add(a.vsum, t);
   }
 }
 

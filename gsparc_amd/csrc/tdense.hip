@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kBlock) void k_tdense(TDenseArgs a) {
   }
   if constexpr (NUM) {
     for (int d = kWave / 2; d > 0; d >>= 1) vs += __shfl_xor(vs, d, kWave);
-    if (lane == 0 && vs != 0.0) atomicAdd(a.vsum, vs);
+    if (lane == 0 && vs != 0.0) slot_add(a.vsum, vs);
   } else {
     if (tid == 0) a.row_cnt[blockIdx.x] = (uint32_t)ocount;
   }

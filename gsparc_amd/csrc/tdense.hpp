@@ -26,7 +26,7 @@ struct TDenseArgs {
   uint32_t* out_row;
   uint64_t* out_col;
   float* out_val;
-  double* vsum;                // numeric: += sum of the products
+  double* vsum;                // numeric: [kSumSlots] += sum of the products
 };
 
 void launch_tdense_count(const TDenseArgs& a, uint64_t rows, hipStream_t s);
