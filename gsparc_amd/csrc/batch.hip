@@ -297,7 +297,7 @@ struct BReduceOp {
   NarrowRows nr;  // narrow form (keys unused)
 };
 
-// Same run detection and compensated summation as the plain reduce; the
+// Same run detection and FP64 sums as the plain reduce; the
 // chunk-local row maps back to a global row through the piece table.
 __global__ __launch_bounds__(kBlock) void k_breduce_emit(BReduceOp op, const U2* tile_offs) {
   __shared__ ReduceSmem sm;
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void k_bdense_count(BDenseArgs a) {
   if (threadIdx.x == 0) a.d.row_cnt[blockIdx.x] = t;
 }
 
-template <int EB, bool ORDERED>
+template <int EB>
 __global__ __launch_bounds__(kBlock) void k_bdense_numeric(BDenseArgs a) {
   constexpr int E = 1 << EB;
   __shared__ double s_acc[E];
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_bdense_numeric(BDenseArgs a) {
   bdense_row(a, blockIdx.x, r, in);
   const uint32_t g = find_seg(a.grp_rows, a.G, blockIdx.x);
   // instance-local row id
-  dense_row_numeric<EB, ORDERED>(a.d, a.d.row_act[r], a.d.row_act[r + 1], low_mask(in.kyf),
+  dense_row_numeric<EB>(a.d, a.d.row_act[r], a.d.row_act[r + 1], low_mask(in.kyf),
                         a.ytab + in.yt_off, (uint32_t)(blockIdx.x - a.grp_rows[g]),
                         a.d.out_off[blockIdx.x], s_acc, sm, &s_ja);
 }
@@ -628,18 +628,10 @@ void launch_bdense_count(const BDenseArgs& a, int eb, uint64_t rows, hipStream_t
 void launch_bdense_numeric(const BDenseArgs& a, int eb, uint64_t rows, hipStream_t s) {
   if (!rows) return;
   const dim3 g((uint32_t)rows), b(kBlock);
-  if (dense_ordered()) {
-    switch (eb) {
-      case 8: hipLaunchKernelGGL((k_bdense_numeric<8, true>), g, b, 0, s, a); break;
-      case 10: hipLaunchKernelGGL((k_bdense_numeric<10, true>), g, b, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_bdense_numeric<13, true>), g, b, 0, s, a); break;
-    }
-  } else {
-    switch (eb) {
-      case 8: hipLaunchKernelGGL((k_bdense_numeric<8, false>), g, b, 0, s, a); break;
-      case 10: hipLaunchKernelGGL((k_bdense_numeric<10, false>), g, b, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_bdense_numeric<13, false>), g, b, 0, s, a); break;
-    }
+  switch (eb) {
+    case 8: hipLaunchKernelGGL(k_bdense_numeric<8>, g, b, 0, s, a); break;
+    case 10: hipLaunchKernelGGL(k_bdense_numeric<10>, g, b, 0, s, a); break;
+    default: hipLaunchKernelGGL(k_bdense_numeric<13>, g, b, 0, s, a); break;
   }
 }
 

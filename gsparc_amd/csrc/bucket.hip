@@ -159,15 +159,14 @@ __global__ __launch_bounds__(kR) void k_bucket_scan(BucketArgs a) {
 template <int LM>
 struct EmitSmem {
   static constexpr int E = 1 << LM;
-  float2 slot[E];       // (sum, compensation) per column of the bucket
+  double slot[E];       // FP64 sum per column of the bucket
   uint32_t srank[E];    // staged outputs: column rank, value
   float sval[E];
   alignas(16) uint8_t seen[E];  // touched columns
 };
 
 // Adds the products of lanes `mine` (one bucket) to their columns' slots:
-// each column's products in lane (= product) order, one compensated step
-// each.  The lowest lane of each column (peers found by one ballot per
+// each column's products in lane (= product) order, in FP64.  The lowest lane of each column (peers found by one ballot per
 // column bit) reads the slot once, takes the others' values in lane order
 // and writes it back, so no two lanes touch one slot.
 template <int LM>
@@ -180,25 +179,22 @@ __device__ __forceinline__ void bucket_accumulate(EmitSmem<LM>& sm, uint64_t min
     peers &= bit ? m : ~m;
   }
   const bool lead = ((mine >> lane) & 1ull) && popc_below(peers) == 0;
-  float s = 0.f, cc = 0.f;
+  double s = 0.0;
   uint64_t rest = 0;
   if (lead) {
-    const float2 q = sm.slot[cl];
-    s = q.x;
-    cc = q.y;
-    kahan_step(s, cc, v);
+    s = sm.slot[cl] + (double)v;
     rest = peers & (peers - 1);
   }
   while (__ballot(rest != 0)) {
     const uint32_t src = rest ? (uint32_t)__builtin_ctzll(rest) : lane;
     const float x = __shfl(v, (int)src, kWave);
     if (rest) {
-      kahan_step(s, cc, x);
+      s += (double)x;
       rest &= rest - 1;
     }
   }
   if (lead) {
-    sm.slot[cl] = make_float2(s, cc);
+    sm.slot[cl] = s;
     sm.seen[cl] = 1;
   }
   wave_sync();
@@ -252,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void k_bucket_emit(BucketArgs a) {
   const uint32_t lmask = nslot - 1;
   // slots and marks start clear; every compaction clears what it takes
   for (uint32_t i = lane; i < nslot; i += kWave) {
-    sm.slot[i] = make_float2(0.f, 0.f);
+    sm.slot[i] = 0.0;
     sm.seen[i] = 0;
   }
   wave_sync();
@@ -282,10 +278,10 @@ __global__ __launch_bounds__(kBlock) void k_bucket_emit(BucketArgs a) {
       while (bits) {
         const uint32_t sl = first + (uint32_t)__builtin_ctz(bits);
         bits &= bits - 1;
-        const float2 acc = sm.slot[sl];
-        sm.slot[sl] = make_float2(0.f, 0.f);
+        const float acc = (float)sm.slot[sl];
+        sm.slot[sl] = 0.0;
         sm.srank[o] = (cur << L) | sl;
-        sm.sval[o] = acc.x + acc.y;
+        sm.sval[o] = acc;
         ++o;
       }
       staged += T;

@@ -166,20 +166,18 @@ __device__ __forceinline__ T block_excl_scan(T v, T* scratch, T* total) {
   return wave_off + inc - v;
 }
 
-// One Neumaier-compensated FP32 step: sum s, compensation c, the sum's
-// value is s + c (error ~2u independent of the count).  Every accumulator
-// takes this one step, so sums of the same values in the same order agree
-// bit for bit whichever kernel adds them.
-__device__ __forceinline__ void kahan_step(float& s, float& c, float x) {
-  const float t = s + x;
-  if (fabsf(s) >= fabsf(x)) c += (s - t) + x;
-  else c += (x - t) + s;
-  s = t;
-}
-struct KahanF32 {
-  float s = 0.f, c = 0.f;
-  __device__ __forceinline__ void add(float x) { kahan_step(s, c, x); }
-  __device__ __forceinline__ float value() const { return s + c; }
+// Every output is the FP64 sum of its FP32 products, rounded once to FP32, on
+// every path.  A product holds 24 bits, so the FP64 sum is exact while the
+// products of one output span less than 2^29 / count in magnitude: the order
+// of the adds then does not matter, and sums taken in product order
+// (reduce), by LDS atomics (dense rows) or by window agree bit for bit.
+// (One add and a conversion per product; the compensated FP32 pair that it
+// replaced took seven operations and, like it, an ordered pass to be
+// reproducible.)
+struct SumF64 {
+  double s = 0.0;
+  __device__ __forceinline__ void add(float x) { s += (double)x; }
+  __device__ __forceinline__ float value() const { return (float)s; }
 };
 
 // Value sums are added into kSumSlots device slots, a workgroup's own by its

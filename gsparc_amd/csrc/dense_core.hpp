@@ -5,13 +5,11 @@
 // active-nonzero order j, of each nonzero's matched Y segment -- are taken in
 // rounds of kBlock * G products: every thread loads its G products of the
 // round at once (strided, so loads coalesce and G of them are in flight per
-// thread), finds their owners j by binary search over the round's
-// act_prefix entries staged in LDS, and then the round's owners are applied
-// one after another with a barrier between owners.  Within one owner the
-// column ranks are distinct (no duplicate Y coordinates), so each rank's
-// products are added in j order -- the order of the ESC path's stable sort --
-// with the same Neumaier-compensated FP32 steps, which makes the two
-// accumulators bit-identical.
+// thread), finds their owners j by binary search over the round's act_prefix
+// entries staged in LDS, and adds each to its column's FP64 slot by an LDS
+// atomic.  FP64 sums do not depend on the order of the adds (SumF64 in
+// common.hpp says when exactly), so rows need no barrier between owners and
+// the outputs equal the ESC path's.
 #pragma once
 #include "kernels.hpp"
 
@@ -102,13 +100,7 @@ __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t
 
 // Numeric pass, then the touched slots in rank order to out_* at obase (row
 // id `row`, column ytab[rank] or rank).  `acc` holds E doubles of LDS.
-//   ORDERED: per slot a Neumaier-compensated FP32 sum in owner order (the
-//            round's owners applied one after another, a barrier between
-//            owners) -- bit-identical to the ESC path;
-//   else:    per slot an FP64 sum by LDS atomic add (no barriers), rounded
-//            once to FP32 -- within FP32 rounding of the exact sum, the
-//            order of concurrent adds not fixed.
-template <int EB, bool ORDERED>
+template <int EB>
 __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j0, uint64_t j1,
                                                   uint64_t cmask, const uint64_t* ytab,
                                                   uint32_t row, uint64_t obase, double* acc,
@@ -116,8 +108,6 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
   constexpr int E = DenseSmem<EB>::E;
   constexpr int S = E / kBlock;  // slots per thread in the compaction (1..32)
   static_assert(E >= kBlock && E % kBlock == 0, "dense row width");
-  float* s_sum = reinterpret_cast<float*>(acc);
-  float* s_cmp = s_sum + E;
   for (int i = threadIdx.x; i < E; i += kBlock) acc[i] = 0.0;
   for (int i = threadIdx.x; i < DenseSmem<EB>::W; i += kBlock) sm.bm[i] = 0;
   const uint64_t p0 = j0 < j1 ? a.act_prefix[j0] : 0;
@@ -127,53 +117,29 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
     uint64_t ja;
     const uint64_t pl = (pb + kDenseRound < p1 ? pb + kDenseRound : p1) - 1;
     const uint32_t m = dense_stage_owners(a.act_prefix, j0, j1, pb, pl, sm, s_ja, &ja);
-    uint32_t own[kDenseG], rank[kDenseG];
+    uint32_t rank[kDenseG];
     float val[kDenseG];
 #pragma unroll
     for (int g = 0; g < kDenseG; ++g) {
       const uint64_t p = pb + (uint64_t)g * kBlock + threadIdx.x;
-      own[g] = ~0u;
       rank[g] = 0;
       val[g] = 0.f;
       if (p < p1) {
         const uint32_t k = dense_owner(sm.pref, m, p);
         const uint64_t y = a.act_ypos[ja + k] + (p - sm.pref[k]);
-        own[g] = k;
         rank[g] = (uint32_t)(a.ykeys[y] & cmask);
         val[g] = a.act_xval[ja + k] * a.yvals[y];
       }
     }
-    if constexpr (!ORDERED) {
 #pragma unroll
-      for (int g = 0; g < kDenseG; ++g) {
-        if (own[g] != ~0u) {
-          vsum += (double)val[g];
-          atomicAdd(&acc[rank[g]], (double)val[g]);
-          atomicOr(&sm.bm[rank[g] >> 5], 1u << (rank[g] & 31));
-        }
+    for (int g = 0; g < kDenseG; ++g) {
+      if (pb + (uint64_t)g * kBlock + threadIdx.x < p1) {
+        vsum += (double)val[g];
+        atomicAdd(&acc[rank[g]], (double)val[g]);
+        atomicOr(&sm.bm[rank[g] >> 5], 1u << (rank[g] & 31));
       }
-      continue;  // the next round's staging starts with a barrier
     }
-    // owners of this round in order: the first is own of product pb, the
-    // last that of pl = min(pb + round, p1) - 1
-    const uint32_t klast = dense_owner(sm.pref, m, pl);
-    for (uint32_t k = 0; k <= klast; ++k) {
-#pragma unroll
-      for (int g = 0; g < kDenseG; ++g) {
-        if (own[g] == k) {
-          const float v = val[g];
-          const uint32_t r = rank[g];
-          vsum += (double)v;
-          const float smv = s_sum[r];
-          const float t = smv + v;
-          if (fabsf(smv) >= fabsf(v)) s_cmp[r] += (smv - t) + v;
-          else s_cmp[r] += (v - t) + smv;
-          s_sum[r] = t;
-          atomicOr(&sm.bm[r >> 5], 1u << (r & 31));
-        }
-      }
-      __syncthreads();
-    }
+    // (the next round's staging starts with a barrier)
   }
   __syncthreads();
   // Compaction in column order: thread t owns slots [t*S, t*S+S).
@@ -189,7 +155,7 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
       const uint32_t rk = first + e;
       a.out_row[obase + o] = row;
       a.out_col[obase + o] = ytab ? ytab[rk] : rk;
-      a.out_val[obase + o] = ORDERED ? s_sum[rk] + s_cmp[rk] : (float)acc[rk];
+      a.out_val[obase + o] = (float)acc[rk];
       ++o;
     }
   }

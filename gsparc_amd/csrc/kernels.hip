@@ -631,8 +631,7 @@ void launch_expand(const ExpandArgs& a, int rb, hipStream_t s) {
 
 // --------------------------------------------------------------------------
 // (d) Reduce by key over sorted products: one output per run of equal keys;
-// the run's values are summed in sorted (stable) order with compensated FP32
-// arithmetic (cub::DeviceReduce::ReduceByKey(Sum), contraction.cuh:512-537).
+// the run's values are summed in sorted (stable) order in FP64 (cub::DeviceReduce::ReduceByKey(Sum), contraction.cuh:512-537).
 struct ReduceOp {
   const uint64_t* keys;
   const float* vals;
@@ -897,17 +896,11 @@ void scan_narrow_tiles(uint64_t n, U2* tmp, hipStream_t s) {
 
 // --------------------------------------------------------------------------
 // (d) Dense per-row accumulation for small column spaces (E = 2^EB slots,
-// the rank space of Y's free keys).  One workgroup per X row.  The row's
-// active X nonzeros are taken in order; each one's Y segment is spread over
-// the threads and added into the dense LDS row with compensated FP32
-// arithmetic, a barrier separating segments, so every slot sums its products
-// in the same order as the ESC path's stable sort (Y free keys are distinct
-// within a segment when Y has no duplicate coordinates, which the caller
-// checks).  A first, symbolic kernel counts each row's touched slots so the
-// numeric kernel writes its outputs, in column order, straight to their
-// final place.
-
-
+// the rank space of Y's free keys).  One workgroup per X row: its products
+// are added into the row's FP64 LDS slots by atomics, whatever their order
+// (dense_core.hpp).  A first, symbolic kernel counts each row's touched slots
+// so the numeric kernel writes its outputs, in column order, straight to
+// their final place.
 template <int EB>
 __global__ __launch_bounds__(kBlock) void k_dense_count(DenseArgs a) {
   __shared__ DenseSmem<EB> sm;
@@ -917,25 +910,15 @@ __global__ __launch_bounds__(kBlock) void k_dense_count(DenseArgs a) {
   if (threadIdx.x == 0) a.row_cnt[blockIdx.x] = t;
 }
 
-template <int EB, bool ORDERED>
+template <int EB>
 __global__ __launch_bounds__(kBlock) void k_dense_numeric(DenseArgs a) {
   constexpr int E = 1 << EB;
   __shared__ double s_acc[E];
   __shared__ DenseSmem<EB> sm;
   __shared__ uint64_t s_ja;
   const uint64_t r = a.r0 + blockIdx.x;
-  dense_row_numeric<EB, ORDERED>(a, a.row_act[r], a.row_act[r + 1], a.fmask, a.ytab,
+  dense_row_numeric<EB>(a, a.row_act[r], a.row_act[r + 1], a.fmask, a.ytab,
                                  (uint32_t)r, a.out_off[blockIdx.x], s_acc, sm, &s_ja);
-}
-
-// Ordered (bit-identical to ESC) unless SPTC_DENSE_ORDER=atomic selects the
-// FP64 LDS-atomic accumulation.
-bool dense_ordered() {
-  static const bool ord = [] {
-    const char* e = getenv("SPTC_DENSE_ORDER");
-    return !(e && std::string(e) == "atomic");
-  }();
-  return ord;
 }
 
 void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s) {
@@ -950,18 +933,10 @@ void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s
 void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s) {
   if (!rows) return;
   const dim3 g((uint32_t)rows), b(kBlock);
-  if (dense_ordered()) {
-    switch (eb) {
-      case 8: hipLaunchKernelGGL((k_dense_numeric<8, true>), g, b, 0, s, a); break;
-      case 10: hipLaunchKernelGGL((k_dense_numeric<10, true>), g, b, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_dense_numeric<13, true>), g, b, 0, s, a); break;
-    }
-  } else {
-    switch (eb) {
-      case 8: hipLaunchKernelGGL((k_dense_numeric<8, false>), g, b, 0, s, a); break;
-      case 10: hipLaunchKernelGGL((k_dense_numeric<10, false>), g, b, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_dense_numeric<13, false>), g, b, 0, s, a); break;
-    }
+  switch (eb) {
+    case 8: hipLaunchKernelGGL(k_dense_numeric<8>, g, b, 0, s, a); break;
+    case 10: hipLaunchKernelGGL(k_dense_numeric<10>, g, b, 0, s, a); break;
+    default: hipLaunchKernelGGL(k_dense_numeric<13>, g, b, 0, s, a); break;
   }
 }
 

@@ -121,9 +121,6 @@ inline bool dense_pays(uint64_t ir, uint64_t rows, uint64_t active, uint64_t slo
          active <= kDenseMaxOwnersPerRow * rows;
 }
 
-// Dense numeric passes sum in owner order (bit-identical to ESC) unless the
-// FP64 LDS-atomic form is selected (SPTC_DENSE_ORDER=atomic).
-bool dense_ordered();
 void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
 void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
 // slots[0] = sum of the kSumSlots slots, added in a fixed order.

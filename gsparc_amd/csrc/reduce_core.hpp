@@ -1,7 +1,7 @@
 // Reduce-by-key tile core shared by the single-contraction and the batched
 // emit kernels (cub::DeviceReduce::ReduceByKey(Sum) semantics,
 // contraction.cuh:512-537): one output per run of equal sorted keys, the
-// run's values summed in sorted order with compensated FP32 arithmetic.
+// run's values summed in sorted order in FP64.
 #pragma once
 #include "scan.hpp"
 
@@ -80,7 +80,7 @@ __device__ __forceinline__ uint32_t reduce_tile(const uint64_t* __restrict__ key
     ov[q] = 0.f;
     if (run >= nruns) continue;
     const uint32_t j0 = sm.rs[run], j1 = sm.rs[run + 1];
-    KahanF32 acc;
+    SumF64 acc;
     uint32_t j = j0;
     for (; j + 4 <= j1; j += 4) {
       const float a = sm.v[j], b = sm.v[j + 1], c = sm.v[j + 2], d = sm.v[j + 3];
@@ -122,8 +122,8 @@ __device__ __forceinline__ uint32_t reduce_tile(const uint64_t* __restrict__ key
 // works alone (no workgroup barriers).  A product starts a run (a head)
 // when it is the first product, a row starts at it or its column differs
 // from its predecessor's, as the 64-bit keys (row << 32 | column) would
-// give.  Each run is summed in sorted order with compensated FP32
-// arithmetic by the lane holding its head; a run that continues past the
+// give.  Each run is summed in sorted order in FP64
+// by the lane holding its head; a run that continues past the
 // lane reads the later lanes' values from LDS and, past the tile, global
 // memory up to another column or its row's end.
 static_assert(kScanItems == 8, "wave tiles hold 8 products per lane");
@@ -277,16 +277,16 @@ __device__ __forceinline__ bool wave_tile_all_big(const NarrowRows& nr, uint64_t
   return nr.big && nr.big[r0] && (r0 + 1 >= nr.nrows || nr.rstart[r0 + 1] >= b + cnt);
 }
 
-// Compensated sums of the lane's products: res[j] = the running sum after
+// FP64 sums of the lane's products: res[j] = the running sum after
 // product j of the run it belongs to (runs restart at the heads); acc is
 // left holding the lane's last run.  FULL: all 8 products are in the tile.
 template <bool FULL>
 __device__ __forceinline__ void wave_lane_sums(uint32_t hm, uint32_t q0, uint32_t cnt,
-                                               const float (&val)[kScanItems], KahanF32& acc,
+                                               const float (&val)[kScanItems], SumF64& acc,
                                                float (&res)[kScanItems]) {
 #pragma unroll
   for (int j = 0; j < kScanItems; ++j) {
-    if ((hm >> j) & 1u) acc = KahanF32();
+    if ((hm >> j) & 1u) acc = SumF64();
     if (FULL || q0 + j < cnt) acc.add(val[j]);
     res[j] = acc.value();
   }
@@ -356,7 +356,7 @@ __device__ __forceinline__ uint32_t wave_tile_reduce(const NarrowRows& nr,
     vp[1] = f32x4{val[4], val[5], val[6], val[7]};
   }
   wave_sync();
-  KahanF32 acc;
+  SumF64 acc;
   float res[kScanItems];
   if (cnt == kWaveTile) wave_lane_sums<true>(hm, q0, cnt, val, acc, res);
   else wave_lane_sums<false>(hm, q0, cnt, val, acc, res);
