@@ -2,13 +2,14 @@
 #include "engine.hpp"
 
 #include "bucket.hpp"
-
+#include "rowacc.hpp"
 #include "tdense.hpp"
 
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -130,6 +131,16 @@ bool prefer_bucket_tail() {
     return e && std::string(e) == "buckets";
   }();
   return msd;
+}
+
+bool prefer_row_acc() {
+  static const bool acc = [] {
+    for (const char* v : {"SPTC_PROD_SORT", "SPTC_BIG_TAIL", "SPTC_SEG_RB", "SPTC_SEG_IPT",
+                          "SPTC_SEG_WIDE"})
+      if (getenv(v)) return false;
+    return true;
+  }();
+  return acc;
 }
 
 uint64_t count_products(const Operand& X, const Operand& Y, hipStream_t s) {
@@ -410,6 +421,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   // kyf: width of the column field inside Y keys and product keys from here
   // on; ytab maps a rank back to the Y free key when the field is a rank.
   int kyf = ynf;
+  uint64_t ranks = kyf < 32 ? 1ull << kyf : 0;  // columns below this
   const uint64_t* ykeys = Y.keys.get();
   DevBuf<uint64_t> ykeys_rank, ytab;
   DevBuf<uint32_t> ytab32;  // ytab as 32-bit words when Y free keys fit them
@@ -433,6 +445,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
                    s_);
       ykeys = ykeys_rank.get();
       kyf = yrb;
+      ranks = U;
       if (ynf <= 32) {
         ytab32.reset(U);
         launch_ycol(ytab.get(), U, 0xFFFFFFFFull, ytab32.get(), s_);
@@ -647,10 +660,6 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     res->chunks.push_back(std::move(oc));
   } else if (ir) {
     DevBuf<uint64_t> scratch(4);
-    launch_max_row(row_prod.get(), R, scratch.get(), s_);
-    SPTC_HIP(hipMemcpyAsync(host_u64_, scratch.get(), 8, hipMemcpyDeviceToHost, s_));
-    SPTC_HIP(hipStreamSynchronize(s_));
-    const uint64_t max_row = host_u64_[0];
     const uint64_t live = DevicePool::get().live_bytes();
     const uint64_t free_b = budget_ > live ? budget_ - live : 0;
     const uint64_t per_prod = 12 + SortWorkspace::bytes_per_key(10) + 1;
@@ -665,12 +674,21 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     // coarse granularity keeps the chunking identical across repeated calls
     if (cap > (1ull << 26)) cap &= ~((1ull << 26) - 1);
     cap = std::min<uint64_t>(cap, std::min<uint64_t>(ir, 4000000000ull));
-    if (cap < max_row) {
-      msg = "one X row's products exceed the memory budget";
-      return SPTC_ERR_OOM_BUDGET;
-    }
     const uint64_t rmax = kyf >= 32 ? (kyf >= 64 ? 1 : (1ull << (64 - kyf))) : (1ull << 32);
-    uint64_t r0 = 0;
+    if (cap >= ir && R <= rmax) {  // one chunk
+      bounds_r.push_back(R);
+      bounds_p.push_back(ir);
+      bounds_a.push_back(A);
+    } else {
+      launch_max_row(row_prod.get(), R, scratch.get(), s_);
+      SPTC_HIP(hipMemcpyAsync(host_u64_, scratch.get(), 8, hipMemcpyDeviceToHost, s_));
+      SPTC_HIP(hipStreamSynchronize(s_));
+      if (cap < host_u64_[0]) {
+        msg = "one X row's products exceed the memory budget";
+        return SPTC_ERR_OOM_BUDGET;
+      }
+    }
+    uint64_t r0 = bounds_r.back();
     while (r0 < R) {
       launch_chunk_end(row_prod.get(), row_act.get(), R, r0, rmax, cap, scratch.get(), s_);
       SPTC_HIP(hipMemcpyAsync(host_u64_, scratch.get(), 24, hipMemcpyDeviceToHost, s_));
@@ -699,19 +717,28 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     uint64_t chunk_cap = 0;
     for (size_t c = 1; c < bounds_p.size(); ++c)
       chunk_cap = std::max(chunk_cap, bounds_p[c] - bounds_p[c - 1]);
-    DevBuf<uint64_t> kA(chunk_cap);
-    DevBuf<float> vA(chunk_cap);
     uint64_t max_rows = 0;
     for (size_t c = 1; c < bounds_r.size(); ++c)
       max_rows = std::max(max_rows, bounds_r[c] - bounds_r[c - 1]);
-    DevBuf<U2> tmp(std::max(reduce_tmp_count(std::max(chunk_cap, max_rows)),
-                            narrow_tmp_count(chunk_cap)));
-    int rb_max = 8;
-    for (size_t c = 1; c < bounds_r.size(); ++c) {
-      const int b = mode_bits(bounds_r[c] - bounds_r[c - 1]) + kyf;
-      rb_max = std::max(rb_max, rb_ ? rb_ : choose_radix_bits(b));
-    }
-    ws_.ensure(chunk_cap, rb_max, s_);
+    // the product sort's buffers, allocated by the first chunk that takes it
+    DevBuf<uint64_t> kA;
+    DevBuf<float> vA;
+    DevBuf<U2> tmp;
+    DevBuf<uint32_t> trow;
+    auto sort_buffers = [&] {
+      if (kA.size()) return;
+      kA.reset(chunk_cap);
+      vA.reset(chunk_cap);
+      tmp.reset(std::max(reduce_tmp_count(std::max(chunk_cap, max_rows)),
+                         narrow_tmp_count(chunk_cap)));
+      trow.reset(2 * (narrow_tile_count(chunk_cap) + 1));
+      int rb_max = 8;
+      for (size_t c = 1; c < bounds_r.size(); ++c) {
+        const int b = mode_bits(bounds_r[c] - bounds_r[c - 1]) + kyf;
+        rb_max = std::max(rb_max, rb_ ? rb_ : choose_radix_bits(b));
+      }
+      ws_.ensure(chunk_cap, rb_max, s_);
+    };
     const uint64_t fmask = low_mask(kyf);
     // 32-bit column field of Y for the expansion (4 bytes per gathered key
     // instead of 8)
@@ -723,7 +750,36 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     // row-segmented product sort
     DevBuf<RowRange> rrange(1);
     RowSegPlan rseg;
-    DevBuf<uint32_t> trow(2 * (narrow_tile_count(chunk_cap) + 1));
+    // row accumulator (column spaces up to kRowAccMaxBits)
+    const bool rowacc = kyf > 0 && kyf <= kRowAccMaxBits && prefer_row_acc() && !partition_only;
+    RowAccPlan rplan;
+    RowAccArgs ra;
+    DevBuf<uint32_t> ydup, yfree32;
+    if (rowacc) {
+      ydup.reset(1);
+      launch_any_dup(Y.keys.get(), ny, ydup.get(), s_);
+      if (ytab.size() && ynf <= 32) {
+        yfree32.reset(ny);
+        launch_ycol(Y.keys.get(), ny, low_mask(ynf), yfree32.get(), s_);
+      }
+      ra.act_prefix = act_prefix.get();
+      ra.act_ypos = act_ypos.get();
+      ra.act_xval = act_xval.get();
+      ra.row_prod = row_prod.get();
+      ra.row_act = row_act.get();
+      ra.ny = ny;
+      ra.ycol = ycol.get();
+      ra.yvals = Y.vals.get();
+      ra.ykeys = Y.keys.get();
+      ra.yfmask = low_mask(ynf);
+      ra.yfree32 = ytab.size() ? yfree32.get() : ycol.get();
+      ra.ytab = ytab.size() ? ytab.get() : nullptr;
+      ra.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
+      ra.K = (uint32_t)ranks;
+      ra.short_max = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(ranks / 128, 256), kGroupHalf);
+      ra.ydup = ydup.get();
+      ra.vsum = vsum.get();
+    }
     // verbose: a progress line on stderr at least every 10 s of chunks
     const auto t_loop = std::chrono::steady_clock::now();
     auto t_log = t_loop;
@@ -735,116 +791,152 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       const uint64_t P0 = bounds_p[c - 1], P1 = bounds_p[c];
       const uint64_t n = P1 - P0;
       if (!n) continue;
-      const int bits = mode_bits(r1c - r0c) + kyf;
-      const int rb = rb_ ? rb_ : choose_radix_bits(bits);
-      const int passes = radix_passes(bits, rb);
-      ws_.ensure(n, rb, s_);
-      ws_.prepare(passes, s_);
-      // row-segmented sort when the column bits leave row bits to skip
-      const bool rowsort = kyf > 0 && kyf < bits && kyf <= 32 && prefer_row_sort();
-      if (rowsort) {
-        const uint64_t lrows = r1c - r0c;
-        RowRange* h = reinterpret_cast<RowRange*>(host_u64_ + 4);
-        h->ra = r0c;
-        h->rows = lrows;
-        h->lrow0 = 0;
-        h->out0 = 0;
-        SPTC_HIP(hipMemcpyAsync(rrange.get(), h, sizeof(RowRange), hipMemcpyHostToDevice, s_));
-        build_row_segments(rrange.get(), 1, lrows, row_prod.get(), kyf, &rseg, ws_, tmp.get(),
-                           s_, prefer_bucket_tail(), row_act.get());
+      bool done = false;
+      uint64_t out_n = 0;
+      if (rowacc) {
+        ra.r0 = r0c;
+        ra.rows = r1c - r0c;
+        done = rowacc_count(ra, n, bounds_a[c] - bounds_a[c - 1], o_.count_only, &rplan,
+                            host_total_, s_, &kt_);
+        out_n = rplan.outs;
       }
-      ExpandArgs ea;
-      ea.act_prefix = act_prefix.get();
-      ea.act_ypos = act_ypos.get();
-      ea.act_xval = act_xval.get();
-      ea.act_row = act_row.get();
-      ea.A0 = bounds_a[c - 1];
-      ea.A1 = bounds_a[c];
-      ea.P0 = P0;
-      ea.P1 = P1;
-      ea.r0 = (uint32_t)r0c;
-      ea.ykeys = ykeys;
-      ea.yvals = Y.vals.get();
-      ea.ynf = kyf;
-      ea.fmask = fmask;
-      ea.out_keys = kA.get();
-      ea.out_vals = vA.get();
-      ea.big_col = nullptr;
-      ea.big_val = nullptr;
-      ea.out_col32 = nullptr;
-      ea.ycol = ycol.size() ? ycol.get() : nullptr;
-      // narrow form: sorted columns land in kA's first 4n bytes
-      uint32_t* fcol = reinterpret_cast<uint32_t*>(kA.get());
-      // count-only runs sort the columns alone: no value is written or moved
-      const bool cols_only = rowsort && o_.count_only;
-      float* const pv = cols_only ? nullptr : vA.get();
-      float* const pv1 = cols_only ? nullptr : ws_.alt_vals.get();
-      if (rowsort) {
-        const NarrowTarget nt =
-            narrow_target(rseg, n, vA.get(), ws_.alt_keys.get(), ws_.alt_vals.get());
-        ea.big_col = nt.col;
-        ea.big_val = cols_only ? nullptr : nt.val;
-        ea.out_col32 = fcol;
-        ea.out_vals = pv;
-      }
-      ea.hist = ws_.hist.get();
-      const bool hist = sort_needs_histogram();
-      ea.passes = hist && passes <= kMaxFusedPasses ? passes : 0;
-      ea.vsum = vsum.get();
-      int tok = kt_.begin(s_);
-      if (rowsort) launch_expand_items(ea, rseg, ws_, s_);  // ycol is set (kyf <= 32)
-      else launch_expand(ea, rb, s_);
-      // matched Y (column, value) read; product written: column + value in
-      // the narrow form of a row-segmented sort, 64-bit key + value otherwise
-      kt_.end(tok, SPTC_K_EXPAND,
-              (rowsort ? (cols_only ? 12.0 : 16.0) : 24.0) * (double)n, s_);
-      bool alt = false;
-      NarrowRows nr{fcol, rowsort ? rseg.row_start() : nullptr, r1c - r0c, trow.get()};
-      // high-digit form: big rows are reduced by buckets, the narrow reduce
-      // takes the small rows
-      const bool buckets = rowsort && rseg.msd && rseg.nbig_rows > 0;
-      BucketArgs ba{};
-      if (buckets) {
-        nr.big = rseg.row_big();
-        ba.segs = rseg.bigseg.get();
-        ba.tiles = rseg.big.get();
-        ba.nsegs = rseg.nbig_rows;
-        ba.starts = ws_.rts_cnt.get();
-        ba.boff = ws_.rts_off.get();
-        ba.cols = fcol;
-        ba.vals = vA.get();
-        ba.bigrow = rseg.bigrow.get();
-        ba.low = kyf - rseg.rb;
-        ba.gshift = bucket_group_shift(n - rseg.nsmall, rseg.nbig_rows);
-        ba.tile_sums = tmp.get();
-        ba.r0 = r0c;
-        ba.ytab = ytab.size() ? ytab.get() : nullptr;
-        ba.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
-      }
-      if (rowsort) {
-        launch_tile_rows(rseg.row_start(), r1c - r0c, n, trow.get(), s_);
-        sort_row_segments(ws_, rseg, n, fcol, pv, ws_.alt_keys.get(), pv1, rseg.row_start(), s_,
-                          &kt_, SPTC_K_SORT_PROD, /*counted=*/true);
+      std::function<void(OutChunk&)> emit;
+      if (done) {
+        emit = [&](OutChunk& oc) {
+          rowacc_emit(ra, rplan, n, oc.row.get(), oc.col.get(), oc.val.get(), s_, &kt_);
+        };
       } else {
+        sort_buffers();
+        const int bits = mode_bits(r1c - r0c) + kyf;
+        const int rb = rb_ ? rb_ : choose_radix_bits(bits);
+        const int passes = radix_passes(bits, rb);
         ws_.ensure(n, rb, s_);
-        if (hist && passes > kMaxFusedPasses) histogram(ws_, kA.get(), n, passes, s_);
-        alt = sort_after_histogram(ws_, kA.get(), vA.get(), n, bits, s_, &kt_, SPTC_K_SORT_PROD);
-      }
-      const uint64_t* sk = alt ? ws_.alt_keys.get() : kA.get();
-      const float* sv = alt ? ws_.alt_vals.get() : vA.get();
-      tok = kt_.begin(s_);
-      if (rowsort) {
-        run_reduce_count_narrow(nr, n, tmp.get(), s_, /*scan=*/!buckets);
-        if (buckets) {
-          run_bucket_count(ba, s_);
-          scan_narrow_tiles(n, tmp.get(), s_);
+        ws_.prepare(passes, s_);
+        // row-segmented sort when the column bits leave row bits to skip
+        const bool rowsort = kyf > 0 && kyf < bits && kyf <= 32 && prefer_row_sort();
+        if (rowsort) {
+          const uint64_t lrows = r1c - r0c;
+          RowRange* h = reinterpret_cast<RowRange*>(host_u64_ + 4);
+          h->ra = r0c;
+          h->rows = lrows;
+          h->lrow0 = 0;
+          h->out0 = 0;
+          SPTC_HIP(hipMemcpyAsync(rrange.get(), h, sizeof(RowRange), hipMemcpyHostToDevice, s_));
+          build_row_segments(rrange.get(), 1, lrows, row_prod.get(), kyf, &rseg, ws_, tmp.get(),
+                             s_, prefer_bucket_tail(), row_act.get());
         }
-      } else {
-        run_reduce_count(sk, n, tmp.get(), s_);
+        ExpandArgs ea;
+        ea.act_prefix = act_prefix.get();
+        ea.act_ypos = act_ypos.get();
+        ea.act_xval = act_xval.get();
+        ea.act_row = act_row.get();
+        ea.A0 = bounds_a[c - 1];
+        ea.A1 = bounds_a[c];
+        ea.P0 = P0;
+        ea.P1 = P1;
+        ea.r0 = (uint32_t)r0c;
+        ea.ykeys = ykeys;
+        ea.yvals = Y.vals.get();
+        ea.ynf = kyf;
+        ea.fmask = fmask;
+        ea.out_keys = kA.get();
+        ea.out_vals = vA.get();
+        ea.big_col = nullptr;
+        ea.big_val = nullptr;
+        ea.out_col32 = nullptr;
+        ea.ycol = ycol.size() ? ycol.get() : nullptr;
+        // narrow form: sorted columns land in kA's first 4n bytes
+        uint32_t* fcol = reinterpret_cast<uint32_t*>(kA.get());
+        // count-only runs sort the columns alone: no value is written or moved
+        const bool cols_only = rowsort && o_.count_only;
+        float* const pv = cols_only ? nullptr : vA.get();
+        float* const pv1 = cols_only ? nullptr : ws_.alt_vals.get();
+        if (rowsort) {
+          const NarrowTarget nt =
+              narrow_target(rseg, n, vA.get(), ws_.alt_keys.get(), ws_.alt_vals.get());
+          ea.big_col = nt.col;
+          ea.big_val = cols_only ? nullptr : nt.val;
+          ea.out_col32 = fcol;
+          ea.out_vals = pv;
+        }
+        ea.hist = ws_.hist.get();
+        const bool hist = sort_needs_histogram();
+        ea.passes = hist && passes <= kMaxFusedPasses ? passes : 0;
+        ea.vsum = vsum.get();
+        int tok = kt_.begin(s_);
+        if (rowsort) launch_expand_items(ea, rseg, ws_, s_);  // ycol is set (kyf <= 32)
+        else launch_expand(ea, rb, s_);
+        // matched Y (column, value) read; product written: column + value in
+        // the narrow form of a row-segmented sort, 64-bit key + value otherwise
+        kt_.end(tok, SPTC_K_EXPAND,
+                (rowsort ? (cols_only ? 12.0 : 16.0) : 24.0) * (double)n, s_);
+        bool alt = false;
+        NarrowRows nr{fcol, rowsort ? rseg.row_start() : nullptr, r1c - r0c, trow.get()};
+        // high-digit form: big rows are reduced by buckets, the narrow reduce
+        // takes the small rows
+        const bool buckets = rowsort && rseg.msd && rseg.nbig_rows > 0;
+        BucketArgs ba{};
+        if (buckets) {
+          nr.big = rseg.row_big();
+          ba.segs = rseg.bigseg.get();
+          ba.tiles = rseg.big.get();
+          ba.nsegs = rseg.nbig_rows;
+          ba.starts = ws_.rts_cnt.get();
+          ba.boff = ws_.rts_off.get();
+          ba.cols = fcol;
+          ba.vals = vA.get();
+          ba.bigrow = rseg.bigrow.get();
+          ba.low = kyf - rseg.rb;
+          ba.gshift = bucket_group_shift(n - rseg.nsmall, rseg.nbig_rows);
+          ba.tile_sums = tmp.get();
+          ba.r0 = r0c;
+          ba.ytab = ytab.size() ? ytab.get() : nullptr;
+          ba.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
+        }
+        if (rowsort) {
+          launch_tile_rows(rseg.row_start(), r1c - r0c, n, trow.get(), s_);
+          sort_row_segments(ws_, rseg, n, fcol, pv, ws_.alt_keys.get(), pv1, rseg.row_start(), s_,
+                            &kt_, SPTC_K_SORT_PROD, /*counted=*/true);
+        } else {
+          ws_.ensure(n, rb, s_);
+          if (hist && passes > kMaxFusedPasses) histogram(ws_, kA.get(), n, passes, s_);
+          alt = sort_after_histogram(ws_, kA.get(), vA.get(), n, bits, s_, &kt_, SPTC_K_SORT_PROD);
+        }
+        const uint64_t* sk = alt ? ws_.alt_keys.get() : kA.get();
+        const float* sv = alt ? ws_.alt_vals.get() : vA.get();
+        tok = kt_.begin(s_);
+        if (rowsort) {
+          run_reduce_count_narrow(nr, n, tmp.get(), s_, /*scan=*/!buckets);
+          if (buckets) {
+            run_bucket_count(ba, s_);
+            scan_narrow_tiles(n, tmp.get(), s_);
+          }
+        } else {
+          run_reduce_count(sk, n, tmp.get(), s_);
+        }
+        kt_.end(tok, SPTC_K_REDUCE, (rowsort ? 4.0 : 8.0) * (double)n, s_);
+        out_n =
+            read_total(tmp.get() + (rowsort ? narrow_tile_count(n) : scan_tmp_count(n))).a;
+        emit = [&, rowsort, buckets, nr, ba, sk, sv, out_n](OutChunk& oc) {
+          const int tok = kt_.begin(s_);
+          if (rowsort) {
+            run_reduce_emit_narrow(nr, vA.get(), n, oc.row.get(), oc.col.get(), oc.val.get(), r0c,
+                                   ytab.size() ? ytab.get() : nullptr,
+                                   ytab32.size() ? ytab32.get() : nullptr, tmp.get(), s_);
+            if (buckets) {
+              BucketArgs b = ba;
+              b.out_row = oc.row.get();
+              b.out_col = oc.col.get();
+              b.out_val = oc.val.get();
+              run_bucket_emit(b, s_);
+            }
+          } else
+            run_reduce_emit(sk, sv, n, oc.row.get(), oc.col.get(), oc.val.get(), r0c, kyf, fmask,
+                            ytab.size() ? ytab.get() : nullptr, tmp.get(), s_);
+          kt_.end(tok, SPTC_K_REDUCE, (rowsort ? 8.0 : 12.0) * (double)n + 16.0 * (double)out_n,
+                  s_);
+        };
       }
-      kt_.end(tok, SPTC_K_REDUCE, (rowsort ? 4.0 : 8.0) * (double)n, s_);
-      const uint64_t out_n =
-          read_total(tmp.get() + (rowsort ? narrow_tile_count(n) : scan_tmp_count(n))).a;
       info.nnz += out_n;
       info.nchunks++;
       if (o_.verbose) {
@@ -870,22 +962,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       oc.row.reset(out_n);
       oc.col.reset(out_n);
       oc.val.reset(out_n);
-      tok = kt_.begin(s_);
-      if (rowsort) {
-        run_reduce_emit_narrow(nr, vA.get(), n, oc.row.get(), oc.col.get(), oc.val.get(), r0c,
-                               ytab.size() ? ytab.get() : nullptr,
-                               ytab32.size() ? ytab32.get() : nullptr, tmp.get(), s_);
-        if (buckets) {
-          ba.out_row = oc.row.get();
-          ba.out_col = oc.col.get();
-          ba.out_val = oc.val.get();
-          run_bucket_emit(ba, s_);
-        }
-      } else
-        run_reduce_emit(sk, sv, n, oc.row.get(), oc.col.get(), oc.val.get(), r0c, kyf, fmask,
-                        ytab.size() ? ytab.get() : nullptr, tmp.get(), s_);
-      kt_.end(tok, SPTC_K_REDUCE, (rowsort ? 8.0 : 12.0) * (double)n + 16.0 * (double)out_n,
-              s_);
+      emit(oc);
       res->chunks.push_back(std::move(oc));
     }
   } else {
@@ -894,7 +971,9 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   launch_fold_sums(vsum.get(), s_);
   SPTC_HIP(hipMemcpyAsync(&info.value_sum, vsum.get(), sizeof(double), hipMemcpyDeviceToHost,
                           s_));
-  SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));
+  host_u64_[0] = 0;
+  if (ws_.counters.size())  // no sort ran: no look-back to have failed
+    SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));
   record(5);
   SPTC_HIP(hipStreamSynchronize(s_));
   kt_.collect(res->kstats, SPTC_K_COUNT);
