@@ -820,7 +820,7 @@ sptc_status sptc_sort_pairs(uint64_t* keys, float* vals, uint64_t n, int32_t nbi
       SPTC_HIP(hipMemcpyAsync(vals, ws.alt_vals.get(), n * 4, hipMemcpyDeviceToDevice, s));
     }
     uint32_t err = 0;
-    SPTC_HIP(hipMemcpyAsync(&err, ws.err(), 4, hipMemcpyDeviceToHost, s));
+    if (ws.err()) SPTC_HIP(hipMemcpyAsync(&err, ws.err(), 4, hipMemcpyDeviceToHost, s));
     SPTC_HIP(hipStreamSynchronize(s));
     if (err) return fail(SPTC_ERR_INTERNAL, "look-back spin limit exceeded");
   } catch (const HipError& he) {

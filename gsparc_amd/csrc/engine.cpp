@@ -184,7 +184,7 @@ uint64_t count_products(const Operand& X, const Operand& Y, hipStream_t s) {
 
 Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o) {
   for (auto& e : ev_) SPTC_HIP(hipEventCreate(&e));
-  SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_total_), sizeof(U2) * 2, 0));
+  SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_total_), sizeof(U2) * 4, 0));
   SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_u64_), sizeof(uint64_t) * 8, 0));
   // The budget caps what this call holds at once, on top of what was
   // already live when it started.
@@ -222,6 +222,10 @@ double Engine::elapsed_ms(int a, int b) {
 
 U2 Engine::read_total(const U2* dev) {
   SPTC_HIP(hipMemcpyAsync(host_total_, dev, sizeof(U2), hipMemcpyDeviceToHost, s_));
+  return wait_total();
+}
+
+U2 Engine::wait_total() {
   SPTC_HIP(hipStreamSynchronize(s_));
   return host_total_[0];
 }
@@ -363,8 +367,8 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
     ws_.prepare(radix_passes(bits, rb), s_);
     if (sort_needs_histogram()) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
     const bool alt = sort_after_histogram(ws_, sorted.get(), payload.get(), n, bits, s_);
-    run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_);
-    U = read_total(tmp.get() + scan_tmp_count(n)).a;
+    run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_, host_total_);
+    U = wait_total().a;
     launch_yrank(key.get(), n, 64, ~0ull, uniq.get(), U, 0, rank->get(), s_);
     rbits = mode_bits(U);
     prev = true;
@@ -436,8 +440,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     const bool alt = sort_after_histogram(ws_, fk.get(), fv.get(), ny, ynf, s_);
     ytab.reset(ny);
     DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-    run_unique(alt ? ws_.alt_keys.get() : fk.get(), ny, ytab.get(), tmp.get(), s_);
-    const uint64_t U = read_total(tmp.get() + scan_tmp_count(ny)).a;
+    run_unique(alt ? ws_.alt_keys.get() : fk.get(), ny, ytab.get(), tmp.get(), s_, host_total_);
+    const uint64_t U = wait_total().a;
     const int yrb = mode_bits(U);
     if (yrb < ynf) {
       ykeys_rank.reset(ny);
@@ -456,28 +460,35 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   }
 
   // ---- (c) index match ---------------------------------------------------
-  DevBuf<uint64_t> tlo, thi, ukey, ustart;
+  // ydup / hdup: set when Y holds duplicate coordinates
+  DevBuf<uint64_t> tlo, ukey, ustart;
+  uint64_t* ydup = nullptr;
+  uint64_t* const hdup = &host_total_[3].a;
+  *hdup = 0;
   YTable tab;
   std::memset(&tab, 0, sizeof(tab));
   if (ncb <= kDirectBits) {
     const uint64_t K = 1ull << ncb;
-    tlo.reset(K);
-    thi.reset(K);
-    fill_u64(tlo.get(), 0, K, s_);
-    fill_u64(thi.get(), 0, K, s_);
-    launch_ytable_direct(ykeys, ny, kyf, K, tlo.get(), thi.get(), s_);
+    tlo.reset(2 * K + 1);  // the table and the duplicate flag, one fill
+    fill_u64(tlo.get(), 0, 2 * K + 1, s_);
+    ydup = tlo.get() + 2 * K;
+    launch_ytable_direct(ykeys, ny, kyf, K, tlo.get(), tlo.get() + K, s_, ydup, hdup);
     tab.direct = 1;
     tab.lo = tlo.get();
-    tab.hi = thi.get();
+    tab.hi = tlo.get() + K;
   } else {
     ukey.reset(ny + 1);
     ustart.reset(ny + 1);
     DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-    run_yunique(ykeys, ny, kyf, ukey.get(), ustart.get(), tmp.get(), s_);
+    tlo.reset(1);
+    ydup = tlo.get();
+    fill_u64(ydup, 0, 1, s_);
+    launch_any_dup(Y.keys.get(), ny, ydup, hdup, s_);
+    run_yunique(ykeys, ny, kyf, ukey.get(), ustart.get(), tmp.get(), s_, host_total_);
     tab.direct = 0;
     tab.ukey = ukey.get();
     tab.ustart = ustart.get();
-    tab.U = read_total(tmp.get() + scan_tmp_count(ny)).a;
+    tab.U = wait_total().a;
   }
   DevBuf<uint64_t> act_prefix(nx + 1), act_ypos(nx + 1), row_key(nx + 1), row_prod(nx + 1),
       row_act(nx + 1);
@@ -496,21 +507,14 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   {
     DevBuf<U2> tmp(scan_tmp_count(nx) + 1);
     int tok = kt_.begin(s_);
-    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_);
+    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_, host_total_);
     // keys read twice, plus the compacted active and row tables written
     kt_.end(tok, SPTC_K_MATCH, (double)nx * (16 + 24 + 24), s_);
-    tot = read_total(tmp.get() + scan_tmp_count(nx));
+    tot = wait_total();
   }
   const uint64_t ir = tot.a;
   const uint64_t A = tot.b >> 32;
   const uint64_t R = tot.b & 0xFFFFFFFFull;
-  host_u64_[0] = ir;
-  host_u64_[1] = A;
-  SPTC_HIP(hipMemcpyAsync(row_prod.get() + R, &host_u64_[0], 8, hipMemcpyHostToDevice, s_));
-  SPTC_HIP(hipMemcpyAsync(row_act.get() + R, &host_u64_[1], 8, hipMemcpyHostToDevice, s_));
-  SPTC_HIP(hipMemcpyAsync(act_prefix.get() + A, &host_u64_[0], 8, hipMemcpyHostToDevice, s_));
-  tlo.release();
-  thi.release();
   ukey.release();
   ustart.release();
   record(3);
@@ -526,11 +530,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   fill_u64(reinterpret_cast<uint64_t*>(vsum.get()), 0, kSumSlots, s_);
   bool use_dense = false;
   if (o_.dense_accumulator >= 0 && ir && kyf <= kDenseMaxBits) {
-    DevBuf<uint32_t> flag(1);
-    launch_any_dup(Y.keys.get(), ny, flag.get(), s_);
-    SPTC_HIP(hipMemcpyAsync(host_u64_, flag.get(), 4, hipMemcpyDeviceToHost, s_));
-    SPTC_HIP(hipStreamSynchronize(s_));
-    const bool dups = *reinterpret_cast<uint32_t*>(host_u64_) != 0;
+    const bool dups = *hdup != 0;  // (waited for with the match)
     const uint64_t E = 1ull << (kyf < 8 ? 8 : kyf);
     // count-only runs stay on ESC, whose expansion also yields the value sum
     if (!dups)
@@ -574,8 +574,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     int tok = kt_.begin(s_);
     launch_dense_count(da, eb, R, s_);
     kt_.end(tok, SPTC_K_DENSE, 8.0 * (double)ir, s_);
-    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_);
-    const uint64_t out_n = read_total(tmp.get() + scan_tmp_count(R)).a;
+    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, host_total_);
+    const uint64_t out_n = wait_total().a;
     info.nnz = out_n;
     info.nchunks = 1;
     if (!o_.count_only) {
@@ -629,8 +629,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       launch_tdense_count(ta, std::min(kRowsPerLaunch, R - b), s_);
     }
     kt_.end(tok, SPTC_K_DENSE, 4.0 * (double)ir, s_);
-    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_);
-    const uint64_t out_n = read_total(tmp.get() + scan_tmp_count(R)).a;
+    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, host_total_);
+    const uint64_t out_n = wait_total().a;
     info.nnz = out_n;
     info.nchunks = 1;
     // the whole output stays resident: one chunk
@@ -754,10 +754,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     const bool rowacc = kyf > 0 && kyf <= kRowAccMaxBits && prefer_row_acc() && !partition_only;
     RowAccPlan rplan;
     RowAccArgs ra;
-    DevBuf<uint32_t> ydup, yfree32;
+    DevBuf<uint32_t> yfree32;
     if (rowacc) {
-      ydup.reset(1);
-      launch_any_dup(Y.keys.get(), ny, ydup.get(), s_);
       if (ytab.size() && ynf <= 32) {
         yfree32.reset(ny);
         launch_ycol(Y.keys.get(), ny, low_mask(ynf), yfree32.get(), s_);
@@ -777,7 +775,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       ra.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
       ra.K = (uint32_t)ranks;
       ra.short_max = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(ranks / 128, 256), kGroupHalf);
-      ra.ydup = ydup.get();
+      ra.ydup = ydup;
       ra.vsum = vsum.get();
     }
     // verbose: a progress line on stderr at least every 10 s of chunks
@@ -968,14 +966,13 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   } else {
     record(4);
   }
-  launch_fold_sums(vsum.get(), s_);
-  SPTC_HIP(hipMemcpyAsync(&info.value_sum, vsum.get(), sizeof(double), hipMemcpyDeviceToHost,
-                          s_));
+  double* const host_sum = reinterpret_cast<double*>(host_u64_ + 2);
+  launch_fold_sums(vsum.get(), host_sum, s_);
   host_u64_[0] = 0;
-  if (ws_.counters.size())  // no sort ran: no look-back to have failed
-    SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));
+  if (ws_.err()) SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));
   record(5);
   SPTC_HIP(hipStreamSynchronize(s_));
+  info.value_sum = *host_sum;
   kt_.collect(res->kstats, SPTC_K_COUNT);
   if (*reinterpret_cast<uint32_t*>(host_u64_) != 0) {
     msg = "radix sort look-back exceeded its spin limit";

@@ -168,6 +168,8 @@ class Engine {
 
  private:
   U2 read_total(const U2* dev);
+  // the total that a scan wrote to host_total_
+  U2 wait_total();
   // Ranks of the contracted coordinates of X then Y in *rank (nx + ny);
   // returns the number of distinct tuples (0 and msg set on failure).
   uint64_t contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const Layout& xl,

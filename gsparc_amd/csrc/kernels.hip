@@ -13,7 +13,8 @@ namespace sptc {
 
 // --------------------------------------------------------------------------
 // Tile-sum scan (one workgroup, loops over the tile sums with a carry).
-__global__ __launch_bounds__(kBlock) void k_scan_tiles(U2* sums, uint64_t nt, U2* total) {
+__global__ __launch_bounds__(kBlock) void k_scan_tiles(U2* sums, uint64_t nt, U2* total,
+                                                       U2* host) {
   __shared__ U2 scratch[kBlock / kWave];
   U2 carry = mk2(0, 0);
   for (uint64_t base = 0; base < nt; base += kScanTile) {
@@ -34,7 +35,10 @@ __global__ __launch_bounds__(kBlock) void k_scan_tiles(U2* sums, uint64_t nt, U2
     }
     carry = carry + tot;
   }
-  if (threadIdx.x == 0) *total = carry;
+  if (threadIdx.x == 0) {
+    *total = carry;
+    if (host) *host = carry;
+  }
 }
 
 // Many-workgroup tile-sum scan: block sums, one scan of the block sums,
@@ -112,8 +116,8 @@ void scan_tiles_parts(U2* sums, uint64_t nt, U2* total, U2* parts, hipStream_t s
   hipLaunchKernelGGL(k_part_apply, dim3(nb), dim3(kPartNT), 0, s, sums, nt, parts);
 }
 
-void scan_tiles(U2* sums, uint64_t nt, U2* total, hipStream_t s) {
-  hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kBlock), 0, s, sums, nt, total);
+void scan_tiles(U2* sums, uint64_t nt, U2* total, hipStream_t s, U2* host) {
+  hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kBlock), 0, s, sums, nt, total, host);
 }
 
 // --------------------------------------------------------------------------
@@ -183,26 +187,38 @@ void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* key
 // compacted list of distinct c with their start offsets, searched per X
 // nonzero.
 
+// dup / hdup (device / pinned host, may be NULL; cleared by the caller): set
+// when two Y keys are equal.
 __global__ __launch_bounds__(kBlock) void k_ytable_direct(const uint64_t* __restrict__ ykeys,
                                                           uint64_t ny, int ynf, uint64_t K,
                                                           uint64_t* __restrict__ lo,
-                                                          uint64_t* __restrict__ hi) {
+                                                          uint64_t* __restrict__ hi,
+                                                          uint64_t* dup, uint64_t* hdup) {
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+  bool same = false;
   for (; i < ny; i += stride) {
-    uint64_t c = shr64(ykeys[i], ynf);
+    const uint64_t k = ykeys[i];
+    const uint64_t prev = i ? ykeys[i - 1] : 0, next = i + 1 < ny ? ykeys[i + 1] : 0;
+    same |= i && prev == k;
+    const uint64_t c = shr64(k, ynf);
     if (c >= K) continue;  // key outside the contract field: matches nothing
-    if (i == 0 || shr64(ykeys[i - 1], ynf) != c) lo[c] = i;
-    if (i == ny - 1 || shr64(ykeys[i + 1], ynf) != c) hi[c] = i + 1;
+    if (i == 0 || shr64(prev, ynf) != c) lo[c] = i;
+    if (i == ny - 1 || shr64(next, ynf) != c) hi[c] = i + 1;
+  }
+  if (dup && __ballot(same) && lane_id() == 0) {
+    *dup = 1;
+    *hdup = 1;
   }
 }
 
 void launch_ytable_direct(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t K,
-                          uint64_t* lo, uint64_t* hi, hipStream_t s) {
+                          uint64_t* lo, uint64_t* hi, hipStream_t s, uint64_t* dup,
+                          uint64_t* hdup) {
   if (!ny) return;
   uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(ny, kBlock), 4096);
   hipLaunchKernelGGL(k_ytable_direct, dim3(grid), dim3(kBlock), 0, s, ykeys, ny, ynf, K, lo,
-                     hi);
+                     hi, dup, hdup);
 }
 
 struct YUniqueOp {
@@ -224,9 +240,10 @@ struct YUniqueOp {
 };
 
 void run_yunique(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t* ukey,
-                 uint64_t* ustart, U2* tmp, hipStream_t s) {
+                 uint64_t* ustart, U2* tmp, hipStream_t s,
+                 U2* host) {
   YUniqueOp op{ykeys, ny, ynf, ukey, ustart};
-  run_scan(op, ny, tmp, s);
+  run_scan(op, ny, tmp, s, true, host);
 }
 
 __device__ __forceinline__ void ytable_lookup(const YTable& t, uint64_t c,
@@ -297,13 +314,19 @@ struct MatchOp {
       o.act_xval[j] = xvals[i];
       o.act_row[j] = (uint32_t)row;
     }
+    if (i == nx - 1) {  // the totals close every table
+      const uint64_t P = excl.a + cnt, A = (excl.b >> 32) + (cnt != 0);
+      o.act_prefix[A] = P;
+      o.row_prod[row + 1] = P;
+      o.row_act[row + 1] = A;
+    }
   }
 };
 
 void run_match(const uint64_t* xkeys, const float* xvals, uint64_t nx, int ncbits,
-               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s) {
+               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s, U2* host) {
   MatchOp op{xkeys, xvals, nx, low_mask(ncbits), ncbits, t, o, api};
-  run_scan(op, nx, tmp, s);
+  run_scan(op, nx, tmp, s, true, host);
 }
 
 void run_match_count(const uint64_t* xkeys, uint64_t nx, int ncbits, const YTable& t, U2* tmp,
@@ -426,9 +449,10 @@ void launch_yfree_extract(const uint64_t* ykeys, uint64_t ny, uint64_t fmask, ui
   hipLaunchKernelGGL(k_yfree_extract, dim3(grid), dim3(kBlock), 0, s, ykeys, ny, fmask, out);
 }
 
-void run_unique(const uint64_t* sorted, uint64_t n, uint64_t* out, U2* tmp, hipStream_t s) {
+void run_unique(const uint64_t* sorted, uint64_t n, uint64_t* out, U2* tmp, hipStream_t s,
+                 U2* host) {
   UniqueOp op{sorted, out};
-  run_scan(op, n, tmp, s);
+  run_scan(op, n, tmp, s, true, host);
 }
 
 void launch_yrank(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t fmask,
@@ -940,7 +964,7 @@ void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_fold_sums(double* slots) {
+__global__ __launch_bounds__(kBlock) void k_fold_sums(const double* slots, double* out) {
   __shared__ double red[kBlock / kWave];
   double t = 0.0;
   for (uint32_t i = threadIdx.x; i < kSumSlots; i += kBlock) t += slots[i];
@@ -950,29 +974,32 @@ __global__ __launch_bounds__(kBlock) void k_fold_sums(double* slots) {
   if (threadIdx.x == 0) {
     double u = 0.0;
     for (int w = 0; w < kBlock / kWave; ++w) u += red[w];
-    slots[0] = u;
+    *out = u;
   }
 }
 
-void launch_fold_sums(double* slots, hipStream_t s) {
-  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kBlock), 0, s, slots);
+void launch_fold_sums(const double* slots, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kBlock), 0, s, slots, out);
 }
 
 // Any two equal adjacent keys in a sorted array (duplicate coordinates).
 __global__ __launch_bounds__(kBlock) void k_any_dup(const uint64_t* __restrict__ keys, uint64_t n,
-                                                    uint32_t* flag) {
+                                                    uint64_t* dup, uint64_t* hdup) {
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x + 1;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  bool dup = false;
-  for (; i < n; i += stride) dup |= keys[i] == keys[i - 1];
-  if (__ballot(dup) && lane_id() == 0) atomicOr(flag, 1u);
+  bool same = false;
+  for (; i < n; i += stride) same |= keys[i] == keys[i - 1];
+  if (__ballot(same) && lane_id() == 0) {
+    *dup = 1;
+    *hdup = 1;
+  }
 }
 
-void launch_any_dup(const uint64_t* keys, uint64_t n, uint32_t* flag, hipStream_t s) {
-  fill_u32(flag, 0, 1, s);
+void launch_any_dup(const uint64_t* keys, uint64_t n, uint64_t* dup, uint64_t* hdup,
+                    hipStream_t s) {
   if (n < 2) return;
   uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock), 2048);
-  hipLaunchKernelGGL(k_any_dup, dim3(grid), dim3(kBlock), 0, s, keys, n, flag);
+  hipLaunchKernelGGL(k_any_dup, dim3(grid), dim3(kBlock), 0, s, keys, n, dup, hdup);
 }
 
 // Exclusive scan of per-row uint32 counts into uint64 offsets (+ total).
@@ -983,8 +1010,9 @@ struct RowCountScanOp {
   __device__ void emit(uint64_t i, U2 excl, U2) const { out[i] = excl.a; }
 };
 
-void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s) {
-  run_scan(RowCountScanOp{cnt, off}, n, tmp, s);
+void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s,
+                 U2* host) {
+  run_scan(RowCountScanOp{cnt, off}, n, tmp, s, true, host);
 }
 
 // --------------------------------------------------------------------------

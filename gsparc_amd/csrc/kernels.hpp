@@ -123,19 +123,26 @@ inline bool dense_pays(uint64_t ir, uint64_t rows, uint64_t active, uint64_t slo
 
 void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
 void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s);
-// slots[0] = sum of the kSumSlots slots, added in a fixed order.
-void launch_fold_sums(double* slots, hipStream_t s);
-void launch_any_dup(const uint64_t* keys, uint64_t n, uint32_t* flag, hipStream_t s);
-void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s);
+// *out (device or pinned host memory) = sum of the kSumSlots slots, added in a
+// fixed order.
+void launch_fold_sums(const double* slots, double* out, hipStream_t s);
+// Sets *dup (device) and *hdup (pinned host), cleared by the caller, when two
+// adjacent keys are equal.
+void launch_any_dup(const uint64_t* keys, uint64_t n, uint64_t* dup, uint64_t* hdup,
+                    hipStream_t s);
+void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s,
+                        U2* host = nullptr);
 
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
                       uint64_t* hist, int passes, int rb, hipStream_t s);
 void launch_ytable_direct(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t K,
-                          uint64_t* lo, uint64_t* hi, hipStream_t s);
+                          uint64_t* lo, uint64_t* hi, hipStream_t s, uint64_t* dup = nullptr,
+                          uint64_t* hdup = nullptr);
 void run_yunique(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t* ukey,
-                 uint64_t* ustart, U2* tmp, hipStream_t s);
+                 uint64_t* ustart, U2* tmp, hipStream_t s, U2* host = nullptr);
 void run_match(const uint64_t* xkeys, const float* xvals, uint64_t nx, int ncbits,
-               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s);
+               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s,
+               U2* host = nullptr);
 // Reduce half of run_match: tmp[scan_tmp_count(nx)] = {ir, A << 32 | R}.
 void run_match_count(const uint64_t* xkeys, uint64_t nx, int ncbits, const YTable& t, U2* tmp,
                      hipStream_t s);
@@ -171,7 +178,8 @@ void run_reduce_emit_narrow(const NarrowRows& nr, const float* vals, uint64_t n,
                             hipStream_t s);
 void launch_yfree_extract(const uint64_t* ykeys, uint64_t ny, uint64_t fmask, uint64_t* out,
                           hipStream_t s);
-void run_unique(const uint64_t* sorted, uint64_t n, uint64_t* out, U2* tmp, hipStream_t s);
+void run_unique(const uint64_t* sorted, uint64_t n, uint64_t* out, U2* tmp, hipStream_t s,
+                U2* host = nullptr);
 void launch_tuple_key(const TupleArgs& a, uint64_t n, uint64_t* out, hipStream_t s);
 // *out = max(*out, largest of the n indices); *out cleared by the caller.
 void launch_mode_max(const void* idx, int bytes, uint64_t n, uint64_t* out, hipStream_t s);

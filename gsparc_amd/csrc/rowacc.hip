@@ -140,7 +140,7 @@ struct RowKindOp {
   RowAccArgs a;
   uint32_t least;
   uint64_t heavy;  // products of an item that one workgroup should not be given
-  uint32_t* flag;
+  uint64_t* flag;  // pinned host memory
   uint32_t *live_row, *live_cnt;
   uint64_t* live_src;
   uint32_t *s_live, *s_prod, *l_live;
@@ -1205,17 +1205,13 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   room(p->s_prod, rows);
   room(p->l_live, rows);
   room(p->tmp, scan_tmp_count(rows) + 1);
-  room(p->flag, 1);
-  fill_u32(p->flag.get(), 0, 1, s);
   const uint32_t least = min_slabs(a.K);
-  RowKindOp kind{a, least, std::max(kHeavyItem, nprod >> 10), p->flag.get(), p->live_row.get(), p->live_cnt.get(), p->live_src.get(), p->s_live.get(),
+  RowKindOp kind{a, least, std::max(kHeavyItem, nprod >> 10), &host[1].a, p->live_row.get(), p->live_cnt.get(), p->live_src.get(), p->s_live.get(),
                  p->s_prod.get(), p->l_live.get()};
-  run_scan(kind, rows, p->tmp.get(), s);
-  SPTC_HIP(hipMemcpyAsync(host, p->tmp.get() + scan_tmp_count(rows), sizeof(U2),
-                          hipMemcpyDeviceToHost, s));
-  SPTC_HIP(hipMemcpyAsync(host + 1, p->flag.get(), 4, hipMemcpyDeviceToHost, s));
+  host[1].a = 0;
+  run_scan(kind, rows, p->tmp.get(), s, true, host);
   SPTC_HIP(hipStreamSynchronize(s));
-  if ((uint32_t)host[1].a) return false;
+  if (host[1].a) return false;
   p->live = host->a & 0xFFFFFFFFull;
   p->short_prods = host->a >> 32;
   p->nshort = host->b >> 32;
@@ -1263,7 +1259,7 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
     if (p->keep_words) room(p->words, max_words);
     SlabOp slab{a, least, p->l_live.get(), p->live_row.get(), p->nlong, p->l_item.get(),
                 p->l_split.get(), p->l_word.get()};
-    run_scan(slab, p->nlong, p->tmp.get(), s);
+    run_scan(slab, p->nlong, p->tmp.get(), s, true, host + 2);
     if (!p->quant.size()) {
       p->quant.reset(kQuant + 1);
       hipLaunchKernelGGL(k_ra_quant, dim3(1), dim3(kQuantNT), 0, s, a.ycol, a.ny, a.K,
@@ -1296,16 +1292,12 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
             p->l_near.get(),
             p->near_pre.get(),
             reinterpret_cast<Near*>(p->near.get())};
-  run_scan(out, p->live, p->tmp.get(), s);
-  SPTC_HIP(hipMemcpyAsync(host, p->tmp.get() + scan_tmp_count(p->live), sizeof(U2),
-                          hipMemcpyDeviceToHost, s));
-  if (p->nlong)
-    SPTC_HIP(hipMemcpyAsync(host + 1, p->l_item.get() + p->nlong, 8, hipMemcpyDeviceToHost, s));
+  run_scan(out, p->live, p->tmp.get(), s, true, host);
   SPTC_HIP(hipStreamSynchronize(s));
   p->outs = host[0].a;
   p->near_rows = host[0].b >> 32;
   p->near_outs = host[0].b & 0xFFFFFFFFull;
-  if (p->nlong) p->items = host[1].a;
+  if (p->nlong) p->items = host[2].a & 0xFFFFFFFFull;
   if (count_only && p->near_outs) {
     const uint32_t nt = (uint32_t)ceil_div(p->near_outs, kNearTile);
     const int tok = kt->begin(s);

@@ -39,7 +39,7 @@ struct RowAccArgs {
   const uint32_t* ytab32;      // the same as 32 bits (NULL: wider)
   uint32_t K;                  // column ranks below K
   uint32_t short_max;          // rows of several owners up to this many products are short
-  const uint32_t* ydup;        // nonzero: Y holds duplicate coordinates
+  const uint64_t* ydup;        // nonzero: Y holds duplicate coordinates
   double* vsum;                // [kSumSlots]
 };
 
@@ -73,11 +73,10 @@ struct RowAccPlan {
   DevBuf<uint32_t> tcol;                     // [short_prods] a group's outputs, compacted
   DevBuf<float> tval;
   DevBuf<U2> tmp;
-  DevBuf<uint32_t> flag;
 };
 
 // Classifies the rows and counts every row's outputs (plan->outs); host
-// receives two U2 of pinned memory.  One wait for the row kinds, one for the
+// receives three U2 of pinned memory.  One wait for the row kinds, one for the
 // counts.  count_only: the groups' outputs are not kept and the value sum is
 // taken here.  nprod and owners: the chunk's products and active X nonzeros.
 // False, with nothing done, when a row is too heavy for one workgroup an item.

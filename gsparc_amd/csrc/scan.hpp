@@ -6,10 +6,14 @@
 // where V is U2 (two uint64 lanes, added lane-wise).  An Op that declares a
 // type Aux instead supplies value(i, Aux&) and emit(i, excl, val, const
 // Aux&): what value() looked up reaches emit() in registers, not loaded
-// again.  Three kernels:
+// again.  Kernels:
 //   k_scan_reduce : per tile of kBlock*kScanItems items, the tile sum
 //   k_scan_tiles  : exclusive scan of tile sums (single workgroup), total
 //   k_scan_emit   : recompute values, block scan + tile offset, emit()
+// Short scans take fewer launches, each about 4 us of a small call's time: up
+// to kScanOneMax items one workgroup runs the whole scan (k_scan_one); up to
+// kScanSelfTiles tiles every emitting workgroup adds up the tile sums before
+// its own (k_scan_emit with SELF; at most 8 KiB read by each).
 // Values are computed and emitted tile-striped (item e*kBlock + t of a tile
 // to thread t, so each of the kScanItems loads and stores of a workgroup is
 // one contiguous run); the emit's scan goes through LDS, where thread t
@@ -98,12 +102,25 @@ __global__ __launch_bounds__(kBlock) void k_scan_reduce(Op op, uint64_t n, U2* t
   if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
 }
 
-template <class Op>
-__global__ __launch_bounds__(kBlock) void k_scan_emit(Op op, uint64_t n, const U2* tile_offs) {
+constexpr uint64_t kScanSelfTiles = 512;
+
+// SELF: tile_offs holds unscanned sums of nt tiles; the last workgroup writes
+// the total.
+template <class Op, bool SELF>
+__global__ __launch_bounds__(kBlock) void k_scan_emit(Op op, uint64_t n, const U2* tile_offs,
+                                                      uint32_t nt, U2* total, U2* host) {
   __shared__ U2 scratch[kBlock / kWave];
   __shared__ U2 sv[kScanTile];  // values, then exclusive prefixes, by tile index
   const uint32_t tid = threadIdx.x;
   const uint64_t base = (uint64_t)blockIdx.x * kScanTile;
+  U2 tile_off;
+  if (SELF) {
+    U2 before = mk2(0, 0);
+    for (uint32_t t = tid; t < blockIdx.x; t += kBlock) before = before + tile_offs[t];
+    block_excl_scan_u2(before, scratch, &tile_off);
+  } else {
+    tile_off = tile_offs[blockIdx.x];
+  }
   U2 vals[kScanItems];
   typename ScanAux<Op>::type aux[kScanItems];
 #pragma unroll
@@ -121,7 +138,11 @@ __global__ __launch_bounds__(kBlock) void k_scan_emit(Op op, uint64_t n, const U
     s = s + mine[e];
   }
   U2 tot;  // (barriers inside: every thread's reads of sv are done after it)
-  U2 excl = block_excl_scan_u2(s, scratch, &tot) + tile_offs[blockIdx.x];
+  U2 excl = block_excl_scan_u2(s, scratch, &tot) + tile_off;
+  if (SELF && tid == 0 && blockIdx.x + 1 == nt) {
+    *total = tile_off + tot;
+    if (host) *host = tile_off + tot;
+  }
 #pragma unroll
   for (int e = 0; e < kScanItems; ++e) {
     sv[tid * kScanItems + e] = excl;
@@ -138,12 +159,83 @@ __global__ __launch_bounds__(kBlock) void k_scan_emit(Op op, uint64_t n, const U
   }
 }
 
+// The whole scan by one workgroup of 1024 threads, tiles of 4 items a thread.
+constexpr int kOneNT = 1024, kOneItems = 4;
+constexpr uint64_t kOneTile = (uint64_t)kOneNT * kOneItems;
+constexpr uint64_t kScanOneMax = 4 * kOneTile;
+
+template <class Op>
+__global__ __launch_bounds__(kOneNT) void k_scan_one(Op op, uint32_t n, bool emit, U2* total,
+                                                     U2* host) {
+  __shared__ U2 scratch[kOneNT / kWave];
+  __shared__ U2 sv[kOneTile];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  U2 carry = mk2(0, 0);
+  for (uint32_t base = 0; base < n; base += (uint32_t)kOneTile) {
+    U2 vals[kOneItems];
+    typename ScanAux<Op>::type aux[kOneItems];
+#pragma unroll
+    for (int e = 0; e < kOneItems; ++e) {
+      const uint32_t i = base + (uint32_t)e * kOneNT + tid;
+      vals[e] = i < n ? scan_value(op, (uint64_t)i, aux[e]) : mk2(0, 0);
+      sv[e * kOneNT + tid] = vals[e];
+    }
+    __syncthreads();
+    U2 mine[kOneItems];
+    U2 t = mk2(0, 0);
+#pragma unroll
+    for (int e = 0; e < kOneItems; ++e) {
+      mine[e] = sv[tid * kOneItems + e];
+      t = t + mine[e];
+    }
+    U2 inc = t;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint64_t oa = __shfl_up(inc.a, d, kWave), ob = __shfl_up(inc.b, d, kWave);
+      if (lane >= (uint32_t)d) inc = inc + mk2(oa, ob);
+    }
+    if (lane == kWave - 1) scratch[wave] = inc;
+    __syncthreads();
+    U2 excl = carry + inc - t;
+    for (uint32_t w = 0; w < (uint32_t)(kOneNT / kWave); ++w) {
+      const U2 x = scratch[w];
+      if (w < wave) excl = excl + x;
+      carry = carry + x;
+    }
+#pragma unroll
+    for (int e = 0; e < kOneItems; ++e) {
+      sv[tid * kOneItems + e] = excl;
+      excl = excl + mine[e];
+    }
+    __syncthreads();
+    if (emit) {
+#pragma unroll
+      for (int e = 0; e < kOneItems; ++e) {
+        const uint32_t i = base + (uint32_t)e * kOneNT + tid;
+        if (i < n) {
+          if constexpr (ScanAux<Op>::on)
+            op.emit((uint64_t)i, sv[e * kOneNT + tid], vals[e], aux[e]);
+          else
+            op.emit((uint64_t)i, sv[e * kOneNT + tid], vals[e]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    *total = carry;
+    if (host) *host = carry;
+  }
+}
+
 // In-place exclusive scan of nt tile sums by one workgroup; total -> *total
 // (defined in kernels.hip).
-void scan_tiles(U2* sums, uint64_t nt, U2* total, hipStream_t s);
+// host (may be NULL): pinned host memory that receives the total too.
+void scan_tiles(U2* sums, uint64_t nt, U2* total, hipStream_t s, U2* host = nullptr);
 
 // Runs reduce -> tile scan -> emit.  `tmp` must hold scan_tmp_count(n)+1 U2
-// entries; the grand total lands in tmp[scan_tmp_count(n)].
+// entries; the grand total lands in tmp[scan_tmp_count(n)] and, when given, in
+// the pinned host memory `host` (readable once the stream is waited for).
 inline uint64_t scan_tmp_count(uint64_t n) { return ceil_div(n ? n : 1, kScanTile); }
 
 // Long tile-sum arrays (one sum per 2048 products of a reduce count) are
@@ -169,18 +261,29 @@ inline uint64_t narrow_tmp_count(uint64_t n) {
 void scan_tiles_parts(U2* sums, uint64_t nt, U2* total, U2* parts, hipStream_t s);
 
 template <class Op>
-void run_scan(const Op& op, uint64_t n, U2* tmp, hipStream_t s, bool emit = true) {
+void run_scan(const Op& op, uint64_t n, U2* tmp, hipStream_t s, bool emit = true,
+              U2* host = nullptr) {
   const uint64_t nt = scan_tmp_count(n);
   U2* total = tmp + nt;
   if (n == 0) {
-    scan_tiles(tmp, 0, total, s);
+    scan_tiles(tmp, 0, total, s, host);
+    return;
+  }
+  if (n <= kScanOneMax) {
+    hipLaunchKernelGGL(k_scan_one<Op>, dim3(1), dim3(kOneNT), 0, s, op, (uint32_t)n, emit, total,
+                       host);
     return;
   }
   hipLaunchKernelGGL(k_scan_reduce<Op>, dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n, tmp);
-  scan_tiles(tmp, nt, total, s);
+  if (emit && nt <= kScanSelfTiles) {
+    hipLaunchKernelGGL((k_scan_emit<Op, true>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
+                       (const U2*)tmp, (uint32_t)nt, total, host);
+    return;
+  }
+  scan_tiles(tmp, nt, total, s, host);
   if (emit)
-    hipLaunchKernelGGL(k_scan_emit<Op>, dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
-                       (const U2*)tmp);
+    hipLaunchKernelGGL((k_scan_emit<Op, false>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
+                       (const U2*)tmp, (uint32_t)nt, (U2*)nullptr, (U2*)nullptr);
 }
 
 }  // namespace sptc

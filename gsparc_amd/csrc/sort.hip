@@ -357,11 +357,11 @@ uint64_t SortWorkspace::bytes_per_key(int rb) {
 
 void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s) {
   const uint64_t R = 1ull << rb_;
-  if (counters.size() == 0) {
+  if (sort_cfg().onesweep && counters.size() == 0) {
     counters.reset(64);
     fill_u32(counters.get(), 0, 64, s);
   }
-  if (hist.size() < kMaxPasses * R) {
+  if (sort_cfg().onesweep && hist.size() < kMaxPasses * R) {
     hist.reset(kMaxPasses * R);
     base.reset(kMaxPasses * R);
   }
@@ -386,6 +386,7 @@ void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s) {
 }
 
 void SortWorkspace::prepare(int passes, hipStream_t s) {
+  if (!sort_cfg().onesweep) return;
   uint64_t R = 1ull << rb;
   fill_u64(hist.get(), 0, (uint64_t)passes * R, s);
   fill_u32(counters.get(), 0, kMaxPasses, s);

@@ -26,9 +26,11 @@ struct SortWorkspace {
 
   // Grows the workspace to hold `n` keys at `rb` radix bits.
   void ensure(uint64_t n, int rb, hipStream_t s);
-  // Clears histograms and tile counters before a producer accumulates.
+  // Clears histograms and tile counters before a producer accumulates (used by
+  // the onesweep passes alone).
   void prepare(int passes, hipStream_t s);
-  uint32_t* err() const { return counters.get() + 32; }
+  // look-back error flag (NULL: no onesweep pass has run)
+  uint32_t* err() const { return counters.size() ? counters.get() + 32 : nullptr; }
   static uint64_t bytes_per_key(int rb);
 };
 
