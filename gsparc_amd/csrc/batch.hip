@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kBlock) void k_bdense_count(BDenseArgs a) {
   BInst in;
   bdense_row(a, blockIdx.x, r, in);
   const uint32_t t = dense_row_count<EB>(a.d, a.d.row_act[r], a.d.row_act[r + 1],
-                                         low_mask(in.kyf), sm, &s_ja);
+                                         sm, &s_ja);
   if (threadIdx.x == 0) a.d.row_cnt[blockIdx.x] = t;
 }
 
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_bdense_numeric(BDenseArgs a) {
   bdense_row(a, blockIdx.x, r, in);
   const uint32_t g = find_seg(a.grp_rows, a.G, blockIdx.x);
   // instance-local row id
-  dense_row_numeric<EB>(a.d, a.d.row_act[r], a.d.row_act[r + 1], low_mask(in.kyf),
+  dense_row_numeric<EB>(a.d, a.d.row_act[r], a.d.row_act[r + 1],
                         a.ytab + in.yt_off, (uint32_t)(blockIdx.x - a.grp_rows[g]),
                         a.d.out_off[blockIdx.x], s_acc, sm, &s_ja);
 }

@@ -501,7 +501,7 @@ sptc_status BatchEngine::run(hipStream_t s, bool P) {
     da.d.act_ypos = act_ypos_.get();
     da.d.act_xval = act_xval_.get();
     da.d.row_act = row_act_.get();
-    da.d.ykeys = yk;
+    da.d.ycol = ycol_.get();
     da.d.yvals = yv;
     da.d.row_cnt = c.row_cnt.get();
     da.d.out_off = c.out_off.get();

@@ -66,8 +66,7 @@ __device__ __forceinline__ uint32_t dense_owner(const uint64_t* pref, uint32_t m
 // (valid in thread 0).
 template <int EB>
 __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t j0, uint64_t j1,
-                                                    uint64_t cmask, DenseSmem<EB>& sm,
-                                                    uint64_t* s_ja) {
+                                                    DenseSmem<EB>& sm, uint64_t* s_ja) {
   for (int i = threadIdx.x; i < DenseSmem<EB>::W; i += kBlock) sm.bm[i] = 0;
   const uint64_t p0 = j0 < j1 ? a.act_prefix[j0] : 0;
   const uint64_t p1 = j0 < j1 ? a.act_prefix[j1] : 0;
@@ -81,7 +80,7 @@ __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t
       if (p < p1) {
         const uint32_t k = dense_owner(sm.pref, m, p);
         const uint64_t y = a.act_ypos[ja + k] + (p - sm.pref[k]);
-        const uint32_t rank = (uint32_t)(a.ykeys[y] & cmask);
+        const uint32_t rank = a.ycol[y];
         atomicOr(&sm.bm[rank >> 5], 1u << (rank & 31));
       }
     }
@@ -102,8 +101,7 @@ __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t
 // id `row`, column ytab[rank] or rank).  `acc` holds E doubles of LDS.
 template <int EB>
 __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j0, uint64_t j1,
-                                                  uint64_t cmask, const uint64_t* ytab,
-                                                  uint32_t row, uint64_t obase, double* acc,
+                                                  const uint64_t* ytab, uint32_t row, uint64_t obase, double* acc,
                                                   DenseSmem<EB>& sm, uint64_t* s_ja) {
   constexpr int E = DenseSmem<EB>::E;
   constexpr int S = E / kBlock;  // slots per thread in the compaction (1..32)
@@ -127,7 +125,7 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
       if (p < p1) {
         const uint32_t k = dense_owner(sm.pref, m, p);
         const uint64_t y = a.act_ypos[ja + k] + (p - sm.pref[k]);
-        rank[g] = (uint32_t)(a.ykeys[y] & cmask);
+        rank[g] = a.ycol[y];
         val[g] = a.act_xval[ja + k] * a.yvals[y];
       }
     }

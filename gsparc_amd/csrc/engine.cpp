@@ -2,6 +2,7 @@
 #include "engine.hpp"
 
 #include "bucket.hpp"
+#include "ranks.hpp"
 #include "rowacc.hpp"
 #include "tdense.hpp"
 
@@ -327,7 +328,6 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
   const int nc = xl.nc;
   if (!nc) return 1;
   DevBuf<uint64_t> key(n), sorted(n);
-  DevBuf<float> payload(n);  // moved with the keys, never read
   DevBuf<uint64_t> uniq(n);
   DevBuf<U2> tmp(scan_tmp_count(n) + 1);
   uint64_t U = 1;
@@ -366,7 +366,7 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
     ws_.ensure(n, rb, s_);
     ws_.prepare(radix_passes(bits, rb), s_);
     if (sort_needs_histogram()) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
-    const bool alt = sort_after_histogram(ws_, sorted.get(), payload.get(), n, bits, s_);
+    const bool alt = sort_after_histogram(ws_, sorted.get(), nullptr, n, bits, s_);
     run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_, host_total_);
     U = wait_total().a;
     launch_yrank(key.get(), n, 64, ~0ull, uniq.get(), U, 0, rank->get(), s_);
@@ -421,41 +421,41 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   res->xl = xl;
   res->yl = yl;
 
-  // ---- Y free-key rank compression (shorter product keys) ----------------
-  // kyf: width of the column field inside Y keys and product keys from here
-  // on; ytab maps a rank back to the Y free key when the field is a rank.
-  int kyf = ynf;
-  uint64_t ranks = kyf < 32 ? 1ull << kyf : 0;  // columns below this
-  const uint64_t* ykeys = Y.keys.get();
-  DevBuf<uint64_t> ykeys_rank, ytab;
-  DevBuf<uint32_t> ytab32;  // ytab as 32-bit words when Y free keys fit them
-  if (ynf > 0 && ny > 1) {
-    DevBuf<uint64_t> fk(ny);
-    DevBuf<float> fv(ny);
-    launch_yfree_extract(Y.keys.get(), ny, low_mask(ynf), fk.get(), s_);
-    const int rbf = rb_ ? rb_ : choose_radix_bits(ynf);
-    ws_.ensure(ny, rbf, s_);
-    ws_.prepare(radix_passes(ynf, rbf), s_);
-    if (sort_needs_histogram()) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
-    const bool alt = sort_after_histogram(ws_, fk.get(), fv.get(), ny, ynf, s_);
-    ytab.reset(ny);
-    DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-    run_unique(alt ? ws_.alt_keys.get() : fk.get(), ny, ytab.get(), tmp.get(), s_, host_total_);
-    const uint64_t U = wait_total().a;
-    const int yrb = mode_bits(U);
-    if (yrb < ynf) {
-      ykeys_rank.reset(ny);
-      launch_yrank(Y.keys.get(), ny, ynf, low_mask(ynf), ytab.get(), U, yrb, ykeys_rank.get(),
-                   s_);
-      ykeys = ykeys_rank.get();
-      kyf = yrb;
-      ranks = U;
-      if (ynf <= 32) {
-        ytab32.reset(U);
-        launch_ycol(ytab.get(), U, 0xFFFFFFFFull, ytab32.get(), s_);
-      }
+  // ---- column ranks: Y free keys -> ranks among the distinct ones -----------
+  // ycol holds every Y entry's column, ytab maps a rank back to the Y free key
+  // (ytab32: as 32-bit words when the keys fit them).  The number of ranks
+  // arrives with the match totals (host_total_[1]).
+  const bool ranked = ynf > 0 && ny > 1;
+  DevBuf<uint64_t> ytab, fk;
+  DevBuf<uint32_t> ytab32, ycol, yfree32;
+  DevBuf<uint8_t> rmap;
+  DevBuf<U2> rtmp;
+  if (ranked) {
+    const uint64_t most = ynf < 32 ? std::min<uint64_t>(ny, 1ull << ynf) : ny;
+    ytab.reset(most);
+    ycol.reset(ny);
+    if (ynf <= 32) {
+      ytab32.reset(most);
+      yfree32.reset(ny);
+    }
+    const RankOut ro{ytab.get(), ytab32.get(), ycol.get(), yfree32.get()};
+    // (a tight budget keeps to the sort, whose workspace its parts are sized for)
+    if (rank_by_map(ny, ynf) && rank_map_bytes(ynf) <= budget_avail() / 16) {
+      const uint64_t nw = rank_words(ynf);
+      rmap.reset(rank_map_bytes(ynf));
+      rtmp.reset(scan_tmp_count(nw) + 1);
+      run_rank_map(Y.keys.get(), ny, ynf, ro, rmap.get(), rtmp.get(), host_total_ + 1, s_);
     } else {
-      ytab.release();
+      fk.reset(ny);
+      launch_yfree_extract(Y.keys.get(), ny, low_mask(ynf), fk.get(), s_);
+      const int rbf = rb_ ? rb_ : choose_radix_bits(ynf);
+      ws_.ensure(ny, rbf, s_);
+      ws_.prepare(radix_passes(ynf, rbf), s_);
+      if (sort_needs_histogram()) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
+      const bool alt = sort_after_histogram(ws_, fk.get(), nullptr, ny, ynf, s_);
+      rtmp.reset(scan_tmp_count(ny) + 1);
+      run_rank_sorted(alt ? ws_.alt_keys.get() : fk.get(), Y.keys.get(), ny, ynf, ro, rtmp.get(),
+                      host_total_ + 1, s_);
     }
   }
 
@@ -472,7 +472,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     tlo.reset(2 * K + 1);  // the table and the duplicate flag, one fill
     fill_u64(tlo.get(), 0, 2 * K + 1, s_);
     ydup = tlo.get() + 2 * K;
-    launch_ytable_direct(ykeys, ny, kyf, K, tlo.get(), tlo.get() + K, s_, ydup, hdup);
+    launch_ytable_direct(Y.keys.get(), ny, ynf, K, tlo.get(), tlo.get() + K, s_, ydup, hdup);
     tab.direct = 1;
     tab.lo = tlo.get();
     tab.hi = tlo.get() + K;
@@ -484,7 +484,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     ydup = tlo.get();
     fill_u64(ydup, 0, 1, s_);
     launch_any_dup(Y.keys.get(), ny, ydup, hdup, s_);
-    run_yunique(ykeys, ny, kyf, ukey.get(), ustart.get(), tmp.get(), s_, host_total_);
+    run_yunique(Y.keys.get(), ny, ynf, ukey.get(), ustart.get(), tmp.get(), s_, host_total_);
     tab.direct = 0;
     tab.ukey = ukey.get();
     tab.ustart = ustart.get();
@@ -518,9 +518,25 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   ukey.release();
   ustart.release();
   record(3);
+  // width of the column field and the columns: the distinct free keys
+  const uint64_t ranks = ranked ? host_total_[1].a : ynf < 32 ? 1ull << ynf : 0;
+  const int kyf = ranked ? mode_bits(ranks) : ynf;
+  fk.release();
+  rmap.release();
+  rtmp.release();
   info.ir_nnz = ir;
   info.nrows = R;
   res->row_key = std::move(row_key);
+
+  // the columns of Y entries that were not ranked (at most one entry, or no
+  // free bits)
+  auto ycol_or_make = [&]() -> const uint32_t* {
+    if (!ycol.size()) {
+      ycol.reset(ny ? ny : 1);
+      launch_ycol(Y.keys.get(), ny, low_mask(ynf), ycol.get(), s_);
+    }
+    return ycol.get();
+  };
 
   // ---- accumulator choice (the reference's -d flag, sptc.cuh:201-218) ------
   // Dense applies when the column space (ranks of Y's free keys) fits an LDS
@@ -564,9 +580,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     da.act_xval = act_xval.get();
     da.row_act = row_act.get();
     da.r0 = 0;
-    da.ykeys = ykeys;
+    da.ycol = ycol_or_make();
     da.yvals = Y.vals.get();
-    da.fmask = low_mask(kyf);
     da.ytab = ytab.size() ? ytab.get() : nullptr;
     da.row_cnt = row_cnt.get();
     da.out_off = out_off.get();
@@ -600,9 +615,6 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     }
   } else if (use_tdense) {
     record(4);
-    const uint64_t fmask = low_mask(kyf);
-    DevBuf<uint32_t> ycol32(ny);
-    launch_ycol(ykeys, ny, fmask, ycol32.get(), s_);
     DevBuf<uint64_t> cur(A ? A : 1);
     DevBuf<uint32_t> row_cnt(R);
     DevBuf<uint64_t> out_off(R + 1);
@@ -613,7 +625,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     ta.act_ypos = act_ypos.get();
     ta.act_xval = act_xval.get();
     ta.row_act = row_act.get();
-    ta.ycol = ycol32.get();
+    ta.ycol = ycol_or_make();
     ta.yvals = Y.vals.get();
     ta.ytab = ytab.size() ? ytab.get() : nullptr;
     ta.cur = cur.get();
@@ -740,13 +752,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       ws_.ensure(chunk_cap, rb_max, s_);
     };
     const uint64_t fmask = low_mask(kyf);
-    // 32-bit column field of Y for the expansion (4 bytes per gathered key
-    // instead of 8)
-    DevBuf<uint32_t> ycol;
-    if (kyf <= 32 && !partition_only) {
-      ycol.reset(ny);
-      launch_ycol(ykeys, ny, fmask, ycol.get(), s_);
-    }
+    if (kyf <= 32 && !partition_only) ycol_or_make();
     // row-segmented product sort
     DevBuf<RowRange> rrange(1);
     RowSegPlan rseg;
@@ -754,12 +760,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     const bool rowacc = kyf > 0 && kyf <= kRowAccMaxBits && prefer_row_acc() && !partition_only;
     RowAccPlan rplan;
     RowAccArgs ra;
-    DevBuf<uint32_t> yfree32;
     if (rowacc) {
-      if (ytab.size() && ynf <= 32) {
-        yfree32.reset(ny);
-        launch_ycol(Y.keys.get(), ny, low_mask(ynf), yfree32.get(), s_);
-      }
       ra.act_prefix = act_prefix.get();
       ra.act_ypos = act_ypos.get();
       ra.act_xval = act_xval.get();
@@ -770,7 +771,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       ra.yvals = Y.vals.get();
       ra.ykeys = Y.keys.get();
       ra.yfmask = low_mask(ynf);
-      ra.yfree32 = ytab.size() ? yfree32.get() : ycol.get();
+      ra.yfree32 = ranked ? yfree32.get() : ycol.get();
       ra.ytab = ytab.size() ? ytab.get() : nullptr;
       ra.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
       ra.K = (uint32_t)ranks;
@@ -833,7 +834,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
         ea.P0 = P0;
         ea.P1 = P1;
         ea.r0 = (uint32_t)r0c;
-        ea.ykeys = ykeys;
+        ea.ykeys = Y.keys.get();
         ea.yvals = Y.vals.get();
         ea.ynf = kyf;
         ea.fmask = fmask;

@@ -930,7 +930,7 @@ __global__ __launch_bounds__(kBlock) void k_dense_count(DenseArgs a) {
   __shared__ DenseSmem<EB> sm;
   __shared__ uint64_t s_ja;
   const uint64_t r = a.r0 + blockIdx.x;
-  const uint32_t t = dense_row_count<EB>(a, a.row_act[r], a.row_act[r + 1], a.fmask, sm, &s_ja);
+  const uint32_t t = dense_row_count<EB>(a, a.row_act[r], a.row_act[r + 1], sm, &s_ja);
   if (threadIdx.x == 0) a.row_cnt[blockIdx.x] = t;
 }
 
@@ -941,7 +941,7 @@ __global__ __launch_bounds__(kBlock) void k_dense_numeric(DenseArgs a) {
   __shared__ DenseSmem<EB> sm;
   __shared__ uint64_t s_ja;
   const uint64_t r = a.r0 + blockIdx.x;
-  dense_row_numeric<EB>(a, a.row_act[r], a.row_act[r + 1], a.fmask, a.ytab,
+  dense_row_numeric<EB>(a, a.row_act[r], a.row_act[r + 1], a.ytab,
                                  (uint32_t)r, a.out_off[blockIdx.x], s_acc, sm, &s_ja);
 }
 

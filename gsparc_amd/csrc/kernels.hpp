@@ -89,9 +89,8 @@ struct DenseArgs {
   const float* act_xval;
   const uint64_t* row_act;     // [R+1]
   uint64_t r0;                 // first row of the chunk
-  const uint64_t* ykeys;
+  const uint32_t* ycol;        // [ny] column rank of each Y entry
   const float* yvals;
-  uint64_t fmask;              // column field mask
   const uint64_t* ytab;        // rank -> Y free key (NULL: field is the key)
   uint32_t* row_cnt;           // [rows] symbolic counts
   const uint64_t* out_off;     // [rows] output offsets

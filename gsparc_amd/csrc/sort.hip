@@ -121,8 +121,8 @@ __global__ __launch_bounds__(NT) void k_onesweep(
   uint64_t k[IPT];
   float v[IPT];
   uint32_t pos[IPT];
-  tile_load_rank<false, RB, IPT, NT>(sm, kin + tile_begin, vin + tile_begin, cnt, shift, k, v,
-                                     pos);
+  tile_load_rank<false, RB, IPT, NT>(sm, kin + tile_begin, vin ? vin + tile_begin : nullptr, cnt,
+                                     shift, k, v, pos);
   __syncthreads();
   for (int d = tid; d < R; d += NT) {
     const uint64_t total = wave_prefixes<RB, IPT, NT>(sm, d);
@@ -198,8 +198,8 @@ __global__ __launch_bounds__(NT) void k_rts_downsweep(
   uint64_t k[IPT];
   float v[IPT];
   uint32_t pos[IPT];
-  tile_load_rank<false, RB, IPT, NT>(sm, kin + tile_begin, vin + tile_begin, cnt, shift, k, v,
-                                     pos);
+  tile_load_rank<false, RB, IPT, NT>(sm, kin + tile_begin, vin ? vin + tile_begin : nullptr, cnt,
+                                     shift, k, v, pos);
   __syncthreads();
   for (int d = tid; d < R; d += NT) sm.dstart[d] = (uint16_t)wave_prefixes<RB, IPT, NT>(sm, d);
   __syncthreads();
@@ -408,6 +408,7 @@ void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
   }
 }
 
+// vals NULL: the keys alone are moved.
 // Sorts keys/vals (n <= ws.cap, n < 2^32) on bits [0, nbits).  With the
 // onesweep algorithm ws.hist must hold the digit histograms of all passes.
 // Result ends in (keys, vals) when the pass count is even, else in
@@ -435,8 +436,8 @@ bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
   const uint64_t tiles = ceil_div(n, sort_tile_items(rb));
   const int tag = (cls == SPTC_K_SORT_PROD || cls == SPTC_K_SORT_PROD_WIDE) ? 1 : 0;
   const int kcls = (cls == SPTC_K_SORT_PROD && rb > 8) ? SPTC_K_SORT_PROD_WIDE : cls;
-  PassArgs a{tag, &ws, keys, vals, ws.alt_keys.get(), ws.alt_vals.get(), n, tiles, 0, s, kt,
-             kcls};
+  PassArgs a{tag, &ws, keys, vals, ws.alt_keys.get(), vals ? ws.alt_vals.get() : nullptr, n, tiles,
+             0, s, kt, kcls};
   for (int p = 0; p < passes; ++p) {
     a.pass = p;
     if (onesweep) {
