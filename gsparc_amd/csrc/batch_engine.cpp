@@ -585,8 +585,8 @@ sptc_status BatchEngine::run(hipStream_t s, bool P) {
     } else {
       ws_.ensure(c.n, c.rb, s);
       const int passes = radix_passes(c.bits, c.rb);
-      ws_.prepare(passes, s);
-      if (sort_needs_histogram()) histogram(ws_, kA_.get(), c.n, passes, s);
+      ws_.prepare(c.n, s);
+      if (sort_onesweep(c.n)) histogram(ws_, kA_.get(), c.n, passes, s);
       alt = sort_after_histogram(ws_, kA_.get(), vA_.get(), c.n, c.bits, s, kt, SPTC_K_SORT_PROD);
     }
     const uint64_t* sk = alt ? ws_.alt_keys.get() : kA_.get();

@@ -187,6 +187,8 @@ Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o) {
   for (auto& e : ev_) SPTC_HIP(hipEventCreate(&e));
   SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_total_), sizeof(U2) * 4, 0));
   SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_u64_), sizeof(uint64_t) * 8, 0));
+  ws_.err_host = reinterpret_cast<uint32_t*>(host_u64_ + 7);
+  *ws_.err_host = 0;
   // The budget caps what this call holds at once, on top of what was
   // already live when it started.
   const uint64_t live = DevicePool::get().live_bytes();
@@ -283,20 +285,28 @@ void Engine::prepare(const StagedCOO& t, const Layout& lay, Operand* out, const 
       a.idx[m] = t.idx[m];
     }
   }
-  SPTC_HIP(hipMemcpyAsync(out->vals.get(), t.val, n * sizeof(float),
-                          hipMemcpyDeviceToDevice, s_));
+  int tok = kt_.begin(s_);
+  if (!rb_ && sort_linearize_small(a, t.idx_bytes, t.val, n, out->keys.get(), out->vals.get(),
+                                   s_)) {
+    kt_.end(tok, SPTC_K_LINEARIZE, (double)n * (lay.order * t.idx_bytes + 16), s_);
+    return;
+  }
   const int rb = rb_ ? rb_ : choose_radix_bits(lay.nbits);
   const int passes = radix_passes(lay.nbits, rb);
   ws_.ensure(n, rb, s_);
-  ws_.prepare(passes, s_);
-  int tok = kt_.begin(s_);
-  const bool hist = sort_needs_histogram();
-  launch_linearize(a, t.idx_bytes, n, out->keys.get(), ws_.hist.get(),
+  ws_.prepare(n, s_);
+  const bool hist = sort_onesweep(n);
+  launch_linearize(a, t.idx_bytes, n, out->keys.get(), ws_.hist(),
                    hist && passes <= kMaxFusedPasses ? passes : 0, rb, s_);
   kt_.end(tok, SPTC_K_LINEARIZE, (double)n * (lay.order * t.idx_bytes + 8), s_);
+  if (!passes) {
+    SPTC_HIP(hipMemcpyAsync(out->vals.get(), t.val, n * sizeof(float), hipMemcpyDeviceToDevice,
+                            s_));
+    return;
+  }
   if (hist && passes > kMaxFusedPasses) histogram(ws_, out->keys.get(), n, passes, s_);
   if (sort_after_histogram(ws_, out->keys.get(), out->vals.get(), n, lay.nbits, s_, &kt_,
-                           SPTC_K_SORT_INPUT)) {
+                           SPTC_K_SORT_INPUT, t.val)) {
     std::swap(out->keys, ws_.alt_keys);
     std::swap(out->vals, ws_.alt_vals);
   }
@@ -363,9 +373,9 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
     const int bits = rbits + W;
     SPTC_HIP(hipMemcpyAsync(sorted.get(), key.get(), n * 8, hipMemcpyDeviceToDevice, s_));
     const int rb = rb_ ? rb_ : choose_radix_bits(bits);
-    ws_.ensure(n, rb, s_);
-    ws_.prepare(radix_passes(bits, rb), s_);
-    if (sort_needs_histogram()) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
+    ws_.ensure(n, rb, s_, /*vals=*/false);
+    ws_.prepare(n, s_);
+    if (sort_onesweep(n)) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
     const bool alt = sort_after_histogram(ws_, sorted.get(), nullptr, n, bits, s_);
     run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_, host_total_);
     U = wait_total().a;
@@ -449,9 +459,9 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       fk.reset(ny);
       launch_yfree_extract(Y.keys.get(), ny, low_mask(ynf), fk.get(), s_);
       const int rbf = rb_ ? rb_ : choose_radix_bits(ynf);
-      ws_.ensure(ny, rbf, s_);
-      ws_.prepare(radix_passes(ynf, rbf), s_);
-      if (sort_needs_histogram()) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
+      ws_.ensure(ny, rbf, s_, /*vals=*/false);
+      ws_.prepare(ny, s_);
+      if (sort_onesweep(ny)) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
       const bool alt = sort_after_histogram(ws_, fk.get(), nullptr, ny, ynf, s_);
       rtmp.reset(scan_tmp_count(ny) + 1);
       run_rank_sorted(alt ? ws_.alt_keys.get() : fk.get(), Y.keys.get(), ny, ynf, ro, rtmp.get(),
@@ -810,7 +820,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
         const int rb = rb_ ? rb_ : choose_radix_bits(bits);
         const int passes = radix_passes(bits, rb);
         ws_.ensure(n, rb, s_);
-        ws_.prepare(passes, s_);
+        if (!(kyf > 0 && kyf < bits && kyf <= 32 && prefer_row_sort())) ws_.prepare(n, s_);
         // row-segmented sort when the column bits leave row bits to skip
         const bool rowsort = kyf > 0 && kyf < bits && kyf <= 32 && prefer_row_sort();
         if (rowsort) {
@@ -858,8 +868,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
           ea.out_col32 = fcol;
           ea.out_vals = pv;
         }
-        ea.hist = ws_.hist.get();
-        const bool hist = sort_needs_histogram();
+        ea.hist = ws_.hist();
+        const bool hist = sort_onesweep(n);
         ea.passes = hist && passes <= kMaxFusedPasses ? passes : 0;
         ea.vsum = vsum.get();
         int tok = kt_.begin(s_);
@@ -969,13 +979,11 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   }
   double* const host_sum = reinterpret_cast<double*>(host_u64_ + 2);
   launch_fold_sums(vsum.get(), host_sum, s_);
-  host_u64_[0] = 0;
-  if (ws_.err()) SPTC_HIP(hipMemcpyAsync(host_u64_, ws_.err(), 4, hipMemcpyDeviceToHost, s_));
   record(5);
   SPTC_HIP(hipStreamSynchronize(s_));
   info.value_sum = *host_sum;
   kt_.collect(res->kstats, SPTC_K_COUNT);
-  if (*reinterpret_cast<uint32_t*>(host_u64_) != 0) {
+  if (*ws_.err() != 0) {
     msg = "radix sort look-back exceeded its spin limit";
     return SPTC_ERR_INTERNAL;
   }

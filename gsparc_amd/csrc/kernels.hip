@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void k_linearize(LinArgs a, uint64_t n,
         k |= shl64((uint64_t)static_cast<const IdxT*>(a.idx[m])[i] & low_mask(a.width[m]),
                    a.shift[m]);
     keys[i] = k;
-    if (passes) hist_add<RB>(sh, k, passes);
+    if (passes) hist_add_wave<RB>(sh, k, true, passes);
   }
   if (passes) {
     __syncthreads();
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kBlock) void k_linearize(LinArgs a, uint64_t n,
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
                       uint64_t* hist, int passes, int rb, hipStream_t s) {
   if (!n) return;
-  uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock * 4), 2048);
+  uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock * 4), passes ? 1024 : 2048);
   if (passes > kMaxFusedPasses) passes = 0;  // caller falls back to histogram()
 #define SPTC_LIN(T, RBV)                                                                   \
   hipLaunchKernelGGL((k_linearize<T, RBV>), dim3(grid), dim3(kBlock), 0, s, a, n, keys, hist, \

@@ -9,13 +9,6 @@ namespace sptc {
 constexpr int kMaxFusedPasses = 8;  // producers fuse histograms up to this many passes
 constexpr int kDirectBits = 22;     // direct-addressed Y segment table up to 2^22 keys
 
-struct LinArgs {
-  const void* idx[SPTC_MAX_ORDER];
-  int shift[SPTC_MAX_ORDER];
-  int width[SPTC_MAX_ORDER];
-  int order;
-};
-
 // Packed key of a group of contracted coordinates, above the previous
 // group's rank: key = prev << prev_shift | OR_j (idx_j & (2^w_j-1)) << s_j.
 struct TupleArgs {

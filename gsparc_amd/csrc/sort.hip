@@ -35,7 +35,7 @@ namespace {
 constexpr uint64_t kFlagAgg = 1ull << 62;
 constexpr uint64_t kFlagPre = 2ull << 62;
 constexpr uint64_t kValMask = (1ull << 48) - 1;
-constexpr uint32_t kSpinLimit = 1u << 28;
+constexpr uint32_t kSpinLimit = 1u << 24;
 
 __device__ __forceinline__ uint64_t pack_status(uint64_t flag, uint32_t epoch,
                                                 uint64_t v) {
@@ -74,46 +74,47 @@ __global__ __launch_bounds__(kBlock) void k_histogram(const uint64_t* __restrict
     if (sh[i2]) atomicAdd((unsigned long long*)&hist[i2], (unsigned long long)sh[i2]);
 }
 
-// hist [passes][R] counts -> base [passes][R] exclusive starts.  One block per
-// pass.
-template <int RB>
-__global__ __launch_bounds__(kBlock) void k_digit_scan(const uint64_t* __restrict__ hist,
-                                                       uint64_t* __restrict__ base) {
-  constexpr int R = 1 << RB;
-  constexpr int PER = (R + kBlock - 1) / kBlock;
-  __shared__ uint64_t scratch[kBlock / kWave];
-  const int p = blockIdx.x;
-  uint64_t local[PER];
-  uint64_t sum = 0;
-  for (int j = 0; j < PER; ++j) {
-    int d = threadIdx.x * PER + j;
-    local[j] = d < R ? hist[p * R + d] : 0;
-    sum += local[j];
-  }
-  uint64_t tot;
-  uint64_t ex = block_excl_scan<uint64_t>(sum, scratch, &tot);
-  for (int j = 0; j < PER; ++j) {
-    int d = threadIdx.x * PER + j;
-    if (d < R) base[p * R + d] = ex;
-    ex += local[j];
-  }
-}
-
+// One pass in one launch: a tile ranks its keys, publishes its digit counts and
+// takes the counts of the tiles before it from their status words (decoupled
+// look-back), eight words in flight per digit: with one at a time a tile whose
+// predecessors run beside it waits for as many loads as there are of them.
+// hist: the pass's digit counts over all keys; err (pinned host memory) is set
+// if a wait exceeds its limit.  Tiles are handed out by a counter, so every
+// predecessor of a running tile is running or done and each wait ends.
 // TAG only separates kernel symbols (0: operand sorts, 1: product sorts) so
 // profiles attribute time to the product sort on its own.
+constexpr int kLook = 8;
+
 template <int RB, int IPT, int NT, int TAG>
 __global__ __launch_bounds__(NT) void k_onesweep(
     const uint64_t* __restrict__ kin, const float* __restrict__ vin,
     uint64_t* __restrict__ kout, float* __restrict__ vout, uint64_t n, int shift,
-    const uint64_t* __restrict__ digit_base, uint64_t* status,
+    const uint64_t* __restrict__ hist, uint64_t* status,
     uint32_t* tile_counter, uint32_t epoch, uint32_t* err) {
   constexpr int R = 1 << RB;
   constexpr int TILE = NT * IPT;
+  constexpr int PER = (R + NT - 1) / NT;
   static_assert(TILE < 65536, "16-bit tile offsets");
   __shared__ TileSmem<RB, IPT, NT> sm;
   const uint32_t tid = threadIdx.x;
   if (tid == 0) sm.tile = atomicAdd(tile_counter, 1u);
   for (int i = tid; i < (NT / kWave) * R; i += NT) (&sm.cnt[0][0])[i] = 0;
+  {  // digit starts
+    uint32_t c[PER], sum = 0, all;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int d = tid * PER + j;
+      c[j] = d < R ? (uint32_t)hist[d] : 0;
+      sum += c[j];
+    }
+    uint32_t ex = block_scan_u32<NT>(sum, sm.scan, &all);  // barriers inside
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int d = tid * PER + j;
+      if (d < R) sm.gbase[d] = ex;
+      ex += c[j];
+    }
+  }
   __syncthreads();
   const uint64_t tile = sm.tile;
   const uint64_t tile_begin = tile * TILE;
@@ -132,28 +133,128 @@ __global__ __launch_bounds__(NT) void k_onesweep(
       st_agent(my, pack_status(kFlagPre, epoch, total));
     } else {
       st_agent(my, pack_status(kFlagAgg, epoch, total));
-      int64_t j = (int64_t)tile - 1;
+      int64_t j = (int64_t)tile - 1;  // the next tile to take
       uint32_t spins = 0;
-      while (j >= 0) {
-        const uint64_t st = ld_agent(status + (uint64_t)j * R + d);
-        const uint32_t se = (uint32_t)((st >> 48) & 0x3FFF);
-        const uint64_t fl = st & (3ull << 62);
-        if (se != epoch || fl == 0) {
-          if (++spins > kSpinLimit) { atomicOr(err, 1u); break; }
-          __builtin_amdgcn_s_sleep(1);
-          continue;
+      bool done = false;
+      while (!done) {
+        uint64_t st[kLook];
+#pragma unroll
+        for (int e = 0; e < kLook; ++e)
+          st[e] = j - e >= 0 ? ld_agent(status + (uint64_t)(j - e) * R + d) : 0;
+        bool wait = false;
+#pragma unroll
+        for (int e = 0; e < kLook; ++e) {
+          const uint64_t fl = st[e] & (3ull << 62);
+          if (done || wait) continue;
+          if (fl == 0 || (uint32_t)((st[e] >> 48) & 0x3FFF) != epoch) {
+            wait = true;  // not published yet
+            continue;
+          }
+          excl += st[e] & kValMask;
+          --j;
+          done = fl == kFlagPre;  // (tile 0 publishes a prefix)
         }
-        excl += st & kValMask;
-        if (fl == kFlagPre) break;
-        --j;
+        if (wait) {
+          if (++spins > kSpinLimit) {
+            if (err) *err = 1;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
       }
       st_agent(my, pack_status(kFlagPre, epoch, excl + total));
     }
-    sm.gbase[d] = (uint32_t)(digit_base[d] + excl);
+    sm.gbase[d] += (uint32_t)excl;
     sm.dstart[d] = (uint16_t)total;
   }
   __syncthreads();
   tile_stage_scatter<false, RB, IPT, NT>(sm, cnt, shift, k, v, pos, kout, vout);
+}
+
+// A sort of at most one tile's keys in one launch: linearize (or copy), then
+// every pass in LDS, on the bits that vary.  Bound by launches: small operands
+// were one for the keys, one for the values and three for each pass.  A call on
+// two operands of 4096 nonzeros went from 370 to 292 us (24 us per operand here).
+constexpr int kSmallNT = 512, kSmallIPT = 12, kSmallRB = 8;
+template <typename IdxT>
+__global__ __launch_bounds__(kSmallNT) void k_sort_small(LinArgs a, const float* __restrict__ val,
+                                                         uint32_t n,
+                                                         uint64_t* __restrict__ keys,
+                                                         float* __restrict__ vals) {
+  constexpr int RB = kSmallRB, IPT = kSmallIPT, NT = kSmallNT, R = 1 << RB;
+  __shared__ TileSmem<RB, IPT, NT> sm;
+  __shared__ float vbuf[NT * IPT];
+  __shared__ uint64_t s_or[NT / kWave], s_and[NT / kWave];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  uint64_t k[IPT], o = 0, an = ~0ull;
+  float v[IPT];
+  uint32_t pos[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const uint32_t p = tile_local<IPT>(i);
+    const uint32_t q = p < n ? p : 0;
+    k[i] = 0;
+#pragma unroll
+    for (int m = 0; m < SPTC_MAX_ORDER; ++m)
+      if (m < a.order)
+        k[i] |= shl64((uint64_t)static_cast<const IdxT*>(a.idx[m])[q] & low_mask(a.width[m]),
+                      a.shift[m]);
+    v[i] = val[q];
+    if (p < n) {
+      o |= k[i];
+      an &= k[i];
+    }
+  }
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    o |= __shfl_xor(o, d, kWave);
+    an &= __shfl_xor(an, d, kWave);
+  }
+  if (lane == 0) {
+    s_or[wave] = o;
+    s_and[wave] = an;
+  }
+  __syncthreads();
+  for (int w = 0; w < NT / kWave; ++w) {
+    o |= s_or[w];
+    an &= s_and[w];
+  }
+  const uint64_t vary = o & ~an;
+  const int lo = vary ? __builtin_ctzll(vary) : 0, hi = vary ? 64 - __builtin_clzll(vary) : 0;
+  for (int shift = lo; shift < hi; shift += RB) {
+    if (!((vary >> shift) & (R - 1))) continue;  // a digit that all keys share
+    for (int i = tid; i < (NT / kWave) * R; i += NT) (&sm.cnt[0][0])[i] = 0;
+    __syncthreads();
+    tile_rank<false, RB, IPT, NT>(sm, n, shift, k, pos);
+    __syncthreads();
+    tile_prefix_fold<RB, IPT, NT>(sm);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) {
+      if (tile_local<IPT>(i) < n) {
+        const uint32_t q = pos[i] + (uint32_t)sm.cnt[wave][(uint32_t)(k[i] >> shift) & (R - 1)];
+        sm.buf[q] = k[i];
+        vbuf[q] = v[i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) {
+      const uint32_t p = tile_local<IPT>(i);
+      if (p < n) {
+        k[i] = sm.buf[p];
+        v[i] = vbuf[p];
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const uint32_t p = tile_local<IPT>(i);
+    if (p < n) {
+      keys[p] = k[i];
+      vals[p] = v[i];
+    }
+  }
 }
 
 template <int RB, int IPT, int NT>
@@ -215,18 +316,19 @@ struct CountScanOp {
 };
 
 // ---- tile configuration ---------------------------------------------------
-// SPTC_SORT selects the pass algorithm ("rts" default, "onesweep");
+// SPTC_SORT selects the pass algorithm ("rts", "onesweep"; by size without it);
 // SPTC_SORT_TILE the 8-bit-digit tile as threads x items ("512x12" default,
 // "512x16", "256x16", "256x12").  9-bit digits use 512x12, wider ones 256x12.
 struct SortCfg {
-  bool onesweep = false;
+  int mode = 0;  // 0: by size, 1: rts, 2: onesweep
   int nt = 512;
   int ipt = 12;
 };
 const SortCfg& sort_cfg() {
   static const SortCfg c = [] {
     SortCfg r;
-    if (const char* e = getenv("SPTC_SORT")) r.onesweep = std::string(e) == "onesweep";
+    if (const char* e = getenv("SPTC_SORT"))
+      r.mode = std::string(e) == "onesweep" ? 2 : std::string(e) == "rts" ? 1 : 0;
     if (const char* e = getenv("SPTC_SORT_TILE")) {
       const std::string t(e);
       if (t == "256x16") { r.nt = 256; r.ipt = 16; }
@@ -277,14 +379,12 @@ struct OnesweepPass {
     const int tok = a.kt ? a.kt->begin(a.s) : -1;
     if (a.tag)
       hipLaunchKernelGGL((k_onesweep<RB, IPT, NT, 1>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
-                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->base.get() + a.pass * R,
-                         a.ws->status.get(), a.ws->counters.get() + a.pass, a.ws->epoch,
-                         a.ws->err());
+                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->hist() + a.pass * R,
+                         a.ws->status(), a.ws->counters() + a.pass, a.ws->epoch, a.ws->err());
     else
       hipLaunchKernelGGL((k_onesweep<RB, IPT, NT, 0>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
-                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->base.get() + a.pass * R,
-                         a.ws->status.get(), a.ws->counters.get() + a.pass, a.ws->epoch,
-                         a.ws->err());
+                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->hist() + a.pass * R,
+                         a.ws->status(), a.ws->counters() + a.pass, a.ws->epoch, a.ws->err());
     if (a.kt) a.kt->end(tok, a.cls, 24.0 * (double)a.n, a.s);
   }
 };
@@ -348,48 +448,50 @@ int choose_radix_bits(int nbits) {
   return 8;
 }
 
-bool sort_needs_histogram() { return sort_cfg().onesweep; }
+bool sort_onesweep(uint64_t n) {
+  const int m = sort_cfg().mode;
+  return m == 2 || (m == 0 && n <= kOnesweepMax);
+}
 
 uint64_t SortWorkspace::bytes_per_key(int rb) {
   // alt keys + values, look-back words, and the two count matrices
   return sizeof(uint64_t) + sizeof(float) + (16ull << rb) / sort_tile_items(rb) + 1;
 }
 
-void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s) {
+void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s, bool vals) {
+  (void)s;
   const uint64_t R = 1ull << rb_;
-  if (sort_cfg().onesweep && counters.size() == 0) {
-    counters.reset(64);
-    fill_u32(counters.get(), 0, 64, s);
-  }
-  if (sort_cfg().onesweep && hist.size() < kMaxPasses * R) {
-    hist.reset(kMaxPasses * R);
-    base.reset(kMaxPasses * R);
-  }
-  if (alt_keys.size() < n || alt_vals.size() < n) {
-    alt_keys.reset(n ? n : 1);
-    alt_vals.reset(n ? n : 1);
-  }
+  if (alt_keys.size() < n) alt_keys.reset(n ? n : 1);
+  if (vals && alt_vals.size() < n) alt_vals.reset(n ? n : 1);
   const uint64_t tiles = ceil_div(n ? n : 1, sort_tile_items(rb_));
-  if (sort_cfg().onesweep && status.size() < tiles * R) {
-    status.reset(tiles * R);
-    fill_u64(status.get(), 0, tiles * R, s);
-    epoch = 0;
-  }
-  if (!sort_cfg().onesweep && rts_cnt.size() < tiles * R) {
+  rb = rb_;
+  if (sort_onesweep(n)) {
+    if (sweep.size() < kMaxPasses * R + kSweepHead + tiles * R)
+      sweep.reset(kMaxPasses * R + kSweepHead + tiles * R);
+  } else if (rts_cnt.size() < tiles * R) {
     rts_cnt.reset(tiles * R);
     rts_off.reset(tiles * R);
     rts_tmp.reset(scan_tmp_count(tiles * R) + 1);
   }
-  rb = rb_;
-  cap = alt_keys.size();
-  max_tiles = status.size() / R;
 }
 
-void SortWorkspace::prepare(int passes, hipStream_t s) {
-  if (!sort_cfg().onesweep) return;
-  uint64_t R = 1ull << rb;
-  fill_u64(hist.get(), 0, (uint64_t)passes * R, s);
-  fill_u32(counters.get(), 0, kMaxPasses, s);
+void SortWorkspace::prepare(uint64_t n, hipStream_t s) {
+  if (!sort_onesweep(n)) return;
+  const uint64_t R = 1ull << rb;
+  fill_u64(sweep.get(), 0, kMaxPasses * R + kSweepHead + ceil_div(n, sort_tile_items(rb)) * R, s);
+  epoch = 0;
+}
+
+bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
+                          uint64_t* keys, float* vals, hipStream_t s) {
+  if (n > (uint64_t)kSmallNT * kSmallIPT || sort_cfg().mode) return false;
+  if (idx_bytes == 4)
+    hipLaunchKernelGGL(k_sort_small<uint32_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
+                       keys, vals);
+  else
+    hipLaunchKernelGGL(k_sort_small<uint64_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
+                       keys, vals);
+  return true;
 }
 
 void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
@@ -398,59 +500,46 @@ void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
   uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock * 8), 2048);
   switch (ws.rb) {
     case 9: hipLaunchKernelGGL(k_histogram<9>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
-                               ws.hist.get()); break;
+                               ws.hist()); break;
     case 10: hipLaunchKernelGGL(k_histogram<10>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
-                                ws.hist.get()); break;
+                                ws.hist()); break;
     case 11: hipLaunchKernelGGL(k_histogram<11>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
-                                ws.hist.get()); break;
+                                ws.hist()); break;
     default: hipLaunchKernelGGL(k_histogram<8>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
-                                ws.hist.get()); break;
+                                ws.hist()); break;
   }
 }
 
-// vals NULL: the keys alone are moved.
+// vals NULL: the keys alone are moved; vsrc: the values are read from there
+// instead of vals (which the second pass writes).
 // Sorts keys/vals (n <= ws.cap, n < 2^32) on bits [0, nbits).  With the
 // onesweep algorithm ws.hist must hold the digit histograms of all passes.
 // Result ends in (keys, vals) when the pass count is even, else in
 // (ws.alt_keys, ws.alt_vals); the returned flag says which (true = alt).
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
-                          uint64_t n, int nbits, hipStream_t s, KTimer* kt, int cls) {
+                          uint64_t n, int nbits, hipStream_t s, KTimer* kt, int cls,
+                          const float* vsrc) {
   const int rb = ws.rb;
   const int passes = radix_passes(nbits, rb);
   if (!n || !passes) return false;
   if (n >= (1ull << 32)) throw std::length_error("radix sort of 2^32 or more keys");
-  const bool onesweep = sort_cfg().onesweep;
-  if (onesweep) {
-    switch (rb) {
-      case 9: hipLaunchKernelGGL(k_digit_scan<9>, dim3(passes), dim3(kBlock), 0, s,
-                                 ws.hist.get(), ws.base.get()); break;
-      case 10: hipLaunchKernelGGL(k_digit_scan<10>, dim3(passes), dim3(kBlock), 0, s,
-                                  ws.hist.get(), ws.base.get()); break;
-      case 11: hipLaunchKernelGGL(k_digit_scan<11>, dim3(passes), dim3(kBlock), 0, s,
-                                  ws.hist.get(), ws.base.get()); break;
-      default: hipLaunchKernelGGL(k_digit_scan<8>, dim3(passes), dim3(kBlock), 0, s,
-                                  ws.hist.get(), ws.base.get()); break;
-    }
-  }
-  const uint64_t R = 1ull << rb;
+  const bool onesweep = sort_onesweep(n);
   const uint64_t tiles = ceil_div(n, sort_tile_items(rb));
   const int tag = (cls == SPTC_K_SORT_PROD || cls == SPTC_K_SORT_PROD_WIDE) ? 1 : 0;
   const int kcls = (cls == SPTC_K_SORT_PROD && rb > 8) ? SPTC_K_SORT_PROD_WIDE : cls;
   PassArgs a{tag, &ws, keys, vals, ws.alt_keys.get(), vals ? ws.alt_vals.get() : nullptr, n, tiles,
              0, s, kt, kcls};
+  if (vsrc) a.va = const_cast<float*>(vsrc);  // read by the first pass only
   for (int p = 0; p < passes; ++p) {
     a.pass = p;
     if (onesweep) {
-      ws.epoch = (ws.epoch + 1) & 0x3FFF;
-      if (ws.epoch == 0) {
-        fill_u64(ws.status.get(), 0, ws.max_tiles * R, s);
-        ws.epoch = 1;
-      }
+      ++ws.epoch;  // (passes fit the status words' 14 bits)
       with_tile(rb, OnesweepPass{a});
     } else {
       with_tile(rb, RtsPass{a});
     }
     std::swap(a.ka, a.kb);
+    if (p == 0 && vsrc) a.va = vals;
     std::swap(a.va, a.vb);
   }
   return (passes & 1) != 0;

@@ -9,48 +9,67 @@ namespace sptc {
 
 constexpr int kMaxPasses = 16;
 
+struct LinArgs {
+  const void* idx[SPTC_MAX_ORDER];
+  int shift[SPTC_MAX_ORDER];
+  int width[SPTC_MAX_ORDER];
+  int order;
+};
+
 struct SortWorkspace {
   int rb = 8;                   // radix bits per pass
-  uint64_t cap = 0;             // max keys
-  uint64_t max_tiles = 0;
   DevBuf<uint64_t> alt_keys;
   DevBuf<float> alt_vals;
-  DevBuf<uint64_t> status;      // [max_tiles][R] look-back words
-  DevBuf<uint64_t> hist;        // [kMaxPasses][R] digit counts
-  DevBuf<uint64_t> base;        // [kMaxPasses][R] digit starts
-  DevBuf<uint32_t> counters;    // [kMaxPasses] tile counters, [32] error flag
+  // onesweep: [kMaxPasses][R] digit counts, kSweepHead words of tile counters,
+  // [tiles][R] look-back words -- one fill clears them
+  DevBuf<uint64_t> sweep;
+  static constexpr uint64_t kSweepHead = 32;
   DevBuf<uint32_t> rts_cnt;     // [R][tiles] per-tile digit counts
   DevBuf<uint32_t> rts_off;     // [R][tiles] their exclusive scan
   DevBuf<U2> rts_tmp;           // scan scratch
   uint32_t epoch = 0;
+  uint32_t* err_host = nullptr; // pinned host memory, set by a failed look-back
 
-  // Grows the workspace to hold `n` keys at `rb` radix bits.
-  void ensure(uint64_t n, int rb, hipStream_t s);
-  // Clears histograms and tile counters before a producer accumulates (used by
-  // the onesweep passes alone).
-  void prepare(int passes, hipStream_t s);
-  // look-back error flag (NULL: no onesweep pass has run)
-  uint32_t* err() const { return counters.size() ? counters.get() + 32 : nullptr; }
+  // Grows the workspace to hold `n` keys (and values) at `rb` radix bits.
+  void ensure(uint64_t n, int rb, hipStream_t s, bool vals = true);
+  // Clears histograms, counters and look-back words before a sort of n keys
+  // (onesweep only).
+  void prepare(uint64_t n, hipStream_t s);
+  uint64_t* hist() const { return sweep.get(); }
+  uint32_t* counters() const {
+    return reinterpret_cast<uint32_t*>(sweep.get() + ((uint64_t)kMaxPasses << rb));
+  }
+  uint64_t* status() const { return sweep.get() + ((uint64_t)kMaxPasses << rb) + kSweepHead; }
+  uint32_t* err() const { return err_host; }
   static uint64_t bytes_per_key(int rb);
 };
 
 int radix_passes(int nbits, int rb);
 uint64_t sort_tile_items(int rb);
 bool radix_bits_supported(int rb);
-// True when the configured pass algorithm needs up-front digit histograms
-// (onesweep); reduce-then-scan counts per tile itself.
-bool sort_needs_histogram();
+// True when n keys are sorted by one-launch passes with look-back, which need
+// the digit histograms of all passes up front (ws.prepare, then a producer or
+// histogram()); reduce-then-scan passes count per tile themselves.
+// The line: 0.3e6 pairs of 40 bits 178 us against 322, 1e6 (with linearize) 303
+// against 348, 3e6 326 against 290, 77e6 4.5 ms against 3.8: past a few tiles per
+// CU the look-back's status words cost more than the launches they save.
+constexpr uint64_t kOnesweepMax = 1ull << 21;
+bool sort_onesweep(uint64_t n);
+// Linearizes and sorts up to one tile of nonzeros in one launch; false when
+// there are more.
+bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
+                          uint64_t* keys, float* vals, hipStream_t s);
 // Digit width for a sort over nbits key bits (fewest passes, digits <= 10).
 int choose_radix_bits(int nbits);
 void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
                int passes, hipStream_t s);
-// Sorts (keys, vals) on bits [0, nbits), ws.hist holding the histograms of
-// all passes.  Returns true when the sorted data ended in (ws.alt_keys,
+// Sorts (keys, vals) on bits [0, nbits), ws.hist() holding the histograms of
+// all passes for sizes that sort_onesweep.  Returns true when the sorted data ended in (ws.alt_keys,
 // ws.alt_vals) (odd pass count).
 // kt (optional) times every pass under kernel class `cls`.
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
                           uint64_t n, int nbits, hipStream_t s, KTimer* kt = nullptr,
-                          int cls = 0);
+                          int cls = 0, const float* vsrc = nullptr);
 
 // Device-side histogram accumulation for producers: call once per key with
 // an LDS array of passes*R uint32 cleared by the block, then flush.
