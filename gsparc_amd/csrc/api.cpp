@@ -854,33 +854,9 @@ sptc_status sptc_index_match(const uint64_t* xkeys, uint64_t nx, const uint64_t*
   if (!device_ok()) return fail(SPTC_ERR_NO_DEVICE, "no GPU");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   try {
-    DevBuf<uint64_t> tlo, thi, ukey, ustart;
-    YTable tab;
-    std::memset(&tab, 0, sizeof(tab));
-    if (ncbits <= kDirectBits) {
-      const uint64_t K = 1ull << ncbits;
-      tlo.reset(K);
-      thi.reset(K);
-      fill_u64(tlo.get(), 0, K, s);
-      fill_u64(thi.get(), 0, K, s);
-      launch_ytable_direct(ykeys, ny, y_nfbits, K, tlo.get(), thi.get(), s);
-      tab.direct = 1;
-      tab.lo = tlo.get();
-      tab.hi = thi.get();
-    } else {
-      ukey.reset(ny + 1);
-      ustart.reset(ny + 1);
-      DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-      run_yunique(ykeys, ny, y_nfbits, ukey.get(), ustart.get(), tmp.get(), s);
-      U2 t;
-      SPTC_HIP(hipMemcpyAsync(&t, tmp.get() + scan_tmp_count(ny), sizeof(U2),
-                              hipMemcpyDeviceToHost, s));
-      SPTC_HIP(hipStreamSynchronize(s));
-      tab.direct = 0;
-      tab.ukey = ukey.get();
-      tab.ustart = ustart.get();
-      tab.U = t.a;
-    }
+    const int tbits = ytable_bits(ncbits, ny);
+    DevBuf<U2> tmem(1ull << tbits);
+    const YTable tab = build_ytable(tmem.get(), tbits, ykeys, ny, ncbits, y_nfbits, s);
     MatchOut mo;
     std::memset(&mo, 0, sizeof(mo));
     mo.mpos = mpos;

@@ -148,33 +148,10 @@ uint64_t count_products(const Operand& X, const Operand& Y, hipStream_t s) {
   const uint64_t nx = X.nnz, ny = Y.nnz;
   if (!nx || !ny) return 0;
   const int ncb = X.lay.ncbits, ynf = Y.lay.nfbits;
-  DevBuf<uint64_t> tlo, thi, ukey, ustart;
-  YTable tab;
-  std::memset(&tab, 0, sizeof(tab));
+  const int tbits = ytable_bits(ncb, ny);
+  DevBuf<U2> tmem(1ull << tbits);
+  const YTable tab = build_ytable(tmem.get(), tbits, Y.keys.get(), ny, ncb, ynf, s);
   U2 host;
-  if (ncb <= kDirectBits) {
-    const uint64_t K = 1ull << ncb;
-    tlo.reset(K);
-    thi.reset(K);
-    fill_u64(tlo.get(), 0, K, s);
-    fill_u64(thi.get(), 0, K, s);
-    launch_ytable_direct(Y.keys.get(), ny, ynf, K, tlo.get(), thi.get(), s);
-    tab.direct = 1;
-    tab.lo = tlo.get();
-    tab.hi = thi.get();
-  } else {
-    ukey.reset(ny + 1);
-    ustart.reset(ny + 1);
-    DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-    run_yunique(Y.keys.get(), ny, ynf, ukey.get(), ustart.get(), tmp.get(), s);
-    SPTC_HIP(hipMemcpyAsync(&host, tmp.get() + scan_tmp_count(ny), sizeof(U2),
-                            hipMemcpyDeviceToHost, s));
-    SPTC_HIP(hipStreamSynchronize(s));
-    tab.direct = 0;
-    tab.ukey = ukey.get();
-    tab.ustart = ustart.get();
-    tab.U = host.a;
-  }
   DevBuf<U2> tmp(scan_tmp_count(nx) + 1);
   run_match_count(X.keys.get(), nx, ncb, tab, tmp.get(), s);
   SPTC_HIP(hipMemcpyAsync(&host, tmp.get() + scan_tmp_count(nx), sizeof(U2),
@@ -470,36 +447,12 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   }
 
   // ---- (c) index match ---------------------------------------------------
-  // ydup / hdup: set when Y holds duplicate coordinates
-  DevBuf<uint64_t> tlo, ukey, ustart;
-  uint64_t* ydup = nullptr;
+  // hdup: set when Y holds duplicate coordinates
   uint64_t* const hdup = &host_total_[3].a;
   *hdup = 0;
-  YTable tab;
-  std::memset(&tab, 0, sizeof(tab));
-  if (ncb <= kDirectBits) {
-    const uint64_t K = 1ull << ncb;
-    tlo.reset(2 * K + 1);  // the table and the duplicate flag, one fill
-    fill_u64(tlo.get(), 0, 2 * K + 1, s_);
-    ydup = tlo.get() + 2 * K;
-    launch_ytable_direct(Y.keys.get(), ny, ynf, K, tlo.get(), tlo.get() + K, s_, ydup, hdup);
-    tab.direct = 1;
-    tab.lo = tlo.get();
-    tab.hi = tlo.get() + K;
-  } else {
-    ukey.reset(ny + 1);
-    ustart.reset(ny + 1);
-    DevBuf<U2> tmp(scan_tmp_count(ny) + 1);
-    tlo.reset(1);
-    ydup = tlo.get();
-    fill_u64(ydup, 0, 1, s_);
-    launch_any_dup(Y.keys.get(), ny, ydup, hdup, s_);
-    run_yunique(Y.keys.get(), ny, ynf, ukey.get(), ustart.get(), tmp.get(), s_, host_total_);
-    tab.direct = 0;
-    tab.ukey = ukey.get();
-    tab.ustart = ustart.get();
-    tab.U = wait_total().a;
-  }
+  const int tbits = ytable_bits(ncb, ny);
+  DevBuf<U2> tmem((1ull << tbits) + 1);
+  const YTable tab = build_ytable(tmem.get(), tbits, Y.keys.get(), ny, ncb, ynf, s_, hdup);
   DevBuf<uint64_t> act_prefix(nx + 1), act_ypos(nx + 1), row_key(nx + 1), row_prod(nx + 1),
       row_act(nx + 1);
   DevBuf<float> act_xval(nx + 1);
@@ -516,8 +469,12 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   U2 tot;
   {
     DevBuf<U2> tmp(scan_tmp_count(nx) + 1);
+    // (a tight budget runs the lookups twice instead of keeping them)
+    DevBuf<uint64_t> look;
+    if (nx > kScanOneMax && 16 * nx <= budget_avail() / 16) look.reset(2 * nx);
     int tok = kt_.begin(s_);
-    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_, host_total_);
+    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_, host_total_,
+              look.size() ? look.get() : nullptr);
     // keys read twice, plus the compacted active and row tables written
     kt_.end(tok, SPTC_K_MATCH, (double)nx * (16 + 24 + 24), s_);
     tot = wait_total();
@@ -525,8 +482,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   const uint64_t ir = tot.a;
   const uint64_t A = tot.b >> 32;
   const uint64_t R = tot.b & 0xFFFFFFFFull;
-  ukey.release();
-  ustart.release();
+  tmem.release();
   record(3);
   // width of the column field and the columns: the distinct free keys
   const uint64_t ranks = ranked ? host_total_[1].a : ynf < 32 ? 1ull << ynf : 0;
@@ -786,7 +742,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       ra.ytab32 = ytab32.size() ? ytab32.get() : nullptr;
       ra.K = (uint32_t)ranks;
       ra.short_max = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(ranks / 128, 256), kGroupHalf);
-      ra.ydup = ydup;
+      ra.ydup = *hdup != 0;
       ra.vsum = vsum.get();
     }
     // verbose: a progress line on stderr at least every 10 s of chunks

@@ -182,18 +182,16 @@ void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* key
 // (c) Index match.
 //
 // Y is sorted by key = c << y_nfbits | f, so every contract value c owns one
-// contiguous segment.  With a small contract field (ncbits <= kDirectBits)
-// the segment table is direct-addressed: lo[c], hi[c]; otherwise it is the
-// compacted list of distinct c with their start offsets, searched per X
-// nonzero.
+// contiguous segment.  A table over c's top bits (ytable_bits) holds where each
+// range of c's starts and ends among the keys; ranges of one c need no more,
+// others compare the range's first and last key and search between them.
 
 // dup / hdup (device / pinned host, may be NULL; cleared by the caller): set
 // when two Y keys are equal.
-__global__ __launch_bounds__(kBlock) void k_ytable_direct(const uint64_t* __restrict__ ykeys,
-                                                          uint64_t ny, int ynf, uint64_t K,
-                                                          uint64_t* __restrict__ lo,
-                                                          uint64_t* __restrict__ hi,
-                                                          uint64_t* dup, uint64_t* hdup) {
+__global__ __launch_bounds__(kBlock) void k_ytable(const uint64_t* __restrict__ ykeys, uint64_t ny,
+                                                   int ynf, int sh, uint64_t K,
+                                                   U2* __restrict__ tab, uint64_t* dup,
+                                                   uint64_t* hdup) {
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   bool same = false;
@@ -201,10 +199,10 @@ __global__ __launch_bounds__(kBlock) void k_ytable_direct(const uint64_t* __rest
     const uint64_t k = ykeys[i];
     const uint64_t prev = i ? ykeys[i - 1] : 0, next = i + 1 < ny ? ykeys[i + 1] : 0;
     same |= i && prev == k;
-    const uint64_t c = shr64(k, ynf);
-    if (c >= K) continue;  // key outside the contract field: matches nothing
-    if (i == 0 || shr64(prev, ynf) != c) lo[c] = i;
-    if (i == ny - 1 || shr64(next, ynf) != c) hi[c] = i + 1;
+    const uint64_t h = shr64(shr64(k, ynf), sh);
+    if (h >= K) continue;  // key outside the contract field: matches nothing
+    if (i == 0 || shr64(shr64(prev, ynf), sh) != h) tab[h].a = i;
+    if (i == ny - 1 || shr64(shr64(next, ynf), sh) != h) tab[h].b = i + 1;
   }
   if (dup && __ballot(same) && lane_id() == 0) {
     *dup = 1;
@@ -212,63 +210,54 @@ __global__ __launch_bounds__(kBlock) void k_ytable_direct(const uint64_t* __rest
   }
 }
 
-void launch_ytable_direct(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t K,
-                          uint64_t* lo, uint64_t* hi, hipStream_t s, uint64_t* dup,
-                          uint64_t* hdup) {
-  if (!ny) return;
-  uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(ny, kBlock), 4096);
-  hipLaunchKernelGGL(k_ytable_direct, dim3(grid), dim3(kBlock), 0, s, ykeys, ny, ynf, K, lo,
-                     hi, dup, hdup);
+YTable build_ytable(U2* tab, int bits, const uint64_t* ykeys, uint64_t ny, int ncbits, int ynf,
+                    hipStream_t s, uint64_t* hdup) {
+  const uint64_t K = 1ull << bits;
+  YTable t{tab, ykeys, ny, ncbits - bits, ynf};
+  fill_u64(reinterpret_cast<uint64_t*>(tab), 0, 2 * K + (hdup ? 1 : 0), s);
+  if (!ny) return t;
+  const uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(ny, kBlock), 4096);
+  hipLaunchKernelGGL(k_ytable, dim3(grid), dim3(kBlock), 0, s, ykeys, ny, ynf, t.sh, K, tab,
+                     hdup ? &tab[K].a : nullptr, hdup);
+  return t;
 }
 
-struct YUniqueOp {
-  const uint64_t* ykeys;
-  uint64_t ny;
-  int ynf;
-  uint64_t* ukey;
-  uint64_t* ustart;
-  __device__ U2 value(uint64_t i) const {
-    return mk2(i == 0 || shr64(ykeys[i - 1], ynf) != shr64(ykeys[i], ynf), 0);
-  }
-  __device__ void emit(uint64_t i, U2 excl, U2 v) const {
-    if (v.a) {
-      ukey[excl.a] = shr64(ykeys[i], ynf);
-      ustart[excl.a] = i;
+// c's segment {pos, cnt} in the range r of keys, whose contract values start at
+// first and end at last (both read by the caller; of no meaning if r is empty).
+__device__ __forceinline__ U2 segment_in(const YTable& t, uint64_t c, const U2& r, uint64_t first,
+                                         uint64_t last) {
+  if (r.a >= r.b || c < first || c > last) return mk2(0, 0);
+  uint64_t lo = r.a, hi = r.b;
+  if (first != c) {  // keys[lo] < c <= keys[hi - 1]
+    uint64_t e = hi - 1;
+    while (lo + 1 < e) {
+      const uint64_t mid = (lo + e) >> 1;
+      if (shr64(t.ykeys[mid], t.ynf) < c) lo = mid; else e = mid;
     }
-    if (i == ny - 1) ustart[excl.a + v.a] = ny;
+    lo = e;
+    if (shr64(t.ykeys[lo], t.ynf) != c) return mk2(0, 0);
   }
-};
-
-void run_yunique(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t* ukey,
-                 uint64_t* ustart, U2* tmp, hipStream_t s,
-                 U2* host) {
-  YUniqueOp op{ykeys, ny, ynf, ukey, ustart};
-  run_scan(op, ny, tmp, s, true, host);
+  if (last != c) {  // keys[lo] == c < keys[hi - 1]
+    uint64_t e = lo;
+    --hi;
+    while (e + 1 < hi) {
+      const uint64_t mid = (e + hi) >> 1;
+      if (shr64(t.ykeys[mid], t.ynf) == c) e = mid; else hi = mid;
+    }
+  }
+  return mk2(lo, hi - lo);
 }
 
-__device__ __forceinline__ void ytable_lookup(const YTable& t, uint64_t c,
-                                              uint64_t& pos, uint64_t& cnt) {
-  if (t.direct) {
-    uint64_t l = t.lo[c], h = t.hi[c];
-    pos = l;
-    cnt = h - l;
-  } else {
-    uint64_t lo = 0, hi = t.U;
-    while (lo < hi) {
-      uint64_t mid = (lo + hi) >> 1;
-      if (t.ukey[mid] < c) lo = mid + 1; else hi = mid;
-    }
-    if (lo < t.U && t.ukey[lo] == c) {
-      pos = t.ustart[lo];
-      cnt = t.ustart[lo + 1] - pos;
-    } else {
-      pos = 0;
-      cnt = 0;
-    }
-  }
+__device__ __forceinline__ U2 ytable_lookup(const YTable& t, uint64_t c) {
+  const U2 r = t.tab[shr64(c, t.sh)];
+  if (t.sh == 0) return mk2(r.a, r.b - r.a);
+  if (r.a >= r.b) return mk2(0, 0);
+  return segment_in(t, c, r, shr64(t.ykeys[r.a], t.ynf), shr64(t.ykeys[r.b - 1], t.ynf));
 }
 
 // value: a = match count; b = (active << 32) | row_head
+// STORED: the lookups' results are read from lpos and lcnt.
+template <bool STORED>
 struct MatchOp {
   const uint64_t* xkeys;
   const float* xvals;
@@ -278,6 +267,8 @@ struct MatchOp {
   YTable t;
   MatchOut o;
   int api;  // 1: write mpos/mcnt/prefix (per-phase entry point)
+  const uint64_t* lpos;
+  const uint64_t* lcnt;
 
   // the X key's Y segment start, from value() to emit() in registers
   struct Aux {
@@ -285,17 +276,25 @@ struct MatchOp {
   };
   __device__ U2 value(uint64_t i, Aux& x) const {
     const uint64_t k = xkeys[i];
-    uint64_t pos, cnt;
-    ytable_lookup(t, k & cmask, pos, cnt);
-    x.pos = pos;
+    uint64_t cnt;
+    if (STORED) {
+      x.pos = lpos[i];
+      cnt = lcnt[i];
+    } else {
+      const U2 m = ytable_lookup(t, k & cmask);
+      x.pos = m.a;
+      cnt = m.b;
+    }
     const uint64_t head = (i == 0) || (shr64(xkeys[i - 1], ncbits) != shr64(k, ncbits));
     return mk2(cnt, ((uint64_t)(cnt != 0) << 32) | head);
   }
   __device__ void emit(uint64_t i, U2 excl, U2 v, const Aux& x) const {
     const uint64_t pos = x.pos, cnt = v.a;
     if (api) {
-      o.mpos[i] = cnt ? pos : 0;
-      o.mcnt[i] = cnt;
+      if (!STORED) {
+        o.mpos[i] = cnt ? pos : 0;
+        o.mcnt[i] = cnt;
+      }
       o.prefix[i] = excl.a;
       if (i == nx - 1) o.prefix[nx] = excl.a + v.a;
       return;
@@ -323,17 +322,89 @@ struct MatchOp {
   }
 };
 
+// The lookups of one scan tile and the tile's sums (the reduce half of the
+// match's scan).  Bound by the reads at random addresses, so each thread's 8
+// table entries, then its 8 first and last keys, are requested together; EXACT
+// tables (one contract value per entry) need no keys.  8e6 X keys against 3e6 Y
+// keys of 28 contract bits: 359 us here and 104 us in the emit, where searches
+// over the distinct contract values, run by both halves, took 859 and 804.
+template <bool EXACT>
+__global__ __launch_bounds__(kBlock) void k_match_lookup(const uint64_t* __restrict__ xkeys,
+                                                         uint64_t nx, uint64_t cmask, int ncbits,
+                                                         YTable t, uint64_t* __restrict__ lpos,
+                                                         uint64_t* __restrict__ lcnt,
+                                                         U2* __restrict__ tile_sums) {
+  __shared__ U2 scratch[kBlock / kWave];
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x;
+  uint64_t k[kScanItems], prev[kScanItems];
+  U2 r[kScanItems];
+#pragma unroll
+  for (int e = 0; e < kScanItems; ++e) {
+    const uint64_t i = base + (uint64_t)e * kBlock, j = i < nx ? i : nx - 1;
+    k[e] = xkeys[j];
+    prev[e] = xkeys[j ? j - 1 : 0];
+  }
+#pragma unroll
+  for (int e = 0; e < kScanItems; ++e) r[e] = t.tab[shr64(k[e] & cmask, t.sh)];
+  uint64_t first[kScanItems], last[kScanItems];
+  if (!EXACT) {
+#pragma unroll
+    for (int e = 0; e < kScanItems; ++e) {
+      first[e] = t.ykeys[r[e].a];  // (an empty range is {0, 0})
+      last[e] = t.ykeys[r[e].b ? r[e].b - 1 : 0];
+    }
+  }
+  U2 s = mk2(0, 0);
+#pragma unroll
+  for (int e = 0; e < kScanItems; ++e) {
+    const uint64_t i = base + (uint64_t)e * kBlock;
+    if (i >= nx) continue;
+    const U2 m = EXACT ? mk2(r[e].a, r[e].b - r[e].a)
+                       : segment_in(t, k[e] & cmask, r[e], shr64(first[e], t.ynf),
+                                    shr64(last[e], t.ynf));
+    if (lpos) {
+      lpos[i] = m.b ? m.a : 0;
+      lcnt[i] = m.b;
+    }
+    const uint64_t head = i == 0 || shr64(prev[e], ncbits) != shr64(k[e], ncbits);
+    s = s + mk2(m.b, ((uint64_t)(m.b != 0) << 32) | head);
+  }
+  U2 tot;
+  block_excl_scan_u2(s, scratch, &tot);
+  if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
+}
+
+void launch_match_lookup(const uint64_t* xkeys, uint64_t nx, int ncbits, const YTable& t,
+                         uint64_t* lpos, uint64_t* lcnt, U2* tmp, hipStream_t s) {
+  const dim3 grid((uint32_t)scan_tmp_count(nx)), nt(kBlock);
+  if (t.sh == 0 || t.ny == 0)
+    hipLaunchKernelGGL(k_match_lookup<true>, grid, nt, 0, s, xkeys, nx, low_mask(ncbits), ncbits, t,
+                       lpos, lcnt, tmp);
+  else
+    hipLaunchKernelGGL(k_match_lookup<false>, grid, nt, 0, s, xkeys, nx, low_mask(ncbits), ncbits,
+                       t, lpos, lcnt, tmp);
+}
+
 void run_match(const uint64_t* xkeys, const float* xvals, uint64_t nx, int ncbits,
-               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s, U2* host) {
-  MatchOp op{xkeys, xvals, nx, low_mask(ncbits), ncbits, t, o, api};
-  run_scan(op, nx, tmp, s, true, host);
+               const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s, U2* host,
+               uint64_t* look) {
+  uint64_t* lpos = api ? o.mpos : look;
+  uint64_t* lcnt = api ? o.mcnt : (look ? look + nx : nullptr);
+  if (nx <= kScanOneMax || !lpos) {
+    run_scan(MatchOp<false>{xkeys, xvals, nx, low_mask(ncbits), ncbits, t, o, api, nullptr, nullptr},
+             nx, tmp, s, true, host);
+    return;
+  }
+  launch_match_lookup(xkeys, nx, ncbits, t, lpos, lcnt, tmp, s);
+  run_scan_emit(MatchOp<true>{xkeys, xvals, nx, low_mask(ncbits), ncbits, t, o, api, lpos, lcnt}, nx,
+                tmp, s, host);
 }
 
 void run_match_count(const uint64_t* xkeys, uint64_t nx, int ncbits, const YTable& t, U2* tmp,
                      hipStream_t s) {
-  MatchOut o{};
-  MatchOp op{xkeys, nullptr, nx, low_mask(ncbits), ncbits, t, o, 0};
-  run_scan(op, nx, tmp, s, /*emit=*/false);
+  if (!nx) return;
+  launch_match_lookup(xkeys, nx, ncbits, t, nullptr, nullptr, tmp, s);
+  scan_tiles(tmp, scan_tmp_count(nx), tmp + scan_tmp_count(nx), s);
 }
 
 struct ExclScanOp {
@@ -980,26 +1051,6 @@ __global__ __launch_bounds__(kBlock) void k_fold_sums(const double* slots, doubl
 
 void launch_fold_sums(const double* slots, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kBlock), 0, s, slots, out);
-}
-
-// Any two equal adjacent keys in a sorted array (duplicate coordinates).
-__global__ __launch_bounds__(kBlock) void k_any_dup(const uint64_t* __restrict__ keys, uint64_t n,
-                                                    uint64_t* dup, uint64_t* hdup) {
-  uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x + 1;
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  bool same = false;
-  for (; i < n; i += stride) same |= keys[i] == keys[i - 1];
-  if (__ballot(same) && lane_id() == 0) {
-    *dup = 1;
-    *hdup = 1;
-  }
-}
-
-void launch_any_dup(const uint64_t* keys, uint64_t n, uint64_t* dup, uint64_t* hdup,
-                    hipStream_t s) {
-  if (n < 2) return;
-  uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock), 2048);
-  hipLaunchKernelGGL(k_any_dup, dim3(grid), dim3(kBlock), 0, s, keys, n, dup, hdup);
 }
 
 // Exclusive scan of per-row uint32 counts into uint64 offsets (+ total).

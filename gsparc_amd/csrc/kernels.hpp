@@ -7,7 +7,6 @@
 namespace sptc {
 
 constexpr int kMaxFusedPasses = 8;  // producers fuse histograms up to this many passes
-constexpr int kDirectBits = 22;     // direct-addressed Y segment table up to 2^22 keys
 
 // Packed key of a group of contracted coordinates, above the previous
 // group's rank: key = prev << prev_shift | OR_j (idx_j & (2^w_j-1)) << s_j.
@@ -21,14 +20,23 @@ struct TupleArgs {
   int prev_shift;
 };
 
+// Y's entries by the top bits of their contract value c: tab[c >> sh] =
+// {first, end} among the sorted keys.  sh == 0: one contract value per entry.
 struct YTable {
-  int direct;
-  const uint64_t* lo;      // direct: [2^ncbits]
-  const uint64_t* hi;
-  const uint64_t* ukey;    // search: [U] distinct contract values
-  const uint64_t* ustart;  // [U+1]
-  uint64_t U;
+  const U2* tab;
+  const uint64_t* ykeys;
+  uint64_t ny;
+  int sh, ynf;
 };
+// Entries of the table (a power of two) for ny keys of ncbits contract bits:
+// one per contract value while that is at most 4 per key (or 2^14 in all, which
+// one short fill clears), else up to one per key -- so that a table takes no more
+// than 64 bytes per key, and a small Y under a wide field no long fill.
+inline int ytable_bits(int ncbits, uint64_t ny, int exact_max = 22) {
+  const int fl = ny ? 63 - __builtin_clzll(ny) : 0;
+  if (ncbits <= 14 || (ncbits <= exact_max && ncbits <= fl + 2)) return ncbits;
+  return ncbits < fl ? ncbits : fl;
+}
 
 struct MatchOut {
   // engine form (compacted active X nonzeros and X rows)
@@ -118,23 +126,21 @@ void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t
 // *out (device or pinned host memory) = sum of the kSumSlots slots, added in a
 // fixed order.
 void launch_fold_sums(const double* slots, double* out, hipStream_t s);
-// Sets *dup (device) and *hdup (pinned host), cleared by the caller, when two
-// adjacent keys are equal.
-void launch_any_dup(const uint64_t* keys, uint64_t n, uint64_t* dup, uint64_t* hdup,
-                    hipStream_t s);
 void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp, hipStream_t s,
                         U2* host = nullptr);
 
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
                       uint64_t* hist, int passes, int rb, hipStream_t s);
-void launch_ytable_direct(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t K,
-                          uint64_t* lo, uint64_t* hi, hipStream_t s, uint64_t* dup = nullptr,
-                          uint64_t* hdup = nullptr);
-void run_yunique(const uint64_t* ykeys, uint64_t ny, int ynf, uint64_t* ukey,
-                 uint64_t* ustart, U2* tmp, hipStream_t s, U2* host = nullptr);
+// Fills and builds the table in tab[0 .. 2^bits - 1] (bits from ytable_bits).  With
+// hdup (pinned host memory, cleared by the caller) the entry after it holds the
+// duplicate flag: both are set when two Y keys are equal.
+YTable build_ytable(U2* tab, int bits, const uint64_t* ykeys, uint64_t ny, int ncbits, int ynf,
+                    hipStream_t s, uint64_t* hdup = nullptr);
+// look (may be NULL): scratch of 2 * nx words for what the lookups find; without
+// it they run twice.  The per-phase form (api) keeps them in mpos and mcnt.
 void run_match(const uint64_t* xkeys, const float* xvals, uint64_t nx, int ncbits,
                const YTable& t, const MatchOut& o, int api, U2* tmp, hipStream_t s,
-               U2* host = nullptr);
+               U2* host = nullptr, uint64_t* look = nullptr);
 // Reduce half of run_match: tmp[scan_tmp_count(nx)] = {ir, A << 32 | R}.
 void run_match_count(const uint64_t* xkeys, uint64_t nx, int ncbits, const YTable& t, U2* tmp,
                      hipStream_t s);

@@ -22,9 +22,8 @@ sptc_status api_fail(sptc_status s, const std::string& m);  // api.cpp
 
 namespace {
 
-// Table region: a direct table (two 8-byte entries per contract key, up to
-// 2^21 keys) or the distinct-key table (two 8-byte entries per Y nonzero,
-// fewer than 2^21 of them).  Tile-sum region: scan_tmp_count(n) + 1 16-byte
+// Table region: two 8-byte entries per contract key (up to 2^21 keys) or at
+// most per Y nonzero (fewer than 2^21 of them).  Tile-sum region: scan_tmp_count(n) + 1 16-byte
 // entries (n below 65535 * 2048).
 constexpr uint64_t kTableBytes = 32ull << 20;
 constexpr uint64_t kTmpBytes = 1ull << 20;
@@ -86,28 +85,10 @@ extern "C" sptc_status sptc_index_match_noalloc(const uint64_t* xkeys, uint64_t 
   if (!base) return api_fail(SPTC_ERR_HIP, err);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   try {
-    uint64_t* t0 = reinterpret_cast<uint64_t*>(base);
     U2* tmp = reinterpret_cast<U2*>(base + kTableBytes);
-    YTable tab;
-    std::memset(&tab, 0, sizeof(tab));
-    if (direct) {
-      const uint64_t K = 1ull << ncbits;
-      fill_u64(t0, 0, 2 * K, s);
-      launch_ytable_direct(ykeys, ny, y_nfbits, K, t0, t0 + K, s);
-      tab.direct = 1;
-      tab.lo = t0;
-      tab.hi = t0 + K;
-    } else {
-      run_yunique(ykeys, ny, y_nfbits, t0, t0 + ny + 1, tmp, s);
-      U2 t;
-      SPTC_HIP(hipMemcpyAsync(&t, tmp + scan_tmp_count(ny), sizeof(U2), hipMemcpyDeviceToHost,
-                              s));
-      SPTC_HIP(hipStreamSynchronize(s));
-      tab.direct = 0;
-      tab.ukey = t0;
-      tab.ustart = t0 + ny + 1;
-      tab.U = t.a;
-    }
+    const YTable tab =
+        build_ytable(reinterpret_cast<U2*>(base), ytable_bits(ncbits, ny, kNoAllocDirectBits),
+                     ykeys, ny, ncbits, y_nfbits, s);
     MatchOut mo;
     std::memset(&mo, 0, sizeof(mo));
     mo.mpos = mpos;

@@ -149,7 +149,7 @@ struct RowKindOp {
     const uint64_t n = a.row_prod[r + 1] - a.row_prod[r];
     if (!n) return mk2(0, 0);
     const uint64_t own = a.row_act[r + 1] - a.row_act[r];
-    if (own == 1 && !*a.ydup) return mk2(1, 0);
+    if (own == 1 && !a.ydup) return mk2(1, 0);
     if (n <= a.short_max) return mk2(n << 32 | 1, 1ull << 32);
     return mk2(1, 1);
   }

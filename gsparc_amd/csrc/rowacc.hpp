@@ -39,7 +39,7 @@ struct RowAccArgs {
   const uint32_t* ytab32;      // the same as 32 bits (NULL: wider)
   uint32_t K;                  // column ranks below K
   uint32_t short_max;          // rows of several owners up to this many products are short
-  const uint64_t* ydup;        // nonzero: Y holds duplicate coordinates
+  bool ydup;                   // Y holds duplicate coordinates
   double* vsum;                // [kSumSlots]
 };
 

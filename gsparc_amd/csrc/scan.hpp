@@ -159,10 +159,12 @@ __global__ __launch_bounds__(kBlock) void k_scan_emit(Op op, uint64_t n, const U
   }
 }
 
-// The whole scan by one workgroup of 1024 threads, tiles of 4 items a thread.
+// The whole scan by one workgroup of 1024 threads, 4 items each.  Up to one such
+// tile: with four of them (16384 items, 37 us) two launches over many workgroups
+// are faster (a chain of two contractions of 9000 nonzeros 823 against 783 us).
 constexpr int kOneNT = 1024, kOneItems = 4;
 constexpr uint64_t kOneTile = (uint64_t)kOneNT * kOneItems;
-constexpr uint64_t kScanOneMax = 4 * kOneTile;
+constexpr uint64_t kScanOneMax = kOneTile;
 
 template <class Op>
 __global__ __launch_bounds__(kOneNT) void k_scan_one(Op op, uint32_t n, bool emit, U2* total,
@@ -260,6 +262,20 @@ inline uint64_t narrow_tmp_count(uint64_t n) {
 // ceil(nt / kScanSumsPerBlock) + 1 entries (defined in kernels.hip).
 void scan_tiles_parts(U2* sums, uint64_t nt, U2* total, U2* parts, hipStream_t s);
 
+// The second half of run_scan, for n > 0 whose tile sums are in tmp.
+template <class Op>
+void run_scan_emit(const Op& op, uint64_t n, U2* tmp, hipStream_t s, U2* host = nullptr) {
+  const uint64_t nt = scan_tmp_count(n);
+  if (nt <= kScanSelfTiles) {
+    hipLaunchKernelGGL((k_scan_emit<Op, true>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
+                       (const U2*)tmp, (uint32_t)nt, tmp + nt, host);
+    return;
+  }
+  scan_tiles(tmp, nt, tmp + nt, s, host);
+  hipLaunchKernelGGL((k_scan_emit<Op, false>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
+                     (const U2*)tmp, (uint32_t)nt, (U2*)nullptr, (U2*)nullptr);
+}
+
 template <class Op>
 void run_scan(const Op& op, uint64_t n, U2* tmp, hipStream_t s, bool emit = true,
               U2* host = nullptr) {
@@ -275,15 +291,8 @@ void run_scan(const Op& op, uint64_t n, U2* tmp, hipStream_t s, bool emit = true
     return;
   }
   hipLaunchKernelGGL(k_scan_reduce<Op>, dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n, tmp);
-  if (emit && nt <= kScanSelfTiles) {
-    hipLaunchKernelGGL((k_scan_emit<Op, true>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
-                       (const U2*)tmp, (uint32_t)nt, total, host);
-    return;
-  }
-  scan_tiles(tmp, nt, total, s, host);
-  if (emit)
-    hipLaunchKernelGGL((k_scan_emit<Op, false>), dim3((uint32_t)nt), dim3(kBlock), 0, s, op, n,
-                       (const U2*)tmp, (uint32_t)nt, (U2*)nullptr, (U2*)nullptr);
+  if (emit) run_scan_emit(op, n, tmp, s, host);
+  else scan_tiles(tmp, nt, total, s, host);
 }
 
 }  // namespace sptc

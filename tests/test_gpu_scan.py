@@ -1,5 +1,5 @@
 """sptc_exclusive_scan_u64 at the sizes where the scan changes its launches: one
-workgroup (up to 16384 items, tiles of 4096), workgroups that add up the tile
+workgroup (up to 4096 items), workgroups that add up the tile
 sums before their own (up to 512 tiles of 2048), a separate tile-sum scan
 above.  Whole numbers: equal to numpy's."""
 import ctypes
