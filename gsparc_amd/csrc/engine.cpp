@@ -722,14 +722,23 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     // row-segmented product sort
     DevBuf<RowRange> rrange(1);
     RowSegPlan rseg;
-    // row accumulator (column spaces up to kRowAccMaxBits)
-    const bool rowacc = kyf > 0 && kyf <= kRowAccMaxBits && prefer_row_acc() && !partition_only;
+    // row accumulator (a tight budget keeps to the product sort, whose parts the
+    // chunks are sized for)
+    bool rowacc = kyf > 0 && kyf < 32 && prefer_row_acc() && !partition_only;
+    if (rowacc && chunk_cap) {
+      uint64_t max_act = 0;
+      for (size_t c = 1; c < bounds_a.size(); ++c)
+        max_act = std::max(max_act, bounds_a[c] - bounds_a[c - 1]);
+      const uint64_t held = DevicePool::get().live_bytes();
+      rowacc = held + rowacc_bytes(max_rows, max_act, chunk_cap, ranks) + out_per * ir <= budget_;
+    }
     RowAccPlan rplan;
     RowAccArgs ra;
     if (rowacc) {
       ra.act_prefix = act_prefix.get();
       ra.act_ypos = act_ypos.get();
       ra.act_xval = act_xval.get();
+      ra.act_row = act_row.get();
       ra.row_prod = row_prod.get();
       ra.row_act = row_act.get();
       ra.ny = ny;
@@ -760,10 +769,12 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       uint64_t out_n = 0;
       if (rowacc) {
         ra.r0 = r0c;
+        ra.a0 = bounds_a[c - 1];
         ra.rows = r1c - r0c;
         done = rowacc_count(ra, n, bounds_a[c] - bounds_a[c - 1], o_.count_only, &rplan,
                             host_total_, s_, &kt_);
         out_n = rplan.outs;
+        if (!done) rplan = RowAccPlan();
       }
       std::function<void(OutChunk&)> emit;
       if (done) {

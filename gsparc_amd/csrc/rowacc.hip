@@ -136,6 +136,9 @@ __global__ __launch_bounds__(kQuantNT) void k_ra_quant(const uint32_t* __restric
 // ---- rows by kind ------------------------------------------------------------
 // One scan over the chunk's rows: a = short products << 32 | live rows,
 // b = short rows << 32 | long rows (a chunk holds fewer than 2^32 products).
+// ACT: over its active X nonzeros instead, each row's first one standing for
+// the row (rows without products are never met).
+template <bool ACT>
 struct RowKindOp {
   RowAccArgs a;
   uint32_t least;
@@ -145,7 +148,11 @@ struct RowKindOp {
   uint64_t* live_src;
   uint32_t *s_live, *s_prod, *l_live;
   __device__ U2 value(uint64_t i) const {
-    const uint64_t r = a.r0 + i;
+    uint64_t r = a.r0 + i;
+    if (ACT) {
+      r = a.act_row[a.a0 + i];
+      if (i && a.act_row[a.a0 + i - 1] == r) return mk2(0, 0);
+    }
     const uint64_t n = a.row_prod[r + 1] - a.row_prod[r];
     if (!n) return mk2(0, 0);
     const uint64_t own = a.row_act[r + 1] - a.row_act[r];
@@ -156,8 +163,8 @@ struct RowKindOp {
   __device__ void emit(uint64_t i, U2 ex, U2 v) const {
     if (!v.a) return;
     const uint32_t k = (uint32_t)ex.a;
-    live_row[k] = (uint32_t)i;
-    const uint64_t r = a.r0 + i;
+    const uint64_t r = ACT ? a.act_row[a.a0 + i] : a.r0 + i;
+    live_row[k] = (uint32_t)(r - a.r0);
     if (v.b >> 32) {
       const uint32_t s = (uint32_t)(ex.b >> 32);
       s_live[s] = k;
@@ -831,8 +838,9 @@ struct GroupOwners {          // while the products are made
   uint16_t first[kGroupTile]; // first product in the group
   uint16_t row[kGroupTile];
 };
+template <typename KT>
 struct GroupSort {            // while they are sorted
-  TileSmem<10, kGroupIPT, kGroupNT, uint32_t> t;
+  TileSmem<10, kGroupIPT, kGroupNT, KT> t;
   float v[kGroupTile];
 };
 constexpr uint32_t kGroupRows = kGroupHalf + 1;  // rows hold two products at least
@@ -843,10 +851,15 @@ constexpr uint32_t kGroupRows = kGroupHalf + 1;  // rows hold two products at le
 // vary by stable LDS passes of 10 bits.  Runs of equal keys are summed by the
 // lane at their head; the outputs go to (tcol, tval) from the group's first
 // product on, compacted, with each row's count and place.
+// KT: 32 bits hold the key while the column has at most kGroupBits.  (8e6 x 3e6
+// nonzeros, 0.23e6 products in short rows over 2^22 columns, 7.4e6 rows: call 2970
+// us by the product sort, of which 590 in its row tables, 1753 here.)
+constexpr int kGroupBits = 21;  // and a row of the group 11
+template <typename KT>
 __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
   __shared__ union {
     GroupOwners own;
-    GroupSort sort;
+    GroupSort<KT> sort;
   } sm;
   __shared__ uint32_t s_live[kGroupRows], s_j0[kGroupRows];
   __shared__ uint16_t s_first[kGroupRows + 1], s_own[kGroupRows + 1];
@@ -899,7 +912,8 @@ __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
   }
   __syncthreads();
   const uint32_t wbase = wave * (kWave * IPT);
-  uint32_t k[IPT], rr[IPT], ow[IPT], pos[IPT];
+  KT k[IPT];
+  uint32_t rr[IPT], ow[IPT], pos[IPT];
   float v[IPT];
   double vs = 0.0;
   uint32_t cor = 0;
@@ -926,7 +940,7 @@ __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
     k[i] = ok ? k[i] : 0;
     v[i] = ok ? sm.own.x[ow[i]] * v[i] : 0.f;
     vs += (double)v[i];
-    cor |= k[i];
+    cor |= (uint32_t)k[i];
   }
   for (int off = kWave / 2; off > 0; off >>= 1) cor |= __shfl_xor(cor, off, kWave);
   for (int off = kWave / 2; off > 0; off >>= 1) vs += __shfl_xor(vs, off, kWave);
@@ -946,7 +960,7 @@ __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
   const int cb = cor ? 32 - __builtin_clz(cor) : 0;
   const int rbits = nr > 1 ? 32 - __builtin_clz(nr - 1) : 0;
 #pragma unroll
-  for (int i = 0; i < IPT; ++i) k[i] |= rr[i] << cb;
+  for (int i = 0; i < IPT; ++i) k[i] |= (KT)rr[i] << cb;
   const int passes = (cb + rbits + RB - 1) / RB;
   auto& sb = sm.sort;
   if (!passes) {  // one column of one row
@@ -970,7 +984,7 @@ __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
     for (int i = 0; i < IPT; ++i) {
       const uint32_t p = wbase + (uint32_t)i * kWave + lane;
       if (p < n) {
-        const uint32_t q = pos[i] + (uint32_t)sb.t.cnt[wave][(k[i] >> shift) & (R - 1)];
+        const uint32_t q = pos[i] + (uint32_t)sb.t.cnt[wave][(uint32_t)(k[i] >> shift) & (R - 1)];
         sb.t.buf[q] = k[i];
         sb.v[q] = v[i];
       }
@@ -1005,18 +1019,19 @@ __global__ __launch_bounds__(kGroupNT) void k_ra_group(GroupArgs g) {
     T += red[w];
   }
   const uint32_t cmask = (uint32_t)low_mask(cb);
+  constexpr int kBits = (int)sizeof(KT) * 8;
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
     if (!((hm >> i) & 1u)) continue;
     const uint32_t p = wbase + (uint32_t)i * kWave + lane;
     const uint32_t o = before + pos[i];
-    const uint32_t row = cb < 32 ? k[i] >> cb : 0;
-    if (p == 0 || (cb < 32 ? sb.t.buf[p - 1] >> cb : 0) != row) s_first[row] = (uint16_t)o;
+    const uint32_t row = cb < kBits ? (uint32_t)(k[i] >> cb) : 0;
+    if (p == 0 || (cb < kBits ? (uint32_t)(sb.t.buf[p - 1] >> cb) : 0) != row) s_first[row] = (uint16_t)o;
     if (g.tcol) {
       SumF64 s;
       s.add(v[i]);
       for (uint32_t q = p + 1; q < n && sb.t.buf[q] == k[i]; ++q) s.add(sb.v[q]);
-      g.tcol[base + o] = k[i] & cmask;
+      g.tcol[base + o] = (uint32_t)k[i] & cmask;
       g.tval[base + o] = s.value();
     }
   }
@@ -1194,9 +1209,20 @@ void room(DevBuf<T>& b, uint64_t n) {
 
 }  // namespace
 
+// Upper bound of what a chunk's plan holds.
+uint64_t rowacc_bytes(uint64_t rows, uint64_t owners, uint64_t nprod, uint64_t K) {
+  const uint64_t live = std::min(rows, owners);
+  const uint64_t least = K <= 1ull << kRowAccMaxBits ? min_slabs((uint32_t)K) : 1;
+  const uint64_t items = nprod / 256 * least + nprod / kItemProds;  // long rows: 256 products
+  return live * (28 + 4 + 4 + kNearBytes) + 8 * nprod + items * (kItemBytes + 4 + 8) +
+         4 * (owners * (least + 1) + nprod / kItemRun) + 4 * nprod + (2ull << 20);
+}
+
 bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool count_only,
                   RowAccPlan* p, U2* host, hipStream_t s, KTimer* kt) {
-  const uint64_t rows = a.rows;
+  // every live row has an active X nonzero: the fewer of both are scanned
+  const bool by_act = owners < a.rows;
+  const uint64_t rows = by_act ? owners : a.rows;
   if (nprod >= (1ull << 32)) throw std::length_error("row accumulator chunk");
   room(p->live_row, rows);
   room(p->live_cnt, rows);
@@ -1205,13 +1231,20 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   room(p->s_prod, rows);
   room(p->l_live, rows);
   room(p->tmp, scan_tmp_count(rows) + 1);
-  const uint32_t least = min_slabs(a.K);
-  RowKindOp kind{a, least, std::max(kHeavyItem, nprod >> 10), &host[1].a, p->live_row.get(), p->live_cnt.get(), p->live_src.get(), p->s_live.get(),
-                 p->s_prod.get(), p->l_live.get()};
+  // (column spaces too wide to cut into slabs take no long rows)
+  const bool slabs = a.K <= 1u << kRowAccMaxBits;
+  const uint32_t least = slabs ? min_slabs(a.K) : 1;
+  const uint64_t heavy = std::max(kHeavyItem, nprod >> 10);
   host[1].a = 0;
-  run_scan(kind, rows, p->tmp.get(), s, true, host);
+  auto kinds = [&](auto op) {
+    op = {a, least, heavy, &host[1].a, p->live_row.get(), p->live_cnt.get(), p->live_src.get(),
+          p->s_live.get(), p->s_prod.get(), p->l_live.get()};
+    run_scan(op, rows, p->tmp.get(), s, true, host);
+  };
+  if (by_act) kinds(RowKindOp<true>{});
+  else kinds(RowKindOp<false>{});
   SPTC_HIP(hipStreamSynchronize(s));
-  if (host[1].a) return false;
+  if (host[1].a || (!slabs && (host->b & 0xFFFFFFFFull))) return false;
   p->live = host->a & 0xFFFFFFFFull;
   p->short_prods = host->a >> 32;
   p->nshort = host->b >> 32;
@@ -1240,8 +1273,11 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
                 count_only ? nullptr : p->tcol.get(),
                 count_only ? nullptr : p->tval.get()};
     const int tok = kt->begin(s);
-    hipLaunchKernelGGL(k_ra_group, dim3((uint32_t)ceil_div(p->short_prods, kGroupHalf)),
-                       dim3(kGroupNT), 0, s, g);
+    const dim3 gg((uint32_t)ceil_div(p->short_prods, kGroupHalf)), gt(kGroupNT);
+    if (a.K <= 1u << kGroupBits)
+      hipLaunchKernelGGL(k_ra_group<uint32_t>, gg, gt, 0, s, g);
+    else
+      hipLaunchKernelGGL(k_ra_group<uint64_t>, gg, gt, 0, s, g);
     kt->end(tok, SPTC_K_SORT_LOCAL, (count_only ? 8.0 : 16.0) * (double)p->short_prods, s);
   }
   if (p->nlong) {

@@ -9,8 +9,9 @@ namespace sptc {
 // column's offset in it fits 16 bits.
 constexpr int kSlabBits = 16;
 constexpr uint32_t kSlabCols = 1u << kSlabBits;
-// Column spaces up to this many bits (16 slabs) take the row accumulator;
-// wider ones the product sort, whose cost does not grow with them.
+// Column spaces up to this many bits (16 slabs) are cut into slabs; over wider
+// ones the row accumulator takes chunks without long rows, and the product sort,
+// whose cost does not grow with the columns, the others.
 constexpr int kRowAccMaxBits = 20;
 
 // Products of a group of short rows (one workgroup's LDS sort) and the most
@@ -28,6 +29,8 @@ struct RowAccArgs {
   const float* act_xval;       // [A]
   const uint64_t* row_prod;    // [R + 1]
   const uint64_t* row_act;     // [R + 1]
+  const uint32_t* act_row;     // [A]
+  uint64_t a0;                 // the chunk's first active X nonzero
   uint64_t r0, rows;
   uint64_t ny;
   const uint32_t* ycol;        // [ny] column rank of each Y entry
@@ -79,9 +82,12 @@ struct RowAccPlan {
 // receives three U2 of pinned memory.  One wait for the row kinds, one for the
 // counts.  count_only: the groups' outputs are not kept and the value sum is
 // taken here.  nprod and owners: the chunk's products and active X nonzeros.
-// False, with nothing done, when a row is too heavy for one workgroup an item.
+// False, with nothing done, when a row is too heavy for one workgroup an item
+// or a long row meets a column space wider than kRowAccMaxBits.
 bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool count_only,
                   RowAccPlan* plan, U2* host, hipStream_t s, KTimer* kt);
+// Bytes a plan holds at most, for K column ranks.
+uint64_t rowacc_bytes(uint64_t rows, uint64_t owners, uint64_t nprod, uint64_t K);
 // Writes the outputs (plan->outs entries, in (row, column) order).
 void rowacc_emit(const RowAccArgs& a, RowAccPlan& plan, uint64_t nprod, uint32_t* out_row,
                  uint64_t* out_col, float* out_val, hipStream_t s, KTimer* kt);

@@ -64,7 +64,7 @@ def test_short_rows_and_group_edges(gpu, K):
                                (1 << 20) + 1])
 def test_long_rows_at_slab_edges(gpu, K):
     """Column spaces around one slab's 2^16 columns, up to the widest that is
-    cut into slabs (2^20) and one wider (the product sort); rows on both sides
+    cut into slabs (2^20) and one wider (its long rows take the product sort); rows on both sides
     of the even and the product-following cut (12288 products) and of
     multiples of an item's 7168."""
     rng = np.random.default_rng(K)
@@ -140,3 +140,18 @@ def test_signed_zero_infinity_and_nan(gpu):
     w = np.array([want[k] for k in keys]).astype(np.float32)
     np.testing.assert_array_equal(v, w)  # NaN where NaN
     assert not np.signbit(v[v == 0]).any()
+
+
+@pytest.mark.parametrize("K", [40, 1 << 20, (1 << 20) + 1, 1 << 21, (1 << 21) + 1, (1 << 22) + 5])
+def test_wide_columns_and_sparse_rows(gpu, K):
+    """Short and one-owner rows over column spaces that are not cut into slabs
+    (keys of 32 and of 64 bits in the groups), found among rows without
+    products (more rows than active X nonzeros, then fewer); and one row too
+    long for such a space, which takes the chunk to the product sort."""
+    rng = np.random.default_rng(K)
+    rows = [[min(n, K) for n in r] for r in SHORT * 2]
+    for empty in (3000, 0):
+        mixed = rows + [[0]] * empty
+        mixed = [mixed[i] for i in rng.permutation(len(mixed))]
+        check(*build(rng, K, mixed, signed=True))
+    check(*build(rng, K, rows + [[min(1536, K)] * 2, [0]], signed=True))
