@@ -129,7 +129,7 @@ template <typename IdxT, int RB>
 __global__ __launch_bounds__(kBlock) void k_linearize(LinArgs a, uint64_t n,
                                                       uint64_t* __restrict__ keys,
                                                       uint64_t* __restrict__ hist,
-                                                      int passes) {
+                                                      int passes, int lo) {
   constexpr int R = 1 << RB;
   __shared__ uint32_t sh[kMaxFusedPasses * R];
   for (int i = threadIdx.x; i < passes * R; i += kBlock) sh[i] = 0;
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void k_linearize(LinArgs a, uint64_t n,
         k |= shl64((uint64_t)static_cast<const IdxT*>(a.idx[m])[i] & low_mask(a.width[m]),
                    a.shift[m]);
     keys[i] = k;
-    if (passes) hist_add_wave<RB>(sh, k, true, passes);
+    if (passes) hist_add_wave<RB>(sh, shr64(k, lo), true, passes);
   }
   if (passes) {
     __syncthreads();
@@ -153,13 +153,13 @@ __global__ __launch_bounds__(kBlock) void k_linearize(LinArgs a, uint64_t n,
 }
 
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
-                      uint64_t* hist, int passes, int rb, hipStream_t s) {
+                      uint64_t* hist, int passes, int rb, hipStream_t s, int lo) {
   if (!n) return;
   uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock * 4), passes ? 1024 : 2048);
   if (passes > kMaxFusedPasses) passes = 0;  // caller falls back to histogram()
 #define SPTC_LIN(T, RBV)                                                                   \
   hipLaunchKernelGGL((k_linearize<T, RBV>), dim3(grid), dim3(kBlock), 0, s, a, n, keys, hist, \
-                     passes)
+                     passes, lo)
   if (idx_bytes == 4) {
     switch (rb) {
       case 9: SPTC_LIN(uint32_t, 9); break;

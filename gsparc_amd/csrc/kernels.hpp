@@ -130,7 +130,7 @@ void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp,
                         U2* host = nullptr);
 
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
-                      uint64_t* hist, int passes, int rb, hipStream_t s);
+                      uint64_t* hist, int passes, int rb, hipStream_t s, int lo = 0);
 // Fills and builds the table in tab[0 .. 2^bits - 1] (bits from ytable_bits).  With
 // hdup (pinned host memory, cleared by the caller) the entry after it holds the
 // duplicate flag: both are set when two Y keys are equal.

@@ -56,7 +56,7 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
 // Standalone histogram of all passes (used when no producer fused it).
 template <int RB>
 __global__ __launch_bounds__(kBlock) void k_histogram(const uint64_t* __restrict__ keys,
-                                                      uint64_t n, int passes,
+                                                      uint64_t n, int lo, int passes,
                                                       uint64_t* __restrict__ hist) {
   constexpr int R = 1 << RB;
   __shared__ uint32_t sh[kMaxPasses * R];
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_histogram(const uint64_t* __restrict
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (; i < n; i += stride) {
-    uint64_t k = keys[i];
+    const uint64_t k = keys[i] >> lo;
     for (int p = 0; p < passes; ++p)
       atomicAdd(&sh[p * R + ((k >> (p * RB)) & (R - 1))], 1u);
   }
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(NT) void k_onesweep(
 constexpr int kSmallNT = 512, kSmallIPT = 12, kSmallRB = 8;
 template <typename IdxT>
 __global__ __launch_bounds__(kSmallNT) void k_sort_small(LinArgs a, const float* __restrict__ val,
-                                                         uint32_t n,
+                                                         uint32_t n, int first_bit,
                                                          uint64_t* __restrict__ keys,
                                                          float* __restrict__ vals) {
   constexpr int RB = kSmallRB, IPT = kSmallIPT, NT = kSmallNT, R = 1 << RB;
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(kSmallNT) void k_sort_small(LinArgs a, const float*
     o |= s_or[w];
     an &= s_and[w];
   }
-  const uint64_t vary = o & ~an;
+  const uint64_t vary = o & ~an & ~low_mask(first_bit);
   const int lo = vary ? __builtin_ctzll(vary) : 0, hi = vary ? 64 - __builtin_clzll(vary) : 0;
   for (int shift = lo; shift < hi; shift += RB) {
     if (!((vary >> shift) & (R - 1))) continue;  // a digit that all keys share
@@ -366,6 +366,7 @@ struct PassArgs {
   uint64_t n;
   uint64_t tiles;
   int pass;
+  int lo;  // the sort's first bit
   hipStream_t s;
   KTimer* kt;
   int cls;
@@ -379,11 +380,11 @@ struct OnesweepPass {
     const int tok = a.kt ? a.kt->begin(a.s) : -1;
     if (a.tag)
       hipLaunchKernelGGL((k_onesweep<RB, IPT, NT, 1>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
-                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->hist() + a.pass * R,
+                         a.ka, a.va, a.kb, a.vb, a.n, a.lo + a.pass * RB, a.ws->hist() + a.pass * R,
                          a.ws->status(), a.ws->counters() + a.pass, a.ws->epoch, a.ws->err());
     else
       hipLaunchKernelGGL((k_onesweep<RB, IPT, NT, 0>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
-                         a.ka, a.va, a.kb, a.vb, a.n, a.pass * RB, a.ws->hist() + a.pass * R,
+                         a.ka, a.va, a.kb, a.vb, a.n, a.lo + a.pass * RB, a.ws->hist() + a.pass * R,
                          a.ws->status(), a.ws->counters() + a.pass, a.ws->epoch, a.ws->err());
     if (a.kt) a.kt->end(tok, a.cls, 24.0 * (double)a.n, a.s);
   }
@@ -394,7 +395,7 @@ struct RtsPass {
   template <int RB, int IPT, int NT>
   void run() {
     const uint64_t m = a.tiles << RB;
-    const int shift = a.pass * RB;
+    const int shift = a.lo + a.pass * RB;
     int tok = a.kt ? a.kt->begin(a.s) : -1;
     hipLaunchKernelGGL((k_rts_upsweep<RB, IPT, NT>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
                        a.ka, a.n, shift, a.ws->rts_cnt.get(), a.tiles);
@@ -483,44 +484,44 @@ void SortWorkspace::prepare(uint64_t n, hipStream_t s) {
 }
 
 bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
-                          uint64_t* keys, float* vals, hipStream_t s) {
+                          uint64_t* keys, float* vals, int lo, hipStream_t s) {
   if (n > (uint64_t)kSmallNT * kSmallIPT || sort_cfg().mode) return false;
   if (idx_bytes == 4)
-    hipLaunchKernelGGL(k_sort_small<uint32_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
+    hipLaunchKernelGGL(k_sort_small<uint32_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n, lo,
                        keys, vals);
   else
-    hipLaunchKernelGGL(k_sort_small<uint64_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
+    hipLaunchKernelGGL(k_sort_small<uint64_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n, lo,
                        keys, vals);
   return true;
 }
 
 void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
-               int passes, hipStream_t s) {
+               int passes, hipStream_t s, int lo) {
   if (!n || !passes) return;
   uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(n, kBlock * 8), 2048);
   switch (ws.rb) {
-    case 9: hipLaunchKernelGGL(k_histogram<9>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
+    case 9: hipLaunchKernelGGL(k_histogram<9>, dim3(grid), dim3(kBlock), 0, s, keys, n, lo, passes,
                                ws.hist()); break;
-    case 10: hipLaunchKernelGGL(k_histogram<10>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
+    case 10: hipLaunchKernelGGL(k_histogram<10>, dim3(grid), dim3(kBlock), 0, s, keys, n, lo, passes,
                                 ws.hist()); break;
-    case 11: hipLaunchKernelGGL(k_histogram<11>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
+    case 11: hipLaunchKernelGGL(k_histogram<11>, dim3(grid), dim3(kBlock), 0, s, keys, n, lo, passes,
                                 ws.hist()); break;
-    default: hipLaunchKernelGGL(k_histogram<8>, dim3(grid), dim3(kBlock), 0, s, keys, n, passes,
+    default: hipLaunchKernelGGL(k_histogram<8>, dim3(grid), dim3(kBlock), 0, s, keys, n, lo, passes,
                                 ws.hist()); break;
   }
 }
 
 // vals NULL: the keys alone are moved; vsrc: the values are read from there
 // instead of vals (which the second pass writes).
-// Sorts keys/vals (n <= ws.cap, n < 2^32) on bits [0, nbits).  With the
+// Sorts keys/vals (n <= ws.cap, n < 2^32) on bits [lo, nbits).  With the
 // onesweep algorithm ws.hist must hold the digit histograms of all passes.
 // Result ends in (keys, vals) when the pass count is even, else in
 // (ws.alt_keys, ws.alt_vals); the returned flag says which (true = alt).
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
                           uint64_t n, int nbits, hipStream_t s, KTimer* kt, int cls,
-                          const float* vsrc) {
+                          const float* vsrc, int lo) {
   const int rb = ws.rb;
-  const int passes = radix_passes(nbits, rb);
+  const int passes = radix_passes(nbits - lo, rb);
   if (!n || !passes) return false;
   if (n >= (1ull << 32)) throw std::length_error("radix sort of 2^32 or more keys");
   const bool onesweep = sort_onesweep(n);
@@ -528,7 +529,7 @@ bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
   const int tag = (cls == SPTC_K_SORT_PROD || cls == SPTC_K_SORT_PROD_WIDE) ? 1 : 0;
   const int kcls = (cls == SPTC_K_SORT_PROD && rb > 8) ? SPTC_K_SORT_PROD_WIDE : cls;
   PassArgs a{tag, &ws, keys, vals, ws.alt_keys.get(), vals ? ws.alt_vals.get() : nullptr, n, tiles,
-             0, s, kt, kcls};
+             0, lo, s, kt, kcls};
   if (vsrc) a.va = const_cast<float*>(vsrc);  // read by the first pass only
   for (int p = 0; p < passes; ++p) {
     a.pass = p;

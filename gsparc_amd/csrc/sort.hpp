@@ -55,21 +55,21 @@ bool radix_bits_supported(int rb);
 // CU the look-back's status words cost more than the launches they save.
 constexpr uint64_t kOnesweepMax = 1ull << 21;
 bool sort_onesweep(uint64_t n);
-// Linearizes and sorts up to one tile of nonzeros in one launch; false when
-// there are more.
+// Linearizes and sorts up to one tile of nonzeros in one launch, on bits [lo, 64);
+// false when there are more.
 bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
-                          uint64_t* keys, float* vals, hipStream_t s);
+                          uint64_t* keys, float* vals, int lo, hipStream_t s);
 // Digit width for a sort over nbits key bits (fewest passes, digits <= 10).
 int choose_radix_bits(int nbits);
 void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
-               int passes, hipStream_t s);
-// Sorts (keys, vals) on bits [0, nbits), ws.hist() holding the histograms of
+               int passes, hipStream_t s, int lo = 0);
+// Sorts (keys, vals), stably, on bits [lo, nbits), ws.hist() holding the histograms of
 // all passes for sizes that sort_onesweep.  Returns true when the sorted data ended in (ws.alt_keys,
 // ws.alt_vals) (odd pass count).
 // kt (optional) times every pass under kernel class `cls`.
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
                           uint64_t n, int nbits, hipStream_t s, KTimer* kt = nullptr,
-                          int cls = 0, const float* vsrc = nullptr);
+                          int cls = 0, const float* vsrc = nullptr, int lo = 0);
 
 // Device-side histogram accumulation for producers: call once per key with
 // an LDS array of passes*R uint32 cleared by the block, then flush.
