@@ -450,7 +450,7 @@ __global__ __launch_bounds__(kBlock) void k_bdense_numeric(BDenseArgs a) {
   const uint32_t g = find_seg(a.grp_rows, a.G, blockIdx.x);
   // instance-local row id
   dense_row_numeric<EB>(a.d, a.d.row_act[r], a.d.row_act[r + 1],
-                        a.ytab + in.yt_off, (uint32_t)(blockIdx.x - a.grp_rows[g]),
+                        a.ytab + in.yt_off, in.kyf < EB ? 1u << in.kyf : 1u << EB, (uint32_t)(blockIdx.x - a.grp_rows[g]),
                         a.d.out_off[blockIdx.x], s_acc, sm, &s_ja);
 }
 

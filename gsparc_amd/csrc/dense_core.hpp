@@ -1,15 +1,19 @@
 // Dense per-row accumulation core shared by the single-contraction and the
 // batched dense kernels.
 //
-// One workgroup owns one X row.  The row's products -- the concatenation, in
-// active-nonzero order j, of each nonzero's matched Y segment -- are taken in
-// rounds of kBlock * G products: every thread loads its G products of the
-// round at once (strided, so loads coalesce and G of them are in flight per
-// thread), finds their owners j by binary search over the round's act_prefix
-// entries staged in LDS, and adds each to its column's FP64 slot by an LDS
-// atomic.  FP64 sums do not depend on the order of the adds (SumF64 in
-// common.hpp says when exactly), so rows need no barrier between owners and
-// the outputs equal the ESC path's.
+// One workgroup owns one X row.  A row of kOwnerRun products per owner or more
+// is taken a wave per owner (dense_owner_runs).  The products of others -- the
+// concatenation, in active-nonzero order j, of each nonzero's matched Y segment
+// -- are taken in rounds of kBlock * G products: every thread loads its G
+// products of the round at once (strided, so loads coalesce and G of them are in
+// flight per thread) and finds their owners j by binary search over the round's
+// act_prefix entries staged in LDS.  Either way each is added to its column's
+// FP64 slot by an LDS atomic.  FP64 sums do not depend on the order of the adds
+// (SumF64 in common.hpp says when exactly), so rows need no barrier between
+// owners and the outputs equal the ESC path's.  Only the slots below the number of
+// columns are cleared and read back, a wave per 64 of them, and stored by adjacent
+// lanes.  (Two operands of 4096 nonzeros over some hundred rows: 35 us a thread
+// per run of slots and a search per product, 20 so.)
 #pragma once
 #include "kernels.hpp"
 
@@ -22,7 +26,7 @@ template <int EB>
 struct DenseSmem {
   static constexpr int E = 1 << EB;
   static constexpr int W = E / 32;
-  uint32_t bm[W];
+  alignas(8) uint32_t bm[W];
   uint64_t pref[kDenseRound + 1];
   uint32_t red[kBlock / kWave];
   uint64_t jl;  // owner of the round's last product
@@ -62,6 +66,45 @@ __device__ __forceinline__ uint32_t dense_owner(const uint64_t* pref, uint32_t m
   return lo - 1;
 }
 
+// The row's products, a wave per owner: this wave takes owners w, w + nw, ...
+// of [j0, j1), 256 products of a segment in flight, and calls f(rank, product) for
+// each (VAL false: no product).  No searches and no barriers, but lanes idle past
+// a segment's end.
+template <bool VAL, class F>
+__device__ __forceinline__ void dense_owner_runs(const DenseArgs& a, uint64_t j0, uint64_t j1,
+                                                 uint32_t w, uint32_t nw, F&& f) {
+  constexpr int G = 4;
+  const uint32_t lane = lane_id();
+  for (uint64_t jb = j0; jb < j1; jb += kWave) {  // 64 owners' places at once
+    const uint64_t j = jb + lane < j1 ? jb + lane : jb;
+    const uint64_t oy = a.act_ypos[j];
+    const uint32_t on = (uint32_t)(a.act_prefix[j + 1] - a.act_prefix[j]);
+    const float ox = VAL ? a.act_xval[j] : 0.f;
+    const uint32_t no = (uint32_t)(j1 - jb < kWave ? j1 - jb : kWave);
+    for (uint32_t k = w; k < no; k += nw) {
+      const uint64_t y0 = __shfl(oy, k, kWave);
+      const uint32_t len = __shfl(on, k, kWave);
+      const float x = __shfl(ox, k, kWave);
+      for (uint32_t b = 0; b < len; b += kWave * G) {
+        uint32_t rk[G];
+        float v[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const uint32_t p = b + (uint32_t)g * kWave + lane;
+          const uint64_t y = y0 + (p < len ? p : len - 1);
+          rk[g] = a.ycol[y];
+          v[g] = VAL ? a.yvals[y] : 0.f;
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          if (b + (uint32_t)g * kWave + lane < len) f(rk[g], x * v[g]);
+      }
+    }
+  }
+}
+// Products per owner from which a row is taken that way by a whole workgroup.
+constexpr uint64_t kOwnerRun = 32;
+
 // Symbolic pass: bitmap of the row's touched column ranks; returns the count
 // (valid in thread 0).
 template <int EB>
@@ -70,7 +113,14 @@ __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t
   for (int i = threadIdx.x; i < DenseSmem<EB>::W; i += kBlock) sm.bm[i] = 0;
   const uint64_t p0 = j0 < j1 ? a.act_prefix[j0] : 0;
   const uint64_t p1 = j0 < j1 ? a.act_prefix[j1] : 0;
-  for (uint64_t pb = p0; pb < p1; pb += kDenseRound) {
+  const bool runs = p1 - p0 >= kOwnerRun * (j1 - j0);
+  if (runs) {
+    __syncthreads();
+    dense_owner_runs<false>(a, j0, j1, threadIdx.x / kWave, kBlock / kWave, [&](uint32_t rk, float) {
+      atomicOr(&sm.bm[rk >> 5], 1u << (rk & 31));
+    });
+  }
+  for (uint64_t pb = runs ? p1 : p0; pb < p1; pb += kDenseRound) {
     uint64_t ja;
     const uint64_t pl = (pb + kDenseRound < p1 ? pb + kDenseRound : p1) - 1;
     const uint32_t m = dense_stage_owners(a.act_prefix, j0, j1, pb, pl, sm, s_ja, &ja);
@@ -98,20 +148,29 @@ __device__ __forceinline__ uint32_t dense_row_count(const DenseArgs& a, uint64_t
 }
 
 // Numeric pass, then the touched slots in rank order to out_* at obase (row
-// id `row`, column ytab[rank] or rank).  `acc` holds E doubles of LDS.
+// id `row`, column ytab[rank] or rank).  `acc` holds E doubles of LDS, of which
+// the first `cols` are used: ranks are below it.
 template <int EB>
 __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j0, uint64_t j1,
-                                                  const uint64_t* ytab, uint32_t row, uint64_t obase, double* acc,
+                                                  const uint64_t* ytab, uint32_t cols,
+                                                  uint32_t row, uint64_t obase, double* acc,
                                                   DenseSmem<EB>& sm, uint64_t* s_ja) {
-  constexpr int E = DenseSmem<EB>::E;
-  constexpr int S = E / kBlock;  // slots per thread in the compaction (1..32)
-  static_assert(E >= kBlock && E % kBlock == 0, "dense row width");
-  for (int i = threadIdx.x; i < E; i += kBlock) acc[i] = 0.0;
+  static_assert(DenseSmem<EB>::E >= 64 && DenseSmem<EB>::E <= 64 * kBlock, "dense row width");
+  for (uint32_t i = threadIdx.x; i < cols; i += kBlock) acc[i] = 0.0;
   for (int i = threadIdx.x; i < DenseSmem<EB>::W; i += kBlock) sm.bm[i] = 0;
   const uint64_t p0 = j0 < j1 ? a.act_prefix[j0] : 0;
   const uint64_t p1 = j0 < j1 ? a.act_prefix[j1] : 0;
   double vsum = 0.0;
-  for (uint64_t pb = p0; pb < p1; pb += kDenseRound) {
+  const bool runs = p1 - p0 >= kOwnerRun * (j1 - j0);
+  if (runs) {
+    __syncthreads();
+    dense_owner_runs<true>(a, j0, j1, threadIdx.x / kWave, kBlock / kWave, [&](uint32_t rk, float z) {
+      vsum += (double)z;
+      atomicAdd(&acc[rk], (double)z);
+      atomicOr(&sm.bm[rk >> 5], 1u << (rk & 31));
+    });
+  }
+  for (uint64_t pb = runs ? p1 : p0; pb < p1; pb += kDenseRound) {
     uint64_t ja;
     const uint64_t pl = (pb + kDenseRound < p1 ? pb + kDenseRound : p1) - 1;
     const uint32_t m = dense_stage_owners(a.act_prefix, j0, j1, pb, pl, sm, s_ja, &ja);
@@ -140,21 +199,24 @@ __device__ __forceinline__ void dense_row_numeric(const DenseArgs& a, uint64_t j
     // (the next round's staging starts with a barrier)
   }
   __syncthreads();
-  // Compaction in column order: thread t owns slots [t*S, t*S+S).
-  const uint32_t first = threadIdx.x * S;
-  const uint32_t word = sm.bm[first >> 5];
-  uint32_t bits;
-  if constexpr (S == 32) bits = word;
-  else bits = (word >> (first & 31)) & ((1u << S) - 1);
+  // Compaction in column order, a wave per word of 64 slots: the outputs before
+  // each word, then every lane stores its slot's (adjacent lanes, adjacent outputs).
+  const uint32_t words = (cols + 63) / 64;  // at most E / 64 <= kBlock
+  const uint64_t* const bm64 = reinterpret_cast<const uint64_t*>(sm.bm);
   uint32_t tot;
-  uint32_t o = block_excl_scan<uint32_t>((uint32_t)__popc(bits), sm.red, &tot);
-  for (int e = 0; e < S; ++e) {
-    if ((bits >> e) & 1u) {
-      const uint32_t rk = first + e;
-      a.out_row[obase + o] = row;
-      a.out_col[obase + o] = ytab ? ytab[rk] : rk;
-      a.out_val[obase + o] = (float)acc[rk];
-      ++o;
+  const uint32_t mine = threadIdx.x < words ? (uint32_t)__popcll(bm64[threadIdx.x]) : 0u;
+  const uint32_t ex = block_excl_scan<uint32_t>(mine, sm.red, &tot);
+  uint32_t* const wpre = reinterpret_cast<uint32_t*>(sm.pref);
+  if (threadIdx.x < words) wpre[threadIdx.x] = ex;
+  __syncthreads();
+  for (uint32_t w = threadIdx.x / kWave; w < words; w += kBlock / kWave) {
+    const uint64_t b = bm64[w];
+    if (b >> lane_id() & 1) {
+      const uint32_t rk = w * 64 + lane_id();
+      const uint64_t o = obase + wpre[w] + popc_below(b);
+      a.out_row[o] = row;
+      a.out_col[o] = ytab ? ytab[rk] : rk;
+      a.out_val[o] = (float)acc[rk];
     }
   }
   if (!a.vsum) return;  // batches sum their outputs instead

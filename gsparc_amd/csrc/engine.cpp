@@ -555,6 +555,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     da.ycol = ycol_or_make();
     da.yvals = Y.vals.get();
     da.ytab = ytab.size() ? ytab.get() : nullptr;
+    da.cols = (uint32_t)std::max<uint64_t>(ranks, 1);
     da.row_cnt = row_cnt.get();
     da.out_off = out_off.get();
     da.vsum = vsum.get();

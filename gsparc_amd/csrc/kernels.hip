@@ -1012,12 +1012,186 @@ __global__ __launch_bounds__(kBlock) void k_dense_numeric(DenseArgs a) {
   __shared__ DenseSmem<EB> sm;
   __shared__ uint64_t s_ja;
   const uint64_t r = a.r0 + blockIdx.x;
-  dense_row_numeric<EB>(a, a.row_act[r], a.row_act[r + 1], a.ytab,
-                                 (uint32_t)r, a.out_off[blockIdx.x], s_acc, sm, &s_ja);
+  dense_row_numeric<EB>(a, a.row_act[r], a.row_act[r + 1], a.ytab, a.cols, (uint32_t)r,
+                        a.out_off[blockIdx.x], s_acc, sm, &s_ja);
+}
+
+// Many rows: a wave per row.  A workgroup per row spends a row of some hundred
+// products on its barriers and tables, so a workgroup takes chunks of rows, its
+// waves one row each, without barriers: a row of one owner is that Y segment (Y
+// has no duplicate coordinates here), others go through the wave's own LDS
+// slots, touched ones marked by a byte (sorted columns would meet in the words
+// of a bitmap).  Rows of many products, or of owners with few, are left to the
+// whole workgroup at the chunk's end.  4.7e5 rows of 380 products over 901
+// columns, counted and summed: 748 + 1650 us by a workgroup each, 133 + 920 so (2.8 GB written).
+constexpr uint32_t kRowChunk = 32;
+constexpr uint64_t kWaveRowMax = 4096;  // products of a wave's row
+constexpr uint64_t kWaveRowRun = 8;     // least products per owner of one
+// Below this many rows a workgroup each is faster (9000 rows: 13 us against 24).
+constexpr uint64_t kDenseWaveRows = 16384;
+
+template <int EB, bool NUM>
+__global__ __launch_bounds__(kBlock) void k_dense_rows(DenseArgs a, uint64_t rows,
+                                                       uint32_t chunk) {
+  constexpr int E = 1 << EB, NW = kBlock / kWave, G = 4;
+  struct WaveRow {
+    double acc[NUM ? E : 1];
+    uint32_t flag[E / 4];  // a byte per column
+  };
+  __shared__ union {
+    WaveRow w[NW];
+    struct {
+      double acc[NUM ? E : 1];
+      DenseSmem<EB> sm;
+    } b;
+  } u;
+  __shared__ uint64_t s_ja;
+  __shared__ uint32_t s_heavy[kRowChunk], s_nheavy;
+  // the chunk's rows, loaded together: first owners and their first products
+  __shared__ uint64_t s_act[kRowChunk + 1], s_prod[kRowChunk + 1], s_y[kRowChunk];
+  __shared__ float s_x[kRowChunk];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  WaveRow& wr = u.w[wave];
+  uint8_t* const flag = reinterpret_cast<uint8_t*>(wr.flag);
+  auto clear = [&] {
+    if (NUM)
+      for (int i = lane; i < E; i += kWave) wr.acc[i] = 0.0;
+    for (int i = lane; i < E / 4; i += kWave) wr.flag[i] = 0;
+  };
+  clear();
+  double vsum = 0.0;
+  const uint64_t nchunks = ceil_div(rows, (uint64_t)chunk);
+  for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+    const uint64_t l0 = c * chunk;  // chunk-local to the launch
+    const uint32_t nr = (uint32_t)(rows - l0 < chunk ? rows - l0 : chunk);
+    __syncthreads();
+    if (tid <= nr) {
+      const uint64_t j = a.row_act[a.r0 + l0 + tid];
+      s_act[tid] = j;
+      s_prod[tid] = a.act_prefix[j];
+    }
+    if (tid == 0) s_nheavy = 0;
+    __syncthreads();
+    if (tid < nr && s_act[tid] < s_act[tid + 1]) {
+      s_y[tid] = a.act_ypos[s_act[tid]];
+      s_x[tid] = a.act_xval[s_act[tid]];
+    }
+    __syncthreads();
+    for (uint32_t i = wave; i < nr; i += NW) {
+      const uint64_t j0 = s_act[i], own = s_act[i + 1] - j0, n = s_prod[i + 1] - s_prod[i];
+      if (own <= 1) {
+        if (!NUM) {
+          if (lane == 0) a.row_cnt[l0 + i] = (uint32_t)n;
+          continue;
+        }
+        const uint64_t y0 = s_y[i], ob = NUM && n ? a.out_off[l0 + i] : 0;
+        const float x = s_x[i];
+        for (uint64_t b = 0; b < n; b += kWave * G) {
+          uint32_t rk[G];
+          float v[G];
+          uint64_t col[G];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const uint64_t p = b + (uint64_t)g * kWave + lane, y = y0 + (p < n ? p : n - 1);
+            rk[g] = a.ycol[y];
+            v[g] = a.yvals[y];
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g) col[g] = a.ytab ? a.ytab[rk[g]] : rk[g];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const uint64_t p = b + (uint64_t)g * kWave + lane;
+            if (p >= n) continue;
+            const float z = x * v[g];
+            vsum += (double)z;
+            a.out_row[ob + p] = (uint32_t)(a.r0 + l0 + i);
+            a.out_col[ob + p] = col[g];
+            a.out_val[ob + p] = z + 0.f;  // a sum of one product: no negative zero
+          }
+        }
+        continue;
+      }
+      if (n > kWaveRowMax || n < kWaveRowRun * own) {
+        if (lane == 0) s_heavy[atomicAdd(&s_nheavy, 1u)] = i;
+        continue;
+      }
+      dense_owner_runs<NUM>(a, j0, j0 + own, 0, 1, [&](uint32_t rk, float z) {
+        flag[rk] = 1;
+        if (NUM) {
+          vsum += (double)z;
+          atomicAdd(&wr.acc[rk], (double)z);
+        }
+      });
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (!NUM) {
+        uint32_t cnt = 0;
+        for (uint32_t q = lane; q < (a.cols + 3) / 4; q += kWave) {
+          cnt += (uint32_t)__popc(wr.flag[q]);
+          wr.flag[q] = 0;
+        }
+        for (int off = kWave / 2; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, kWave);
+        if (lane == 0) a.row_cnt[l0 + i] = cnt;
+      } else {
+        uint64_t o = a.out_off[l0 + i];
+        for (uint32_t q = lane; q < (a.cols + 63) / 64 * 64; q += kWave) {  // (within E)
+          const bool on = flag[q] != 0;
+          const uint64_t b = __ballot(on);
+          if (on) {
+            const uint64_t w = o + popc_below(b);
+            a.out_row[w] = (uint32_t)(a.r0 + l0 + i);
+            a.out_col[w] = a.ytab ? a.ytab[q] : q;
+            a.out_val[w] = (float)wr.acc[q];
+            wr.acc[q] = 0.0;
+            flag[q] = 0;
+          }
+          o += (uint64_t)__popcll(b);
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    const uint32_t nh = s_nheavy;
+    for (uint32_t h = 0; h < nh; ++h) {
+      const uint32_t i = s_heavy[h];
+      if (!NUM) {
+        const uint32_t t = dense_row_count<EB>(a, s_act[i], s_act[i + 1], u.b.sm, &s_ja);
+        if (tid == 0) a.row_cnt[l0 + i] = t;
+      } else {
+        dense_row_numeric<EB>(a, s_act[i], s_act[i + 1], a.ytab, a.cols,
+                              (uint32_t)(a.r0 + l0 + i), a.out_off[l0 + i], u.b.acc, u.b.sm,
+                              &s_ja);
+      }
+      __syncthreads();
+    }
+    if (nh) clear();
+  }
+  if (!NUM) return;
+  for (int off = kWave / 2; off > 0; off >>= 1) vsum += __shfl_xor(vsum, off, kWave);
+  if (lane == 0 && vsum != 0.0) slot_add(a.vsum, vsum);
+}
+
+// Rows of a chunk when waves take them, 0 when each row is given a workgroup:
+// slots for four rows fit a workgroup up to 2^10 columns, and fewer rows than
+// kDenseWaveRows leave the chip's waves without one each.  Chunks shrink with the
+// rows, down to one row a wave, so that there are 2048 workgroups.
+inline uint32_t dense_row_chunk(int eb, uint64_t rows) {
+  if (eb > 10 || rows < kDenseWaveRows) return 0;
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(rows / 2048, kBlock / kWave), kRowChunk);
+}
+
+template <bool NUM>
+void launch_dense_rows(const DenseArgs& a, int eb, uint64_t rows, uint32_t chunk, hipStream_t s) {
+  const dim3 g((uint32_t)std::min<uint64_t>(ceil_div(rows, (uint64_t)chunk), 2048)), b(kBlock);
+  if (eb == 8) hipLaunchKernelGGL((k_dense_rows<8, NUM>), g, b, 0, s, a, rows, chunk);
+  else hipLaunchKernelGGL((k_dense_rows<10, NUM>), g, b, 0, s, a, rows, chunk);
 }
 
 void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s) {
   if (!rows) return;
+  if (const uint32_t c = dense_row_chunk(eb, rows))
+    return launch_dense_rows<false>(a, eb, rows, c, s);
   switch (eb) {
     case 8: hipLaunchKernelGGL(k_dense_count<8>, dim3((uint32_t)rows), dim3(kBlock), 0, s, a); break;
     case 10: hipLaunchKernelGGL(k_dense_count<10>, dim3((uint32_t)rows), dim3(kBlock), 0, s, a); break;
@@ -1027,6 +1201,8 @@ void launch_dense_count(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s
 
 void launch_dense_numeric(const DenseArgs& a, int eb, uint64_t rows, hipStream_t s) {
   if (!rows) return;
+  if (const uint32_t c = dense_row_chunk(eb, rows))
+    return launch_dense_rows<true>(a, eb, rows, c, s);
   const dim3 g((uint32_t)rows), b(kBlock);
   switch (eb) {
     case 8: hipLaunchKernelGGL(k_dense_numeric<8>, g, b, 0, s, a); break;

@@ -93,6 +93,7 @@ struct DenseArgs {
   const uint32_t* ycol;        // [ny] column rank of each Y entry
   const float* yvals;
   const uint64_t* ytab;        // rank -> Y free key (NULL: field is the key)
+  uint32_t cols;               // ranks below it
   uint32_t* row_cnt;           // [rows] symbolic counts
   const uint64_t* out_off;     // [rows] output offsets
   uint32_t* out_row;
