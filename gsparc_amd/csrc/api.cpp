@@ -919,7 +919,10 @@ sptc_status sptc_device_info(int32_t* num_cus, uint64_t* free_bytes, uint64_t* t
   return SPTC_OK;
 }
 
-void sptc_trim_cache(void) { DevicePool::get().trim(); }
+void sptc_trim_cache(void) {
+  DevicePool::get().trim();
+  trim_engine_hosts();
+}
 
 // ---- batched contractions -------------------------------------------------
 

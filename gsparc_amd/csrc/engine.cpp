@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -160,10 +161,74 @@ uint64_t count_products(const Operand& X, const Operand& Y, hipStream_t s) {
   return host.a;
 }
 
-Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o) {
-  for (auto& e : ev_) SPTC_HIP(hipEventCreate(&e));
-  SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_total_), sizeof(U2) * 4, 0));
-  SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_u64_), sizeof(uint64_t) * 8, 0));
+// The pinned words and events of engines that are done, for the next ones: a
+// call made and freed its own (two operands of 4096 nonzeros 251 us, 201 so; a
+// chain of two calls 800 and 673).  At most kHostKept are kept, per process and
+// by device; sptc_trim_cache frees them.
+namespace {
+constexpr size_t kHostKept = 16;
+struct HostCache {
+  std::mutex mu;
+  std::vector<EngineHost> kept;
+};
+HostCache& host_cache() {
+  static HostCache* c = [] {  // (outlives every engine)
+    auto* h = new HostCache;
+    h->kept.reserve(kHostKept);  // engines end without allocating
+    return h;
+  }();
+  return *c;
+}
+void destroy_host(EngineHost& h) {
+  for (auto e : h.ev)
+    if (e) (void)hipEventDestroy(e);
+  if (h.total) (void)hipHostFree(h.total);
+  if (h.words) (void)hipHostFree(h.words);
+  h = EngineHost();
+}
+EngineHost take_host() {
+  int dev = 0;
+  SPTC_HIP(hipGetDevice(&dev));
+  {
+    HostCache& c = host_cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    for (size_t i = 0; i < c.kept.size(); ++i)
+      if (c.kept[i].dev == dev) {
+        const EngineHost h = c.kept[i];
+        c.kept[i] = c.kept.back();
+        c.kept.pop_back();
+        return h;
+      }
+  }
+  EngineHost h;
+  h.dev = dev;
+  try {
+    for (auto& e : h.ev) SPTC_HIP(hipEventCreate(&e));
+    SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&h.total), sizeof(U2) * 4, 0));
+    SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&h.words), sizeof(uint64_t) * 8, 0));
+  } catch (...) {
+    destroy_host(h);
+    throw;
+  }
+  return h;
+}
+}  // namespace
+
+void trim_engine_hosts() {
+  std::vector<EngineHost> old;
+  {
+    HostCache& c = host_cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    old = c.kept;
+    c.kept.clear();
+  }
+  for (EngineHost& h : old) destroy_host(h);
+}
+
+Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(take_host()) {
+  for (int i = 0; i < 8; ++i) ev_[i] = host_.ev[i];
+  host_total_ = host_.total;
+  host_u64_ = host_.words;
   ws_.err_host = reinterpret_cast<uint32_t*>(host_u64_ + 7);
   *ws_.err_host = 0;
   // The budget caps what this call holds at once, on top of what was
@@ -182,9 +247,17 @@ Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o) {
 }
 
 Engine::~Engine() {
-  for (auto& e : ev_) (void)hipEventDestroy(e);
-  (void)hipHostFree(host_total_);
-  (void)hipHostFree(host_u64_);
+  // work that a failed call left behind may still write to the words; if it
+  // cannot be waited for they are not handed on
+  if (hipStreamSynchronize(s_) == hipSuccess) {
+    HostCache& c = host_cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    if (c.kept.size() < kHostKept) {
+      c.kept.push_back(host_);
+      return;
+    }
+  }
+  destroy_host(host_);
 }
 
 void Engine::record(int i) {

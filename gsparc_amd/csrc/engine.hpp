@@ -127,6 +127,15 @@ bool prefer_bucket_tail();
 // (SPTC_PROD_SORT, SPTC_BIG_TAIL, SPTC_SEG_RB, SPTC_SEG_IPT, SPTC_SEG_WIDE).
 bool prefer_row_acc();
 
+// Pinned words and events of an engine, kept between engines.
+struct EngineHost {
+  hipEvent_t ev[8] = {};
+  U2* total = nullptr;        // [4]
+  uint64_t* words = nullptr;  // [8]
+  int dev = 0;
+};
+void trim_engine_hosts();  // frees what is kept
+
 class Engine {
  public:
   Engine(hipStream_t s, const sptc_opts& o);
@@ -181,6 +190,7 @@ class Engine {
   int rb_ = 8;
   SortWorkspace ws_;
   KTimer kt_;
+  EngineHost host_;
   hipEvent_t ev_[8];
   bool ev_used_[8] = {false};
   U2* host_total_ = nullptr;

@@ -492,7 +492,7 @@ const char* sptc_status_string(sptc_status s);
 /* Detail of the last failure on the calling thread (empty when none). */
 const char* sptc_last_error(void);
 
-/* Returns cached device blocks to the HIP runtime. */
+/* Returns cached device blocks, pinned words and events to the HIP runtime. */
 void sptc_trim_cache(void);
 
 #ifdef __cplusplus
