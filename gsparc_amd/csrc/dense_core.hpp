@@ -12,7 +12,7 @@
 // (SumF64 in common.hpp says when exactly), so rows need no barrier between
 // owners and the outputs equal the ESC path's.  Only the slots below the number of
 // columns are cleared and read back, a wave per 64 of them, and stored by adjacent
-// lanes.  (Two operands of 4096 nonzeros over some hundred rows: 35 us a thread
+// lanes.  (Two operands of 3001 nonzeros over some hundred rows: 35 us a thread
 // per run of slots and a search per product, 20 so.)
 #pragma once
 #include "kernels.hpp"

@@ -162,7 +162,7 @@ uint64_t count_products(const Operand& X, const Operand& Y, hipStream_t s) {
 }
 
 // The pinned words and events of engines that are done, for the next ones: a
-// call made and freed its own (two operands of 4096 nonzeros 251 us, 201 so; a
+// call made and freed its own (two operands of 3001 nonzeros 251 us, 201 so; a
 // chain of two calls 800 and 673).  At most kHostKept are kept, per process and
 // by device; sptc_trim_cache frees them.
 namespace {
