@@ -524,19 +524,21 @@ __global__ void k_check_digest(const uint64_t* got, const uint64_t* want, uint32
   if (threadIdx.x == 0 && blockIdx.x == 0 && *got != *want) *bad = 1;
 }
 
-__global__ __launch_bounds__(kBlock) void k_sum_f64(const float* v, uint64_t n, double* out) {
+// Sums of slices of outputs, bps workgroups each, added to out[slice's inst].
+__global__ __launch_bounds__(kBlock) void k_sum_f64(const SumSlice* sl, uint32_t bps, double* out) {
   __shared__ double s_red[kBlock / kWave];
-  uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+  const SumSlice x = sl[blockIdx.x / bps];
+  uint64_t i = (uint64_t)(blockIdx.x % bps) * kBlock + threadIdx.x;
+  const uint64_t stride = (uint64_t)bps * kBlock;
   double t = 0.0;
-  for (; i < n; i += stride) t += (double)v[i];
+  for (; i < x.n; i += stride) t += (double)x.v[i];
   for (int off = kWave / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, kWave);
   if (lane_id() == 0) s_red[threadIdx.x / kWave] = t;
   __syncthreads();
   if (threadIdx.x == 0) {
     double u = 0.0;
     for (int w = 0; w < kBlock / kWave; ++w) u += s_red[w];
-    if (u != 0.0) atomicAdd(out, u);
+    if (u != 0.0) atomicAdd(&out[x.inst], u);
   }
 }
 
@@ -673,9 +675,11 @@ void launch_check_digest(const uint64_t* got, const uint64_t* want, uint32_t* ba
   hipLaunchKernelGGL(k_check_digest, dim3(1), dim3(64), 0, s, got, want, bad);
 }
 
-void launch_sum_f64(const float* vals, uint64_t n, double* out, hipStream_t s) {
+void launch_sum_f64(const SumSlice* slices, uint32_t n, uint64_t longest, double* out,
+                    hipStream_t s) {
   if (!n) return;
-  hipLaunchKernelGGL(k_sum_f64, dim3(grid_for(n, 1024)), dim3(kBlock), 0, s, vals, n, out);
+  const uint32_t bps = grid_for(ceil_div(longest, 16), 1024);
+  hipLaunchKernelGGL(k_sum_f64, dim3(n * bps), dim3(kBlock), 0, s, slices, bps, out);
 }
 
 }  // namespace sptc

@@ -176,6 +176,13 @@ void launch_digest(const uint64_t* keys, uint64_t n, uint64_t* out, hipStream_t 
 void launch_check_digest(const uint64_t* got, const uint64_t* want, uint32_t* bad,
                          hipStream_t s);
 // *out += sum of vals[0, n) in FP64.
-void launch_sum_f64(const float* vals, uint64_t n, double* out, hipStream_t s);
+struct SumSlice {
+  const float* v;
+  uint64_t n;
+  uint64_t inst;
+};
+// out[inst] += the FP64 sums of n slices, the longest of `longest` values.
+void launch_sum_f64(const SumSlice* slices, uint32_t n, uint64_t longest, double* out,
+                    hipStream_t s);
 
 }  // namespace sptc

@@ -717,7 +717,31 @@ sptc_status BatchEngine::sync(hipStream_t s) {
   return SPTC_OK;
 }
 
-sptc_status BatchEngine::instance_result(int i, sptc_result_s* r, hipStream_t s) {
+std::vector<double> BatchEngine::value_sums(int i0, int i1, hipStream_t s) {
+  std::vector<double> sums(i1 - i0, 0.0);
+  std::vector<SumSlice> sl;
+  uint64_t longest = 0;
+  for (int i = i0; i < i1; ++i)
+    for (const InstSlice& x : slices_[i]) {
+      sl.push_back({outs_[x.out].val.get() + x.b, x.e - x.b, (uint64_t)(i - i0)});
+      longest = std::max(longest, x.e - x.b);
+    }
+  if (sl.empty()) {
+    SPTC_HIP(hipStreamSynchronize(s));
+    return sums;
+  }
+  DevBuf<double> dev(sums.size());
+  DevBuf<SumSlice> tab(sl.size());
+  fill_u64(reinterpret_cast<uint64_t*>(dev.get()), 0, sums.size(), s);
+  SPTC_HIP(hipMemcpyAsync(tab.get(), sl.data(), sl.size() * sizeof(SumSlice),
+                          hipMemcpyHostToDevice, s));
+  launch_sum_f64(tab.get(), (uint32_t)sl.size(), longest, dev.get(), s);
+  readback(sums.data(), dev.get(), sums.size() * sizeof(double), s);
+  return sums;
+}
+
+sptc_status BatchEngine::instance_result(int i, sptc_result_s* r, hipStream_t s,
+                                         const double* value_sum) {
   const Layout& xl = xl_[i];
   const Layout& yl = yl_[i];
   sptc_result_info& in = r->info;
@@ -734,8 +758,6 @@ sptc_status BatchEngine::instance_result(int i, sptc_result_s* r, hipStream_t s)
   r->yl = yl;
   r->vrow_key = row_key_.get() + iR_[i];
   in.row_key = r->vrow_key;
-  DevBuf<double> sum(1);
-  fill_u64(reinterpret_cast<uint64_t*>(sum.get()), 0, 1, s);
   for (const InstSlice& sl : slices_[i]) {
     const BOut& ob = outs_[sl.out];
     OutChunk c;
@@ -745,13 +767,11 @@ sptc_status BatchEngine::instance_result(int i, sptc_result_s* r, hipStream_t s)
     c.vrow = ob.row.get() + sl.b;
     c.vcol = ob.col.get() + sl.b;
     c.vval = ob.val.get() + sl.b;
-    launch_sum_f64(c.vval, c.nnz, sum.get(), s);
     in.nnz += c.nnz;
     r->chunks.push_back(std::move(c));
   }
   in.nchunks = (int32_t)r->chunks.size();
-  SPTC_HIP(hipMemcpyAsync(&in.value_sum, sum.get(), 8, hipMemcpyDeviceToHost, s));
-  SPTC_HIP(hipStreamSynchronize(s));
+  in.value_sum = value_sum ? *value_sum : value_sums(i, i + 1, s)[0];
   if (r->chunks.size() == 1) {
     in.row = r->chunks[0].vrow;
     in.col = r->chunks[0].vcol;

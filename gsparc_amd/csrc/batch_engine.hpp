@@ -78,7 +78,12 @@ class BatchEngine {
   sptc_status launch_graph(hipStream_t s);
   // Waits for stream s and reports a stale plan.
   sptc_status sync(hipStream_t s);
-  sptc_status instance_result(int i, sptc_result_s* out, hipStream_t s = nullptr);
+  // Value sums of instances [i0, i1) by one launch and one wait: twelve requests
+  // took a buffer, two launches and a wait each.
+  std::vector<double> value_sums(int i0, int i1, hipStream_t s);
+  // value_sum: the instance's, if the caller has it.
+  sptc_status instance_result(int i, sptc_result_s* out, hipStream_t s = nullptr,
+                              const double* value_sum = nullptr);
   sptc_batch_info info;
   std::string msg;
   KTimer& ktimer() { return kt_; }

@@ -405,6 +405,8 @@ void Server::run_batch(int w, std::vector<std::shared_ptr<Request>>& rs) {
   std::memset(&o, 0, sizeof(o));
   sptc_status st = holder->eng->plan(B, X.data(), Y.data(), nc.data(), cx.data(), cy.data(), o,
                                      s, pre.data());
+  std::vector<double> sums;
+  if (st == SPTC_OK) sums = holder->eng->value_sums(0, B, s);
   for (int i = 0; i < B; ++i) {
     rs[i]->st = st;
     if (st != SPTC_OK) {
@@ -412,7 +414,7 @@ void Server::run_batch(int w, std::vector<std::shared_ptr<Request>>& rs) {
       continue;
     }
     auto res = std::make_shared<sptc_result_s>();
-    holder->eng->instance_result(i, res.get(), s);
+    holder->eng->instance_result(i, res.get(), s, &sums[i]);
     res->keep = holder;
     rs[i]->result = res;
   }
