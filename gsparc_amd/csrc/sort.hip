@@ -396,6 +396,9 @@ struct RtsPass {
   void run() {
     const uint64_t m = a.tiles << RB;
     const int shift = a.lo + a.pass * RB;
+    if (a.ws->rts_cnt.size() < m || a.ws->rts_off.size() < m ||
+        a.ws->rts_tmp.size() < scan_tmp_count(m) + 1)
+      throw std::logic_error("radix sort workspace not reserved");
     int tok = a.kt ? a.kt->begin(a.s) : -1;
     hipLaunchKernelGGL((k_rts_upsweep<RB, IPT, NT>), dim3((uint32_t)a.tiles), dim3(NT), 0, a.s,
                        a.ka, a.n, shift, a.ws->rts_cnt.get(), a.tiles);
@@ -469,10 +472,11 @@ void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s, bool vals) {
   if (sort_onesweep(n)) {
     if (sweep.size() < kMaxPasses * R + kSweepHead + tiles * R)
       sweep.reset(kMaxPasses * R + kSweepHead + tiles * R);
-  } else if (rts_cnt.size() < tiles * R) {
-    rts_cnt.reset(tiles * R);
-    rts_off.reset(tiles * R);
-    rts_tmp.reset(scan_tmp_count(tiles * R) + 1);
+  } else {  // (each by its own size: segmented sorts grow the matrices alone)
+    const uint64_t m = tiles * R, nt = scan_tmp_count(m) + 1;
+    if (rts_cnt.size() < m) rts_cnt.reset(m);
+    if (rts_off.size() < m) rts_off.reset(m);
+    if (rts_tmp.size() < nt) rts_tmp.reset(nt);
   }
 }
 

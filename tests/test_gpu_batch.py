@@ -8,7 +8,8 @@ import pytest
 from gsparc_amd import sptc
 from gsparc_amd.coo import COOTensor
 from gsparc_amd.workloads import batch_specs
-from helpers import REL_TOL, assert_same_coo, dense_friendly, load_fixtures, random_coo
+from helpers import (REL_TOL, assert_same_coo, compare_with_oracle, dense_friendly,
+                     load_fixtures, random_coo)
 
 pytestmark = pytest.mark.gpu
 FIXTURES = load_fixtures()
@@ -211,3 +212,19 @@ def test_batch_errors(gpu):
     b = sptc.Batch([(X, X, [2], [2])])
     with pytest.raises(sptc.SpTCError):
         b.result(1)
+
+
+def test_batch_large_chunk_that_is_not_row_segmented(gpu):
+    """Tensor times vector (no column bits): the chunk's 2.4e6 products are
+    sorted on their row bits by the large sort, in the workspace that the
+    operands' segmented sorts used before."""
+    rng = np.random.default_rng(23)
+    X = random_coo(rng, (300, 200, 50), 1_200_000, positive=False)
+    v = random_coo(rng, (50,), 50)
+    b = sptc.Batch([(X, v, [2], [0]), (X, v, [2], [0])], dense_accumulator=-1)
+    assert b.info["esc_chunks"] == 1
+    for use_graph in (False, True):
+        b.run(use_graph=use_graph)
+        b.sync()
+        for i in range(2):
+            compare_with_oracle(X, v, [2], [0], b.result(i))
