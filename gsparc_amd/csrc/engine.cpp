@@ -182,7 +182,6 @@ HostCache& host_cache() {
 void destroy_host(EngineHost& h) {
   for (auto e : h.ev)
     if (e) (void)hipEventDestroy(e);
-  if (h.total) (void)hipHostFree(h.total);
   if (h.words) (void)hipHostFree(h.words);
   h = EngineHost();
 }
@@ -204,8 +203,7 @@ EngineHost take_host() {
   h.dev = dev;
   try {
     for (auto& e : h.ev) SPTC_HIP(hipEventCreate(&e));
-    SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&h.total), sizeof(U2) * 4, 0));
-    SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&h.words), sizeof(uint64_t) * 8, 0));
+    SPTC_HIP(hipHostMalloc(reinterpret_cast<void**>(&h.words), sizeof(EngineWords), 0));
   } catch (...) {
     destroy_host(h);
     throw;
@@ -227,10 +225,9 @@ void trim_engine_hosts() {
 
 Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(take_host()) {
   for (int i = 0; i < 8; ++i) ev_[i] = host_.ev[i];
-  host_total_ = host_.total;
-  host_u64_ = host_.words;
-  ws_.err_host = reinterpret_cast<uint32_t*>(host_u64_ + 7);
-  *ws_.err_host = 0;
+  words_ = host_.words;
+  words_->lookback = 0;
+  ws_.err_host = &words_->lookback;
   // The budget caps what this call holds at once, on top of what was
   // already live when it started.
   const uint64_t live = DevicePool::get().live_bytes();
@@ -274,13 +271,13 @@ double Engine::elapsed_ms(int a, int b) {
 }
 
 U2 Engine::read_total(const U2* dev) {
-  SPTC_HIP(hipMemcpyAsync(host_total_, dev, sizeof(U2), hipMemcpyDeviceToHost, s_));
+  SPTC_HIP(hipMemcpyAsync(&words_->total, dev, sizeof(U2), hipMemcpyDeviceToHost, s_));
   return wait_total();
 }
 
 U2 Engine::wait_total() {
   SPTC_HIP(hipStreamSynchronize(s_));
-  return host_total_[0];
+  return words_->total;
 }
 
 void Engine::stage(const sptc_coo& t, StagedCOO* out) {
@@ -433,7 +430,8 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
     ws_.prepare(n, s_);
     if (sort_onesweep(n)) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
     const bool alt = sort_after_histogram(ws_, sorted.get(), nullptr, n, bits, s_);
-    run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_, host_total_);
+    run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_,
+               &words_->total);
     U = wait_total().a;
     launch_yrank(key.get(), n, 64, ~0ull, uniq.get(), U, 0, rank->get(), s_);
     rbits = mode_bits(U);
@@ -490,7 +488,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   // ---- column ranks: Y free keys -> ranks among the distinct ones -----------
   // ycol holds every Y entry's column, ytab maps a rank back to the Y free key
   // (ytab32: as 32-bit words when the keys fit them).  The number of ranks
-  // arrives with the match totals (host_total_[1]).
+  // arrives with the match totals (words_->ranks).
   const bool ranked = ynf > 0 && ny > 1;
   DevBuf<uint64_t> ytab, fk;
   DevBuf<uint32_t> ytab32, ycol, yfree32;
@@ -510,7 +508,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       const uint64_t nw = rank_words(ynf);
       rmap.reset(rank_map_bytes(ynf));
       rtmp.reset(scan_tmp_count(nw) + 1);
-      run_rank_map(Y.keys.get(), ny, ynf, ro, rmap.get(), rtmp.get(), host_total_ + 1, s_);
+      run_rank_map(Y.keys.get(), ny, ynf, ro, rmap.get(), rtmp.get(), &words_->ranks, s_);
     } else {
       fk.reset(ny);
       launch_yfree_extract(Y.keys.get(), ny, low_mask(ynf), fk.get(), s_);
@@ -521,13 +519,13 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       const bool alt = sort_after_histogram(ws_, fk.get(), nullptr, ny, ynf, s_);
       rtmp.reset(scan_tmp_count(ny) + 1);
       run_rank_sorted(alt ? ws_.alt_keys.get() : fk.get(), Y.keys.get(), ny, ynf, ro, rtmp.get(),
-                      host_total_ + 1, s_);
+                      &words_->ranks, s_);
     }
   }
 
   // ---- (c) index match ---------------------------------------------------
   // hdup: set when Y holds duplicate coordinates
-  uint64_t* const hdup = &host_total_[3].a;
+  uint64_t* const hdup = &words_->dup;
   *hdup = 0;
   const int tbits = ytable_bits(ncb, ny);
   DevBuf<U2> tmem((1ull << tbits) + 1);
@@ -552,7 +550,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     DevBuf<uint64_t> look;
     if (nx > kScanOneMax && 16 * nx <= budget_avail() / 16) look.reset(2 * nx);
     int tok = kt_.begin(s_);
-    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_, host_total_,
+    run_match(X.keys.get(), X.vals.get(), nx, ncb, tab, mo, 0, tmp.get(), s_, &words_->total,
               look.size() ? look.get() : nullptr);
     // keys read twice, plus the compacted active and row tables written
     kt_.end(tok, SPTC_K_MATCH, (double)nx * (16 + 24 + 24), s_);
@@ -564,7 +562,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   tmem.release();
   record(3);
   // width of the column field and the columns: the distinct free keys
-  const uint64_t ranks = ranked ? host_total_[1].a : ynf < 32 ? 1ull << ynf : 0;
+  const uint64_t ranks = ranked ? words_->ranks.a : ynf < 32 ? 1ull << ynf : 0;
   const int kyf = ranked ? mode_bits(ranks) : ynf;
   fk.release();
   rmap.release();
@@ -635,7 +633,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     int tok = kt_.begin(s_);
     launch_dense_count(da, eb, R, s_);
     kt_.end(tok, SPTC_K_DENSE, 8.0 * (double)ir, s_);
-    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, host_total_);
+    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, &words_->total);
     const uint64_t out_n = wait_total().a;
     info.nnz = out_n;
     info.nchunks = 1;
@@ -687,7 +685,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       launch_tdense_count(ta, std::min(kRowsPerLaunch, R - b), s_);
     }
     kt_.end(tok, SPTC_K_DENSE, 4.0 * (double)ir, s_);
-    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, host_total_);
+    run_row_count_scan(row_cnt.get(), out_off.get(), R, tmp.get(), s_, &words_->total);
     const uint64_t out_n = wait_total().a;
     info.nnz = out_n;
     info.nchunks = 1;
@@ -739,9 +737,9 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       bounds_a.push_back(A);
     } else {
       launch_max_row(row_prod.get(), R, scratch.get(), s_);
-      SPTC_HIP(hipMemcpyAsync(host_u64_, scratch.get(), 8, hipMemcpyDeviceToHost, s_));
+      SPTC_HIP(hipMemcpyAsync(&words_->max_row, scratch.get(), 8, hipMemcpyDeviceToHost, s_));
       SPTC_HIP(hipStreamSynchronize(s_));
-      if (cap < host_u64_[0]) {
+      if (cap < words_->max_row) {
         msg = "one X row's products exceed the memory budget";
         return SPTC_ERR_OOM_BUDGET;
       }
@@ -749,16 +747,16 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     uint64_t r0 = bounds_r.back();
     while (r0 < R) {
       launch_chunk_end(row_prod.get(), row_act.get(), R, r0, rmax, cap, scratch.get(), s_);
-      SPTC_HIP(hipMemcpyAsync(host_u64_, scratch.get(), 24, hipMemcpyDeviceToHost, s_));
+      SPTC_HIP(hipMemcpyAsync(words_->chunk, scratch.get(), 24, hipMemcpyDeviceToHost, s_));
       SPTC_HIP(hipStreamSynchronize(s_));
-      uint64_t r1 = host_u64_[0];
+      uint64_t r1 = words_->chunk[0];
       if (r1 <= r0) {
         msg = "partitioning made no progress";
         return SPTC_ERR_INTERNAL;
       }
       bounds_r.push_back(r1);
-      bounds_p.push_back(host_u64_[1]);
-      bounds_a.push_back(host_u64_[2]);
+      bounds_p.push_back(words_->chunk[1]);
+      bounds_a.push_back(words_->chunk[2]);
       r0 = r1;
     }
     record(4);
@@ -852,7 +850,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
         ra.a0 = bounds_a[c - 1];
         ra.rows = r1c - r0c;
         done = rowacc_count(ra, n, bounds_a[c] - bounds_a[c - 1], o_.count_only, &rplan,
-                            host_total_, s_, &kt_);
+                            words_->acc, s_, &kt_);
         out_n = rplan.outs;
         if (!done) rplan = RowAccPlan();
       }
@@ -872,12 +870,9 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
         const bool rowsort = kyf > 0 && kyf < bits && kyf <= 32 && prefer_row_sort();
         if (rowsort) {
           const uint64_t lrows = r1c - r0c;
-          RowRange* h = reinterpret_cast<RowRange*>(host_u64_ + 4);
-          h->ra = r0c;
-          h->rows = lrows;
-          h->lrow0 = 0;
-          h->out0 = 0;
-          SPTC_HIP(hipMemcpyAsync(rrange.get(), h, sizeof(RowRange), hipMemcpyHostToDevice, s_));
+          words_->range = RowRange{r0c, lrows, 0, 0};
+          SPTC_HIP(hipMemcpyAsync(rrange.get(), &words_->range, sizeof(RowRange),
+                                  hipMemcpyHostToDevice, s_));
           build_row_segments(rrange.get(), 1, lrows, row_prod.get(), kyf, &rseg, ws_, tmp.get(),
                              s_, prefer_bucket_tail(), row_act.get());
         }
@@ -1024,11 +1019,10 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   } else {
     record(4);
   }
-  double* const host_sum = reinterpret_cast<double*>(host_u64_ + 2);
-  launch_fold_sums(vsum.get(), host_sum, s_);
+  launch_fold_sums(vsum.get(), &words_->sum, s_);
   record(5);
   SPTC_HIP(hipStreamSynchronize(s_));
-  info.value_sum = *host_sum;
+  info.value_sum = words_->sum;
   kt_.collect(res->kstats, SPTC_K_COUNT);
   if (*ws_.err() != 0) {
     msg = "radix sort look-back exceeded its spin limit";

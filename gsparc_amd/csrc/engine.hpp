@@ -127,11 +127,25 @@ bool prefer_bucket_tail();
 // (SPTC_PROD_SORT, SPTC_BIG_TAIL, SPTC_SEG_RB, SPTC_SEG_IPT, SPTC_SEG_WIDE).
 bool prefer_row_acc();
 
+// Pinned words that a call's kernels and copies write and the host reads (or the
+// other way round).  Each use has words of its own: lookback stays set through
+// whatever runs before it is read.
+struct EngineWords {
+  U2 total;           // a scan's total
+  U2 ranks;           // a: distinct columns
+  U2 acc[3];          // the row accumulator's totals
+  uint64_t dup;       // Y holds duplicate coordinates
+  uint64_t chunk[3];  // a chunk's end
+  uint64_t max_row;   // products of the largest row
+  RowRange range;     // a chunk's rows, on their way to the device
+  double sum;         // value sum
+  uint32_t lookback;  // a look-back pass exceeded its wait limit
+};
+
 // Pinned words and events of an engine, kept between engines.
 struct EngineHost {
   hipEvent_t ev[8] = {};
-  U2* total = nullptr;        // [4]
-  uint64_t* words = nullptr;  // [8]
+  EngineWords* words = nullptr;
   int dev = 0;
 };
 void trim_engine_hosts();  // frees what is kept
@@ -177,7 +191,7 @@ class Engine {
 
  private:
   U2 read_total(const U2* dev);
-  // the total that a scan wrote to host_total_
+  // the total that a scan wrote to words_->total
   U2 wait_total();
   // Ranks of the contracted coordinates of X then Y in *rank (nx + ny);
   // returns the number of distinct tuples (0 and msg set on failure).
@@ -193,8 +207,7 @@ class Engine {
   EngineHost host_;
   hipEvent_t ev_[8];
   bool ev_used_[8] = {false};
-  U2* host_total_ = nullptr;
-  uint64_t* host_u64_ = nullptr;
+  EngineWords* words_ = nullptr;
 };
 
 }  // namespace sptc

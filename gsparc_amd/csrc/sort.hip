@@ -340,6 +340,16 @@ const SortCfg& sort_cfg() {
   return c;
 }
 
+// SPTC_LOOKBACK_FAILS=1: every look-back pass reports that its wait exceeded the
+// limit, though none did (tests of the error paths).
+bool lookback_fails() {
+  static const bool f = [] {
+    const char* e = getenv("SPTC_LOOKBACK_FAILS");
+    return e && e[0] == '1';
+  }();
+  return f;
+}
+
 // Calls f.template run<RB, IPT, NT>() for the configured tile of digit width rb.
 template <class F>
 void with_tile(int rb, F&& f) {
@@ -387,6 +397,7 @@ struct OnesweepPass {
                          a.ka, a.va, a.kb, a.vb, a.n, a.lo + a.pass * RB, a.ws->hist() + a.pass * R,
                          a.ws->status(), a.ws->counters() + a.pass, a.ws->epoch, a.ws->err());
     if (a.kt) a.kt->end(tok, a.cls, 24.0 * (double)a.n, a.s);
+    if (lookback_fails() && a.ws->err()) fill_u32(a.ws->err(), 1, 1, a.s);
   }
 };
 
