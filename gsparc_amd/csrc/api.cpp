@@ -269,6 +269,11 @@ sptc_status sptc_plan(const sptc_coo* X, const sptc_coo* Y, int32_t nc, const in
       }
       e.record(1);
       SPTC_HIP(hipStreamSynchronize(s));
+      st = e.check_sorts();
+      if (st != SPTC_OK) {
+        delete p;
+        return fail(st, e.msg);
+      }
       p->prepare_ms = e.elapsed_ms(0, 1);
     }
   } catch (const HipError& he) {
@@ -826,7 +831,7 @@ sptc_status sptc_sort_pairs(uint64_t* keys, float* vals, uint64_t n, int32_t nbi
     ws.ensure(n, rb, s);
     const int passes = radix_passes(nbits, rb);
     PinnedWord err;
-    ws.err_host = err.p;
+    ws.err_word = err.p;
     ws.prepare(n, s);
     if (sort_onesweep(n)) histogram(ws, keys, n, passes, s);
     if (sort_after_histogram(ws, keys, vals, n, nbits, s)) {

@@ -177,7 +177,8 @@ sptc_status BatchEngine::plan(int B, const sptc_coo* X, const sptc_coo* Y, const
   row_act_.reset(nx1);
   itab_.reset(3 * (B + 1));
   dup_.reset(B);
-  bad_.reset(1);
+  bad_.reset(2);
+  ws_.err_word = bad_.get() + 1;
   digest_.reset(2);
   scratch_.reset(4);
   tmp_.reset(scan_tmp_count(n1) + 1);
@@ -185,6 +186,11 @@ sptc_status BatchEngine::plan(int B, const sptc_coo* X, const sptc_coo* Y, const
   sptc_status st = run(s, true);
   if (st != SPTC_OK) return st;
   SPTC_HIP(hipStreamSynchronize(s));
+  for (const EscChunk& c : esc_)  // (operands are sorted without look-back)
+    if (!c.rowsort && sort_onesweep(c.n)) {
+      if ((st = sync(s)) != SPTC_OK) return st;
+      break;
+    }
   planned_ = true;
   info.instances = B;
   info.nnz_in = N_;
@@ -399,7 +405,7 @@ sptc_status BatchEngine::build_chunks(hipStream_t s) {
 sptc_status BatchEngine::run(hipStream_t s, bool P) {
   const uint32_t B = B_;
   KTimer* kt = (P && kt_.on) ? &kt_ : nullptr;
-  fill_u32(bad_.get(), 0, 1, s);
+  fill_u32(bad_.get(), 0, 2, s);
 
   // ---- (a)+(b) linearize and sort every operand (segmented) ---------------
   {
@@ -707,11 +713,15 @@ sptc_status BatchEngine::launch_graph(hipStream_t s) {
 }
 
 sptc_status BatchEngine::sync(hipStream_t s) {
-  uint32_t bad = 0;
-  SPTC_HIP(hipMemcpyAsync(&bad, bad_.get(), 4, hipMemcpyDeviceToHost, s));
+  uint32_t bad[2] = {0, 0};
+  SPTC_HIP(hipMemcpyAsync(bad, bad_.get(), sizeof(bad), hipMemcpyDeviceToHost, s));
   SPTC_HIP(hipStreamSynchronize(s));
-  if (bad) {
+  if (bad[0]) {
     msg = "operand index arrays changed since the batch was planned";
+    return SPTC_ERR_INTERNAL;
+  }
+  if (bad[1]) {
+    msg = "radix sort look-back exceeded its spin limit";
     return SPTC_ERR_INTERNAL;
   }
   return SPTC_OK;

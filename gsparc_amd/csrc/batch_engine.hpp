@@ -76,7 +76,7 @@ class BatchEngine {
   void enqueue(hipStream_t s) { run(s, false); }
   sptc_status capture();
   sptc_status launch_graph(hipStream_t s);
-  // Waits for stream s and reports a stale plan.
+  // Waits for stream s and reports a stale plan or a failed look-back sort.
   sptc_status sync(hipStream_t s);
   // Value sums of instances [i0, i1) by one launch and one wait: twelve requests
   // took a buffer, two launches and a wait each.
@@ -118,7 +118,8 @@ class BatchEngine {
   DevBuf<BInst> inst_;
   DevBuf<uint64_t> act_prefix_, act_ypos_, row_key_, row_prod_, row_act_, itab_;
   DevBuf<float> act_xval_;
-  DevBuf<uint32_t> act_row_, dup_, bad_;
+  DevBuf<uint32_t> act_row_, dup_;
+  DevBuf<uint32_t> bad_;  // [0] stale plan, [1] a look-back sort gave up
   DevBuf<U2> tmp_;
   DevBuf<uint64_t> digest_, scratch_;
   std::vector<uint64_t> iP_, iA_, iR_, ytoff_h_;

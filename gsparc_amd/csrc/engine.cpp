@@ -227,7 +227,7 @@ Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(take_hos
   for (int i = 0; i < 8; ++i) ev_[i] = host_.ev[i];
   words_ = host_.words;
   words_->lookback = 0;
-  ws_.err_host = &words_->lookback;
+  ws_.err_word = &words_->lookback;
   // The budget caps what this call holds at once, on top of what was
   // already live when it started.
   const uint64_t live = DevicePool::get().live_bytes();
@@ -363,6 +363,12 @@ void Engine::prepare(const StagedCOO& t, const Layout& lay, Operand* out, const 
     std::swap(out->keys, ws_.alt_keys);
     std::swap(out->vals, ws_.alt_vals);
   }
+}
+
+sptc_status Engine::check_sorts() {
+  if (!words_->lookback) return SPTC_OK;
+  msg = "radix sort look-back exceeded its spin limit";
+  return SPTC_ERR_INTERNAL;
 }
 
 sptc_status Engine::check_indices(const StagedCOO& t, const uint64_t* dims, const char* name) {
@@ -555,6 +561,8 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     // keys read twice, plus the compacted active and row tables written
     kt_.end(tok, SPTC_K_MATCH, (double)nx * (16 + 24 + 24), s_);
     tot = wait_total();
+    // (tables of operands out of order mean nothing: no further)
+    if (const sptc_status st = check_sorts()) return st;
   }
   const uint64_t ir = tot.a;
   const uint64_t A = tot.b >> 32;
@@ -1024,10 +1032,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   SPTC_HIP(hipStreamSynchronize(s_));
   info.value_sum = words_->sum;
   kt_.collect(res->kstats, SPTC_K_COUNT);
-  if (*ws_.err() != 0) {
-    msg = "radix sort look-back exceeded its spin limit";
-    return SPTC_ERR_INTERNAL;
-  }
+  if (const sptc_status st = check_sorts()) return st;
   float t;
   auto el = [&](int a, int b) -> double {
     if (!ev_used_[a] || !ev_used_[b]) return 0.0;

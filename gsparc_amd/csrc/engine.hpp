@@ -173,6 +173,10 @@ class Engine {
                            const Layout& yl, Operand* ox, Operand* oy);
   // Match + partition + accumulate.  X and Y are prepared operands.
   sptc_status contract(const Operand& X, const Operand& Y, sptc_result_s* res);
+  // SPTC_ERR_INTERNAL (detail in msg) when a look-back pass of this engine gave
+  // up: what it sorted is not in order.  The stream must have been waited for;
+  // whoever keeps prepared operands checks this first.
+  sptc_status check_sorts();
   uint64_t budget() const { return budget_; }
   const sptc_opts& options() const { return o_; }
   // budget bytes above what was live when the engine was made

@@ -2,6 +2,7 @@
 #include "serve.hpp"
 
 #include <cstring>
+#include <stdexcept>
 
 namespace sptc {
 
@@ -180,6 +181,7 @@ std::shared_ptr<Operand> Server::prepared(int32_t t, const Layout& lay) {
     Engine e(plan_stream_, o);
     e.prepare(rt->staged, lay, op.get());
     SPTC_HIP(hipStreamSynchronize(plan_stream_));
+    if (e.check_sorts() != SPTC_OK) throw std::runtime_error(e.msg);
   }
   rt->prepared[k] = op;
   std::lock_guard<std::mutex> g(mu_);

@@ -28,7 +28,9 @@ struct SortWorkspace {
   DevBuf<uint32_t> rts_off;     // [R][tiles] their exclusive scan
   DevBuf<U2> rts_tmp;           // scan scratch
   uint32_t epoch = 0;
-  uint32_t* err_host = nullptr; // pinned host memory, set by a failed look-back
+  // set by a failed look-back: pinned host memory or a device word, which the
+  // workspace's user clears, and reads after a wait
+  uint32_t* err_word = nullptr;
 
   // Grows the workspace to hold `n` keys (and values) at `rb` radix bits.
   void ensure(uint64_t n, int rb, hipStream_t s, bool vals = true);
@@ -40,7 +42,7 @@ struct SortWorkspace {
     return reinterpret_cast<uint32_t*>(sweep.get() + ((uint64_t)kMaxPasses << rb));
   }
   uint64_t* status() const { return sweep.get() + ((uint64_t)kMaxPasses << rb) + kSweepHead; }
-  uint32_t* err() const { return err_host; }
+  uint32_t* err() const { return err_word; }
   static uint64_t bytes_per_key(int rb);
 };
 

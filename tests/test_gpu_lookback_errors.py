@@ -24,6 +24,15 @@ rng = np.random.default_rng(1)
 X = random_coo(rng, (300, 80, 50), 30_000)   # more than one sort tile, look-back sizes
 Y = random_coo(rng, (50, 900), 20_000)
 small = random_coo(rng, (30, 20, 50), 3000)  # operands of one tile: no look-back pass
+v = random_coo(rng, (50,), 50)
+
+def serve():
+    srv = sptc.Server(budget_bytes=4 << 30)
+    try:
+        a, b = srv.add_tensor(X), srv.add_tensor(Y)
+        srv.wait(srv.submit(a, b, [2], [0]))
+    finally:
+        srv.close()
 
 def pairs():
     k = torch.randint(0, 1 << 40, (50_000,), dtype=torch.int64, device="cuda")
@@ -35,6 +44,9 @@ forms = {
     "call": lambda: sptc.SpTC(X, Y, [2], [0]),
     "esc": lambda: sptc.SpTC(X, Y, [2], [0], dense_accumulator=-1),
     "count": lambda: sptc.SpTC(X, Y, [2], [0], dense_accumulator=-1, count_only=True),
+    "plan": lambda: sptc.Plan(X, Y, [2], [0]),
+    "batch": lambda: sptc.Batch([(X, v, [2], [0])], dense_accumulator=-1),
+    "server": serve,
     "pairs": pairs,
     "small": lambda: sptc.SpTC(small, small, [2], [2]),
 }
@@ -63,7 +75,7 @@ def test_failed_look_back_is_reported(gpu, product_sort):
     env = {"SPTC_PROD_SORT": "rows"} if product_sort else {}
     print(f"[look-back] {env}", flush=True)
     good = _forms(**env)
-    assert set(good.values()) == {"ok"} and len(good) == 5
+    assert set(good.values()) == {"ok"} and len(good) == 8
     bad = _forms(SPTC_LOOKBACK_FAILS="1", **env)
     assert bad.pop("small") == "ok"
     assert bad == {k: str(sptc.ERR_INTERNAL) for k in bad}
