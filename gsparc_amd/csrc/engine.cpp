@@ -784,7 +784,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     uint64_t max_rows = 0;
     for (size_t c = 1; c < bounds_r.size(); ++c)
       max_rows = std::max(max_rows, bounds_r[c] - bounds_r[c - 1]);
-    // the product sort's buffers, allocated by the first chunk that takes it
+    // the product sort's buffers, allocated by a chunk that takes it
     DevBuf<uint64_t> kA;
     DevBuf<float> vA;
     DevBuf<U2> tmp;
@@ -853,6 +853,20 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       if (!n) continue;
       bool done = false;
       uint64_t out_n = 0;
+      if (rowacc && kA.size() &&
+          DevicePool::get().live_bytes() +
+                  rowacc_bytes(r1c - r0c, bounds_a[c] - bounds_a[c - 1], n, ranks) +
+                  out_per * (ir - P0) >
+              budget_) {
+        // an earlier chunk fell back and the chunks are sized for either, not both
+        SPTC_HIP(hipStreamSynchronize(s_));
+        kA.release();
+        vA.release();
+        tmp.release();
+        trow.release();
+        rseg = RowSegPlan();
+        ws_.release();
+      }
       if (rowacc) {
         ra.r0 = r0c;
         ra.a0 = bounds_a[c - 1];

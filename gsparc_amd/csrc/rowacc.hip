@@ -1214,8 +1214,9 @@ uint64_t rowacc_bytes(uint64_t rows, uint64_t owners, uint64_t nprod, uint64_t K
   const uint64_t live = std::min(rows, owners);
   const uint64_t least = K <= 1ull << kRowAccMaxBits ? min_slabs((uint32_t)K) : 1;
   const uint64_t items = nprod / 256 * least + nprod / kItemProds;  // long rows: 256 products
-  return live * (28 + 4 + 4 + kNearBytes) + 8 * nprod + items * (kItemBytes + 4 + 8) +
-         4 * (owners * (least + 1) + nprod / kItemRun) + 4 * nprod + (2ull << 20);
+  const uint64_t b = live * (28 + 4 + 4 + kNearBytes) + 8 * nprod + items * (kItemBytes + 4 + 8) +
+                     4 * (owners * (least + 1) + nprod / kItemRun) + 4 * nprod + (2ull << 20);
+  return b + b / 8;  // the pool rounds large blocks up by as much
 }
 
 bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool count_only,

@@ -34,6 +34,15 @@ struct SortWorkspace {
 
   // Grows the workspace to hold `n` keys (and values) at `rb` radix bits.
   void ensure(uint64_t n, int rb, hipStream_t s, bool vals = true);
+  // Gives everything back (the stream must have been waited for).
+  void release() {
+    alt_keys.release();
+    alt_vals.release();
+    sweep.release();
+    rts_cnt.release();
+    rts_off.release();
+    rts_tmp.release();
+  }
   // Clears histograms, counters and look-back words before a sort of n keys
   // (onesweep only).
   void prepare(uint64_t n, hipStream_t s);

@@ -105,6 +105,46 @@ def test_heavy_row_goes_to_the_product_sort(gpu):
     check(*build(rng, 1000, [[900] * 300, [5, 6], [700]]))
 
 
+def test_fallback_chunk_beside_others_under_a_budget(gpu):
+    """A budget that cuts the products into chunks; the first holds a row that
+    sends it to the product sort, the others take the row accumulator.  The
+    sort's buffers and the accumulator's tables do not fit together.  Results as
+    without a budget."""
+    import torch
+
+    class Dev:
+        pass
+
+    def dev(dims, idx, val):
+        t = Dev()
+        t.dims, t.order, t.nnz = dims, len(dims), len(val)
+        t.idx = [torch.from_numpy(i.astype(np.int32)).cuda() for i in idx]
+        t.val = torch.from_numpy(val.astype(np.float32)).cuda()
+        return t
+
+    rng = np.random.default_rng(12)
+    K, heavy, C, N, per = 1000, 300, 300, 1_500_000, 8
+    xr = np.concatenate([np.zeros(heavy, np.int64), 1 + np.repeat(np.arange(N), 2)])
+    xc = np.concatenate([np.arange(heavy), heavy + rng.integers(0, C, 2 * N)])
+    yc = np.concatenate([np.repeat(np.arange(heavy), 900), heavy + np.repeat(np.arange(C), per)])
+    yj = np.concatenate([rng.choice(K, 900, replace=False) for _ in range(heavy)] +
+                        [rng.choice(K, per, replace=False) for _ in range(C)])
+    X = dev((N + 1, heavy + C), [xr, xc], rng.random(len(xr)) + 0.1)
+    Y = dev((heavy + C, K), [yc, yj], rng.random(len(yc)) + 0.1)
+    run = lambda **kw: sptc.SpTC(X, Y, [1], [0], dense_accumulator=-1, on_device=True, **kw)
+    free = run()
+    want = free.to_host()
+    chunks = set()
+    for f in (0.8, 0.9, 1.0, 1.1):
+        r = run(mem_budget_bytes=int(f * 35 * free.ir_nnz) + 44 * len(xr), kernel_timing=True)
+        chunks.add(r.info.nchunks)
+        st = r.kernel_stats()
+        assert st["sort_products"][0] + st["sort_products_wide"][0] > 0  # the first chunk
+        for a, b in zip(r.to_host(), want):
+            np.testing.assert_array_equal(a, b)
+    assert min(chunks) > 1 and max(chunks) > 2
+
+
 def test_duplicate_columns_of_one_owner(gpu):
     """Y with duplicate coordinates: one-owner rows are summed like others."""
     rng = np.random.default_rng(10)
