@@ -618,12 +618,31 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   }
   info.accumulator = use_dense ? 1 : (use_tdense ? 2 : 0);
   std::vector<uint64_t> bounds_r{0}, bounds_p{0}, bounds_a{0};
+  // What the accumulation's kernels use goes back to the pool after the last wait,
+  // however the call ends: another thread may take a block for its own stream.
+  DevBuf<uint32_t> row_cnt;
+  DevBuf<uint64_t> out_off, cur, scratch;
+  DevBuf<U2> tmp;
+  // the product sort's, allocated by a chunk that takes it
+  DevBuf<uint64_t> kA;
+  DevBuf<float> vA;
+  DevBuf<uint32_t> trow;
+  DevBuf<RowRange> rrange;
+  RowSegPlan rseg;
+  RowAccPlan rplan;
+  struct Wait {
+    hipStream_t s;
+    bool idle = false;
+    ~Wait() {
+      if (!idle) (void)hipStreamSynchronize(s);
+    }
+  } wait{s_};
   if (use_dense) {
     record(4);
     const int eb = kyf <= 8 ? 8 : (kyf <= 10 ? 10 : 13);
-    DevBuf<uint32_t> row_cnt(R);
-    DevBuf<uint64_t> out_off(R + 1);
-    DevBuf<U2> tmp(scan_tmp_count(R) + 1);
+    row_cnt.reset(R);
+    out_off.reset(R + 1);
+    tmp.reset(scan_tmp_count(R) + 1);
     DenseArgs da;
     std::memset(&da, 0, sizeof(da));
     da.act_prefix = act_prefix.get();
@@ -667,10 +686,10 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     }
   } else if (use_tdense) {
     record(4);
-    DevBuf<uint64_t> cur(A ? A : 1);
-    DevBuf<uint32_t> row_cnt(R);
-    DevBuf<uint64_t> out_off(R + 1);
-    DevBuf<U2> tmp(scan_tmp_count(R) + 1);
+    cur.reset(A ? A : 1);
+    row_cnt.reset(R);
+    out_off.reset(R + 1);
+    tmp.reset(scan_tmp_count(R) + 1);
     TDenseArgs ta;
     std::memset(&ta, 0, sizeof(ta));
     ta.act_prefix = act_prefix.get();
@@ -723,7 +742,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     kt_.end(tok, SPTC_K_DENSE, 8.0 * (double)ir + 16.0 * (double)out_n, s_);
     res->chunks.push_back(std::move(oc));
   } else if (ir) {
-    DevBuf<uint64_t> scratch(4);
+    scratch.reset(4);
     const uint64_t live = DevicePool::get().live_bytes();
     const uint64_t free_b = budget_ > live ? budget_ - live : 0;
     const uint64_t per_prod = 12 + SortWorkspace::bytes_per_key(10) + 1;
@@ -784,11 +803,6 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     uint64_t max_rows = 0;
     for (size_t c = 1; c < bounds_r.size(); ++c)
       max_rows = std::max(max_rows, bounds_r[c] - bounds_r[c - 1]);
-    // the product sort's buffers, allocated by a chunk that takes it
-    DevBuf<uint64_t> kA;
-    DevBuf<float> vA;
-    DevBuf<U2> tmp;
-    DevBuf<uint32_t> trow;
     auto sort_buffers = [&] {
       if (kA.size()) return;
       kA.reset(chunk_cap);
@@ -805,9 +819,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     };
     const uint64_t fmask = low_mask(kyf);
     if (kyf <= 32 && !partition_only) ycol_or_make();
-    // row-segmented product sort
-    DevBuf<RowRange> rrange(1);
-    RowSegPlan rseg;
+    rrange.reset(1);
     // row accumulator (a tight budget keeps to the product sort, whose parts the
     // chunks are sized for)
     bool rowacc = kyf > 0 && kyf < 32 && prefer_row_acc() && !partition_only;
@@ -818,7 +830,6 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       const uint64_t held = DevicePool::get().live_bytes();
       rowacc = held + rowacc_bytes(max_rows, max_act, chunk_cap, ranks) + out_per * ir <= budget_;
     }
-    RowAccPlan rplan;
     RowAccArgs ra;
     if (rowacc) {
       ra.act_prefix = act_prefix.get();
@@ -1044,6 +1055,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   launch_fold_sums(vsum.get(), &words_->sum, s_);
   record(5);
   SPTC_HIP(hipStreamSynchronize(s_));
+  wait.idle = true;
   info.value_sum = words_->sum;
   kt_.collect(res->kstats, SPTC_K_COUNT);
   if (const sptc_status st = check_sorts()) return st;

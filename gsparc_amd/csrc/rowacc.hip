@@ -1202,9 +1202,13 @@ NearArgs near_args(const RowAccArgs& a, const RowAccPlan& p) {
   return g;
 }
 
+// A buffer that grows goes back to the pool, where another thread may take it for
+// its own stream: the kernels of the chunk before are waited for first.
 template <class T>
-void room(DevBuf<T>& b, uint64_t n) {
-  if (b.size() < n) b.reset(n);
+void room(DevBuf<T>& b, uint64_t n, hipStream_t s) {
+  if (b.size() >= n) return;
+  if (b.size()) SPTC_HIP(hipStreamSynchronize(s));
+  b.reset(n);
 }
 
 }  // namespace
@@ -1225,16 +1229,17 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   const bool by_act = owners < a.rows;
   const uint64_t rows = by_act ? owners : a.rows;
   if (nprod >= (1ull << 32)) throw std::length_error("row accumulator chunk");
-  room(p->live_row, rows);
-  room(p->live_cnt, rows);
-  room(p->live_src, rows);
-  room(p->s_live, rows);
-  room(p->s_prod, rows);
-  room(p->l_live, rows);
-  room(p->tmp, scan_tmp_count(rows) + 1);
+  room(p->live_row, rows, s);
+  room(p->live_cnt, rows, s);
+  room(p->live_src, rows, s);
+  room(p->s_live, rows, s);
+  room(p->s_prod, rows, s);
+  room(p->l_live, rows, s);
   // (column spaces too wide to cut into slabs take no long rows)
   const bool slabs = a.K <= 1u << kRowAccMaxBits;
   const uint32_t least = slabs ? min_slabs(a.K) : 1;
+  // (items: long rows hold more than 256 products)
+  room(p->tmp, scan_tmp_count(std::max(rows, nprod / 256 * least + nprod / kItemProds)) + 1, s);
   const uint64_t heavy = std::max(kHeavyItem, nprod >> 10);
   host[1].a = 0;
   auto kinds = [&](auto op) {
@@ -1260,8 +1265,8 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   if (max_split >= (1ull << 32)) return false;  // 32-bit places in the descriptors
   if (p->nshort) {
     if (!count_only) {
-      room(p->tcol, p->short_prods);
-      room(p->tval, p->short_prods);
+      room(p->tcol, p->short_prods, s);
+      room(p->tval, p->short_prods, s);
     }
     GroupArgs g{a,
                 p->live_row.get(),
@@ -1287,13 +1292,13 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
     // row against another gather and LDS atomic per product)
     const uint64_t max_words = p->nlong * (a.K / 64 + 1) + max_items;
     p->keep_words = !count_only && max_words * 8 <= 4 * nprod + (1ull << 20);
-    room(p->l_item, p->nlong + 1);
-    room(p->l_split, p->nlong);
-    room(p->l_word, p->nlong);
-    room(p->item, max_items * (kItemBytes / 4));
-    room(p->item_cnt, max_items);
-    room(p->split, max_split);
-    if (p->keep_words) room(p->words, max_words);
+    room(p->l_item, p->nlong + 1, s);
+    room(p->l_split, p->nlong, s);
+    room(p->l_word, p->nlong, s);
+    room(p->item, max_items * (kItemBytes / 4), s);
+    room(p->item_cnt, max_items, s);
+    room(p->split, max_split, s);
+    if (p->keep_words) room(p->words, max_words, s);
     SlabOp slab{a, least, p->l_live.get(), p->live_row.get(), p->nlong, p->l_item.get(),
                 p->l_split.get(), p->l_word.get()};
     run_scan(slab, p->nlong, p->tmp.get(), s, true, host + 2);
@@ -1319,9 +1324,9 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
                          p->item_cnt.get());
     kt->end(tok, SPTC_K_REDUCE, (count_only ? 8.0 : 4.0) * (double)(nprod - p->short_prods), s);
   }
-  room(p->l_near, p->live);
-  room(p->near_pre, p->live);
-  room(p->near, p->live * (kNearBytes / 8));
+  room(p->l_near, p->live, s);
+  room(p->near_pre, p->live, s);
+  room(p->near, p->live * (kNearBytes / 8), s);
   OutOp out{a,
             p->live_cnt.get(),
             p->live_row.get(),
@@ -1358,8 +1363,7 @@ void rowacc_emit(const RowAccArgs& a, RowAccPlan& p, uint64_t nprod, uint32_t* o
     kt->end(tok, SPTC_K_EXPAND, 24.0 * (double)p.near_outs, s);
   }
   if (p.items) {
-    room(p.item_off, p.items);
-    room(p.tmp, scan_tmp_count(p.items) + 1);
+    room(p.item_off, p.items, s);
     const int tok = kt->begin(s);
     ItemOutOp op{p.item_cnt.get(), reinterpret_cast<const Item*>(p.item.get()), p.l_near.get(),
                  p.item_off.get()};
