@@ -223,9 +223,25 @@ void trim_engine_hosts() {
   for (EngineHost& h : old) destroy_host(h);
 }
 
-Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(take_host()) {
-  for (int i = 0; i < 8; ++i) ev_[i] = host_.ev[i];
-  words_ = host_.words;
+HostLease::HostLease(hipStream_t s) : s_(s), host_(take_host()) {}
+
+HostLease::~HostLease() {
+  // work that a failed call left behind may still write to the words; if it
+  // cannot be waited for they are not handed on
+  if (hipStreamSynchronize(s_) == hipSuccess) {
+    HostCache& c = host_cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    if (c.kept.size() < kHostKept) {
+      c.kept.push_back(host_);
+      return;
+    }
+  }
+  destroy_host(host_);
+}
+
+Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(s) {
+  for (int i = 0; i < 8; ++i) ev_[i] = host_.get().ev[i];
+  words_ = host_.get().words;
   words_->lookback = 0;
   ws_.err_word = &words_->lookback;
   // The budget caps what this call holds at once, on top of what was
@@ -241,20 +257,6 @@ Engine::Engine(hipStream_t s, const sptc_opts& o) : s_(s), o_(o), host_(take_hos
   }
   rb_ = radix_bits_supported(o.radix_bits) ? o.radix_bits : 0;  // 0: per sort
   kt_.on = o.kernel_timing != 0;
-}
-
-Engine::~Engine() {
-  // work that a failed call left behind may still write to the words; if it
-  // cannot be waited for they are not handed on
-  if (hipStreamSynchronize(s_) == hipSuccess) {
-    HostCache& c = host_cache();
-    std::lock_guard<std::mutex> g(c.mu);
-    if (c.kept.size() < kHostKept) {
-      c.kept.push_back(host_);
-      return;
-    }
-  }
-  destroy_host(host_);
 }
 
 void Engine::record(int i) {

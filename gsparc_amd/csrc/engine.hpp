@@ -148,12 +148,24 @@ struct EngineHost {
   EngineWords* words = nullptr;
   int dev = 0;
 };
+// One of them, for work on stream s, which is waited for before it is handed on.
+class HostLease {
+ public:
+  explicit HostLease(hipStream_t s);
+  ~HostLease();
+  HostLease(const HostLease&) = delete;
+  HostLease& operator=(const HostLease&) = delete;
+  const EngineHost& get() const { return host_; }
+
+ private:
+  hipStream_t s_;
+  EngineHost host_;
+};
 void trim_engine_hosts();  // frees what is kept
 
 class Engine {
  public:
   Engine(hipStream_t s, const sptc_opts& o);
-  ~Engine();
   // Copies host-resident COO arrays to the device (no-op for device ones).
   void stage(const sptc_coo& t, StagedCOO* out);
   // SPTC_ERR_BAD_ARGS (detail in msg) when an index of t is not below its
@@ -208,10 +220,10 @@ class Engine {
   int rb_ = 8;
   SortWorkspace ws_;
   KTimer kt_;
-  EngineHost host_;
   hipEvent_t ev_[8];
   bool ev_used_[8] = {false};
   EngineWords* words_ = nullptr;
+  HostLease host_;  // last: the stream is waited for before the buffers above go back
 };
 
 }  // namespace sptc
