@@ -187,7 +187,7 @@ sptc_status BatchEngine::plan(int B, const sptc_coo* X, const sptc_coo* Y, const
   if (st != SPTC_OK) return st;
   SPTC_HIP(hipStreamSynchronize(s));
   for (const EscChunk& c : esc_)  // (operands are sorted without look-back)
-    if (!c.rowsort && sort_onesweep(c.n)) {
+    if (!c.rowsort && sort_onesweep(c.n, c.rb)) {
       if ((st = sync(s)) != SPTC_OK) return st;
       break;
     }
@@ -592,7 +592,7 @@ sptc_status BatchEngine::run(hipStream_t s, bool P) {
       ws_.ensure(c.n, c.rb, s);
       const int passes = radix_passes(c.bits, c.rb);
       ws_.prepare(c.n, s);
-      if (sort_onesweep(c.n)) histogram(ws_, kA_.get(), c.n, passes, s);
+      if (sort_onesweep(c.n, c.rb)) histogram(ws_, kA_.get(), c.n, passes, s);
       alt = sort_after_histogram(ws_, kA_.get(), vA_.get(), c.n, c.bits, s, kt, SPTC_K_SORT_PROD);
     }
     const uint64_t* sk = alt ? ws_.alt_keys.get() : kA_.get();

@@ -350,7 +350,7 @@ void Engine::prepare(const StagedCOO& t, const Layout& lay, Operand* out, const 
   const int passes = radix_passes(lay.nbits - lo, rb);
   ws_.ensure(n, rb, s_);
   ws_.prepare(n, s_);
-  const bool hist = sort_onesweep(n);
+  const bool hist = sort_onesweep(n, rb);
   launch_linearize(a, t.idx_bytes, n, out->keys.get(), ws_.hist(),
                    hist && passes <= kMaxFusedPasses ? passes : 0, rb, s_, lo);
   kt_.end(tok, SPTC_K_LINEARIZE, (double)n * (lay.order * t.idx_bytes + 8), s_);
@@ -436,7 +436,7 @@ uint64_t Engine::contract_ranks(const StagedCOO& sx, const StagedCOO& sy, const 
     const int rb = rb_ ? rb_ : choose_radix_bits(bits);
     ws_.ensure(n, rb, s_, /*vals=*/false);
     ws_.prepare(n, s_);
-    if (sort_onesweep(n)) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
+    if (sort_onesweep(n, rb)) histogram(ws_, sorted.get(), n, radix_passes(bits, rb), s_);
     const bool alt = sort_after_histogram(ws_, sorted.get(), nullptr, n, bits, s_);
     run_unique(alt ? ws_.alt_keys.get() : sorted.get(), n, uniq.get(), tmp.get(), s_,
                &words_->total);
@@ -523,7 +523,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       const int rbf = rb_ ? rb_ : choose_radix_bits(ynf);
       ws_.ensure(ny, rbf, s_, /*vals=*/false);
       ws_.prepare(ny, s_);
-      if (sort_onesweep(ny)) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
+      if (sort_onesweep(ny, rbf)) histogram(ws_, fk.get(), ny, radix_passes(ynf, rbf), s_);
       const bool alt = sort_after_histogram(ws_, fk.get(), nullptr, ny, ynf, s_);
       rtmp.reset(scan_tmp_count(ny) + 1);
       run_rank_sorted(alt ? ws_.alt_keys.get() : fk.get(), Y.keys.get(), ny, ynf, ro, rtmp.get(),
@@ -946,7 +946,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
           ea.out_vals = pv;
         }
         ea.hist = ws_.hist();
-        const bool hist = sort_onesweep(n);
+        const bool hist = sort_onesweep(n, rb);
         ea.passes = hist && passes <= kMaxFusedPasses ? passes : 0;
         ea.vsum = vsum.get();
         int tok = kt_.begin(s_);

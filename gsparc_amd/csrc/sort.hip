@@ -463,9 +463,9 @@ int choose_radix_bits(int nbits) {
   return 8;
 }
 
-bool sort_onesweep(uint64_t n) {
+bool sort_onesweep(uint64_t n, int rb) {
   const int m = sort_cfg().mode;
-  return m == 2 || (m == 0 && n <= kOnesweepMax);
+  return m == 2 || (m == 0 && n <= onesweep_max(rb));
 }
 
 uint64_t SortWorkspace::bytes_per_key(int rb) {
@@ -480,7 +480,7 @@ void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s, bool vals) {
   if (vals && alt_vals.size() < n) alt_vals.reset(n ? n : 1);
   const uint64_t tiles = ceil_div(n ? n : 1, sort_tile_items(rb_));
   rb = rb_;
-  if (sort_onesweep(n)) {
+  if (sort_onesweep(n, rb)) {
     if (sweep.size() < kMaxPasses * R + kSweepHead + tiles * R)
       sweep.reset(kMaxPasses * R + kSweepHead + tiles * R);
   } else {  // (each by its own size: segmented sorts grow the matrices alone)
@@ -492,7 +492,7 @@ void SortWorkspace::ensure(uint64_t n, int rb_, hipStream_t s, bool vals) {
 }
 
 void SortWorkspace::prepare(uint64_t n, hipStream_t s) {
-  if (!sort_onesweep(n)) return;
+  if (!sort_onesweep(n, rb)) return;
   const uint64_t R = 1ull << rb;
   fill_u64(sweep.get(), 0, kMaxPasses * R + kSweepHead + ceil_div(n, sort_tile_items(rb)) * R, s);
   epoch = 0;
@@ -539,7 +539,7 @@ bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
   const int passes = radix_passes(nbits - lo, rb);
   if (!n || !passes) return false;
   if (n >= (1ull << 32)) throw std::length_error("radix sort of 2^32 or more keys");
-  const bool onesweep = sort_onesweep(n);
+  const bool onesweep = sort_onesweep(n, rb);
   const uint64_t tiles = ceil_div(n, sort_tile_items(rb));
   const int tag = (cls == SPTC_K_SORT_PROD || cls == SPTC_K_SORT_PROD_WIDE) ? 1 : 0;
   const int kcls = (cls == SPTC_K_SORT_PROD && rb > 8) ? SPTC_K_SORT_PROD_WIDE : cls;

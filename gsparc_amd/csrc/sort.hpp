@@ -61,11 +61,18 @@ bool radix_bits_supported(int rb);
 // True when n keys are sorted by one-launch passes with look-back, which need
 // the digit histograms of all passes up front (ws.prepare, then a producer or
 // histogram()); reduce-then-scan passes count per tile themselves.
-// The line: 0.3e6 pairs of 40 bits 178 us against 322, 1e6 (with linearize) 303
-// against 348, 3e6 326 against 290, 77e6 4.5 ms against 3.8: past a few tiles per
-// CU the look-back's status words cost more than the launches they save.
+// The line, look-back against reduce-then-scan: with 8- and 9-bit digits 0.26e6 pairs
+// of 40 bits 116 us against 167, 1e6 165 against 195, 2e6 212 against 206 (24 bits
+// 154 / 139, 64 bits 282 / 293), 77e6 4.5 ms against 3.8: past a few tiles per CU the
+// status words cost more than the launches they save.  Wider digits have more of
+// them per key, so their line lies lower: 10 bits at 0.26e6 pairs 140 us against
+// 144, 0.4e6 160 / 149, 2e6 330 / 208; 11 bits at 0.1e6 146 / 148, 0.2e6 173 / 152,
+// 2e6 472 / 267.
 constexpr uint64_t kOnesweepMax = 1ull << 21;
-bool sort_onesweep(uint64_t n);
+constexpr uint64_t onesweep_max(int rb) {
+  return rb <= 9 ? kOnesweepMax : rb == 10 ? 1ull << 18 : 1ull << 16;
+}
+bool sort_onesweep(uint64_t n, int rb);
 // Linearizes and sorts up to one tile of nonzeros in one launch, on bits [lo, 64);
 // false when there are more.
 bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,

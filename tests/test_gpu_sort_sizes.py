@@ -1,7 +1,10 @@
 """Operand preparation at the sizes where the sort changes its form: one
 workgroup in LDS (up to one tile of 6144 nonzeros), one-launch look-back passes
-above, reduce-then-scan passes on X's free bits alone above 2^21.  The plan's contraction with a permutation returns the operand in key
+above, reduce-then-scan passes on X's free bits alone above 2^21 (pairs of 10- and
+11-bit digits above 2^18 and 2^16).  The plan's contraction with a permutation returns the operand in key
 order, so the sorted keys and values are checked exactly."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -32,3 +35,19 @@ def test_operand_order_and_values(gpu, n, wide):
     for a, b in zip(idx, X.idx):
         np.testing.assert_array_equal(a.astype(np.int64), b[o].astype(np.int64))
     np.testing.assert_array_equal(v, X.val[o])
+
+
+@pytest.mark.parametrize("n,rb", [(1 << 18, 10), ((1 << 18) + 1, 10), (1 << 16, 11),
+                                  ((1 << 16) + 1, 11), (3073, 10), (3073, 11)])
+def test_wide_digits_on_both_sides_of_their_line(gpu, n, rb):
+    import torch
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 1 << 33, n).astype(np.int64) >> rng.integers(0, 30, n)
+    k = torch.from_numpy(keys).cuda()
+    v = torch.arange(n, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    sptc.check(sptc.lib().sptc_sort_pairs(ctypes.c_void_p(k.data_ptr()),
+                                          ctypes.c_void_p(v.data_ptr()), n, 33, rb, None))
+    o = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k.cpu().numpy(), keys[o])
+    np.testing.assert_array_equal(v.cpu().numpy(), o.astype(np.float32))
