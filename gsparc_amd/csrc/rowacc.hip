@@ -49,10 +49,23 @@ constexpr uint64_t kItemProds = 7168;
 // ... and products per owner of an item, below which the owner table costs
 // more than the products.
 constexpr uint64_t kItemRun = 4;
-// An item is one workgroup's.  A chunk holding one of more products than this
-// (and than a 1024th of the chunk) -- long rows over few columns, or of very
-// many owners -- goes to the product sort, which spreads a row over the chip.
+// An item is one workgroup's: it takes about 1.7 ns a product and 19 ns an owner
+// (one row over few columns, 1e6 products of owners with 100 each 2.0 ms, with 1 each
+// 21 ms), so an owner weighs as much as kOwnerWeight products.  A chunk with a heavy
+// item -- long rows over few columns, or of very many owners -- goes to the product
+// sort, which spreads a row over the chip.  Two lines:
+//   weight above kHeavyWeight and a 64th of the chunk's products: the item alone
+//     outlasts what the sort takes longer (0.13 ms and 0.03 ns a product of long
+//     rows).  20 rows of owners with 100 products meet the sort at 1e5 products each
+//     (385 us against 423 with 0.65e5, 504 / 453 with 1.3e5), with 5 at 0.25e5 (388 /
+//     442 with 0.16e5, 744 / 559 with 0.65e5), with 1 below 0.16e5 (686 / 511); 250
+//     rows of 1.3e5 products: 517 / 961;
+//   products above kHeavyItem and a 1024th of the chunk's: among short rows, where
+//     the sort is no slower, an item is all that differs (1.5e5 products in one row
+//     beside 2e7 in short ones: 1185 us against 921).
 constexpr uint64_t kHeavyItem = 1ull << 17;
+constexpr uint64_t kHeavyWeight = 5ull << 14;
+constexpr uint64_t kOwnerWeight = 11;
 
 // Slab bounds follow the products: columns that occur often in Y hold most of
 // a row's products (the first quarter of the benchmark's columns 61 %), so
@@ -142,7 +155,7 @@ template <bool ACT>
 struct RowKindOp {
   RowAccArgs a;
   uint32_t least;
-  uint64_t heavy;  // products of an item that one workgroup should not be given
+  uint64_t heavy, weight;  // products, and weight, that one workgroup should not be given
   uint64_t* flag;  // pinned host memory
   uint32_t *live_row, *live_cnt;
   uint64_t* live_src;
@@ -175,7 +188,9 @@ struct RowKindOp {
       live_cnt[k] = 0;  // k_ra_count adds
       live_src[k] = kLongSrc;
       const uint64_t n = a.row_prod[r + 1] - a.row_prod[r];
-      if (n / row_slabs(n, a.row_act[r + 1] - a.row_act[r], a.K, least) > heavy) *flag = 1;
+      const uint64_t own = a.row_act[r + 1] - a.row_act[r];
+      const uint64_t prods = n / row_slabs(n, own, a.K, least);
+      if (prods > heavy || prods + kOwnerWeight * own > weight) *flag = 1;
     } else {
       live_cnt[k] = (uint32_t)(a.row_prod[r + 1] - a.row_prod[r]);
       live_src[k] = a.row_act[r];
@@ -1241,10 +1256,11 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   // (items: long rows hold more than 256 products)
   room(p->tmp, scan_tmp_count(std::max(rows, nprod / 256 * least + nprod / kItemProds)) + 1, s);
   const uint64_t heavy = std::max(kHeavyItem, nprod >> 10);
+  const uint64_t weight = kHeavyWeight + (nprod >> 6);
   host[1].a = 0;
   auto kinds = [&](auto op) {
-    op = {a, least, heavy, &host[1].a, p->live_row.get(), p->live_cnt.get(), p->live_src.get(),
-          p->s_live.get(), p->s_prod.get(), p->l_live.get()};
+    op = {a, least, heavy, weight, &host[1].a, p->live_row.get(), p->live_cnt.get(),
+          p->live_src.get(), p->s_live.get(), p->s_prod.get(), p->l_live.get()};
     run_scan(op, rows, p->tmp.get(), s, true, host);
   };
   if (by_act) kinds(RowKindOp<true>{});

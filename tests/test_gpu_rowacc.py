@@ -105,6 +105,21 @@ def test_heavy_row_goes_to_the_product_sort(gpu):
     check(*build(rng, 1000, [[900] * 300, [5, 6], [700]]))
 
 
+@pytest.mark.parametrize("rows,owners,per,K,sorted_", [
+    (1, 6000, 1, 40, False), (1, 8000, 1, 40, True), (1, 75, 1000, 1000, False),
+    (1, 85, 1000, 1000, True), (30, 85, 1000, 1000, False), (30, 135, 1000, 1000, True),
+    (2, 12_000, 2, 40, True),
+    (1, 3000, 8, 70_000, False), (1, 20_000, 2, 70_000, True)])
+def test_heavy_items_on_both_sides_of_the_line(gpu, rows, owners, per, K, sorted_):
+    """An item's weight is its products and 11 per owner: above 81920 and a 64th of
+    the chunk's products the chunk takes the product sort, as above 2^17 products."""
+    rng = np.random.default_rng(owners)
+    X, Y = build(rng, K, [[per] * owners] * rows + [[5, 6]], signed=True)
+    check(X, Y)
+    st = sptc.SpTC(X, Y, [1], [0], dense_accumulator=-1, kernel_timing=True).kernel_stats()
+    assert (st["sort_products"][0] + st["sort_products_wide"][0] > 0) == sorted_
+
+
 def test_fallback_chunk_beside_others_under_a_budget(gpu):
     """A budget that cuts the products into chunks; the first holds a row that
     sends it to the product sort, the others take the row accumulator.  The
