@@ -175,7 +175,7 @@ void launch_bany_dup(const uint64_t* keys, const uint64_t* seg_off, uint32_t nse
 void launch_digest(const uint64_t* keys, uint64_t n, uint64_t* out, hipStream_t s);
 void launch_check_digest(const uint64_t* got, const uint64_t* want, uint32_t* bad,
                          hipStream_t s);
-// *out += sum of vals[0, n) in FP64.
+// A run of values of instance `inst`.
 struct SumSlice {
   const float* v;
   uint64_t n;

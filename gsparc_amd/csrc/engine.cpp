@@ -341,7 +341,7 @@ void Engine::prepare(const StagedCOO& t, const Layout& lay, Operand* out, const 
   // passes (1e6 nonzeros, 1.7e9 products: 11.57 ms unsorted, 11.38 sorted).
   const int lo = lay.role == 1 && n > kOnesweepMax ? lay.ncbits : 0;
   int tok = kt_.begin(s_);
-  if (!rb_ && sort_linearize_small(a, t.idx_bytes, t.val, n, out->keys.get(), out->vals.get(), lo,
+  if (!rb_ && sort_linearize_small(a, t.idx_bytes, t.val, n, out->keys.get(), out->vals.get(),
                                    s_)) {
     kt_.end(tok, SPTC_K_LINEARIZE, (double)n * (lay.order * t.idx_bytes + 16), s_);
     return;
@@ -536,7 +536,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
   uint64_t* const hdup = &words_->dup;
   *hdup = 0;
   const int tbits = ytable_bits(ncb, ny);
-  DevBuf<U2> tmem((1ull << tbits) + 1);
+  DevBuf<U2> tmem(1ull << tbits);
   const YTable tab = build_ytable(tmem.get(), tbits, Y.keys.get(), ny, ncb, ynf, s_, hdup);
   DevBuf<uint64_t> act_prefix(nx + 1), act_ypos(nx + 1), row_key(nx + 1), row_prod(nx + 1),
       row_act(nx + 1);

@@ -122,8 +122,9 @@ bool prefer_row_sort();
 // bits allow; by default they are sorted on all column bits.
 bool prefer_bucket_tail();
 
-// Chunks over column spaces of at most kRowAccMaxBits take the row accumulator
-// (rowacc.hpp) unless a variant of the product sort is asked for
+// Chunks take the row accumulator (rowacc.hpp) where it applies (column ranks below
+// 2^31; long rows only over at most kRowAccMaxBits of them; no heavy item) unless a
+// variant of the product sort is asked for
 // (SPTC_PROD_SORT, SPTC_BIG_TAIL, SPTC_SEG_RB, SPTC_SEG_IPT, SPTC_SEG_WIDE).
 bool prefer_row_acc();
 

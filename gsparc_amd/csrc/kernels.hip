@@ -186,12 +186,11 @@ void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* key
 // range of c's starts and ends among the keys; ranges of one c need no more,
 // others compare the range's first and last key and search between them.
 
-// dup / hdup (device / pinned host, may be NULL; cleared by the caller): set
-// when two Y keys are equal.
+// hdup (pinned host memory, may be NULL; cleared by the caller): set when two Y
+// keys are equal.
 __global__ __launch_bounds__(kBlock) void k_ytable(const uint64_t* __restrict__ ykeys, uint64_t ny,
                                                    int ynf, int sh, uint64_t K,
-                                                   U2* __restrict__ tab, uint64_t* dup,
-                                                   uint64_t* hdup) {
+                                                   U2* __restrict__ tab, uint64_t* hdup) {
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   bool same = false;
@@ -204,21 +203,18 @@ __global__ __launch_bounds__(kBlock) void k_ytable(const uint64_t* __restrict__ 
     if (i == 0 || shr64(shr64(prev, ynf), sh) != h) tab[h].a = i;
     if (i == ny - 1 || shr64(shr64(next, ynf), sh) != h) tab[h].b = i + 1;
   }
-  if (dup && __ballot(same) && lane_id() == 0) {
-    *dup = 1;
-    *hdup = 1;
-  }
+  if (hdup && __ballot(same) && lane_id() == 0) *hdup = 1;
 }
 
 YTable build_ytable(U2* tab, int bits, const uint64_t* ykeys, uint64_t ny, int ncbits, int ynf,
                     hipStream_t s, uint64_t* hdup) {
   const uint64_t K = 1ull << bits;
   YTable t{tab, ykeys, ny, ncbits - bits, ynf};
-  fill_u64(reinterpret_cast<uint64_t*>(tab), 0, 2 * K + (hdup ? 1 : 0), s);
+  fill_u64(reinterpret_cast<uint64_t*>(tab), 0, 2 * K, s);
   if (!ny) return t;
   const uint32_t grid = (uint32_t)std::min<uint64_t>(ceil_div(ny, kBlock), 4096);
   hipLaunchKernelGGL(k_ytable, dim3(grid), dim3(kBlock), 0, s, ykeys, ny, ynf, t.sh, K, tab,
-                     hdup ? &tab[K].a : nullptr, hdup);
+                     hdup);
   return t;
 }
 

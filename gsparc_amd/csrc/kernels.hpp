@@ -103,16 +103,17 @@ struct DenseArgs {
 };
 
 constexpr int kDenseMaxBits = 13;  // dense LDS rows up to 8192 slots
-// The dense kernels spread one active X nonzero's Y segment over a 256-thread
-// workgroup at a time; below this many products per active nonzero most
-// threads idle and ESC is faster (measured: ~3e9 products/s at 3-4 per
-// nonzero, against ~1e10 for ESC on the same instances).
+// Products per active X nonzero below which ESC is taken.  5e4 rows of 5 owners over
+// 1000 columns, dense against ESC: 491 us / 299 with 4 products per owner, 348 / 327
+// with 8, 372 / 385 with 16, 400 / 485 with 32.  (5e3 rows: 208 / 250 with 4.)
 constexpr uint64_t kDenseMinRun = 16;
-// The ordered dense pass applies a round's owners (active X nonzeros) one
-// after another, a barrier between them, and a row is one workgroup: rows
-// with many owners serialise on those barriers.  On the batched workload's
-// 57 dense-eligible instances dense won (0.74-0.99x of ESC's time) up to 5.1
-// owners per row and lost from 5.5 on (1.03x, up to 2.9x at 4000 per row).
+// Owners (active X nonzeros) per row up to which dense is chosen.  The line was drawn
+// for a pass that added owner by owner, and is not where the two meet now: the same
+// rows with 16 products per owner take 372 us / 385 with 5 owners, 416 / 455 with 8,
+// 546 / 661 with 16; eight batched instances of 2000 rows with 32 products per owner
+// 276 / 243 with 1, 325 / 341 with 5, 588 / 1172 with 64.  Nor does it know the
+// columns: over 8000 of them, 2 owners of 400 products, 500 rows take 206 us / 255,
+// 5e3 355 / 387, 5e4 1464 / 815.
 constexpr uint64_t kDenseMaxOwnersPerRow = 5;
 // The automatic choice (single and batched planners alike): dense when its
 // rows are dense enough for the slots (ir * 32 >= rows * slots), the Y
@@ -132,9 +133,9 @@ void run_row_count_scan(const uint32_t* cnt, uint64_t* off, uint64_t n, U2* tmp,
 
 void launch_linearize(const LinArgs& a, int idx_bytes, uint64_t n, uint64_t* keys,
                       uint64_t* hist, int passes, int rb, hipStream_t s, int lo = 0);
-// Fills and builds the table in tab[0 .. 2^bits - 1] (bits from ytable_bits).  With
-// hdup (pinned host memory, cleared by the caller) the entry after it holds the
-// duplicate flag: both are set when two Y keys are equal.
+// Fills and builds the table in tab[0 .. 2^bits - 1] (bits from ytable_bits).  hdup
+// (pinned host memory, cleared by the caller; may be NULL) is set when two Y keys are
+// equal.
 YTable build_ytable(U2* tab, int bits, const uint64_t* ykeys, uint64_t ny, int ncbits, int ynf,
                     hipStream_t s, uint64_t* hdup = nullptr);
 // look (may be NULL): scratch of 2 * nx words for what the lookups find; without

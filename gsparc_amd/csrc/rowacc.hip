@@ -858,7 +858,7 @@ struct GroupSort {            // while they are sorted
   TileSmem<10, kGroupIPT, kGroupNT, KT> t;
   float v[kGroupTile];
 };
-constexpr uint32_t kGroupRows = kGroupHalf + 1;  // rows hold two products at least
+constexpr uint32_t kGroupRows = kGroupHalf + 1;  // rows hold a product at least
 
 // One workgroup per group of short rows: their owners are staged (a lane
 // each), every product finds its owner by an LDS search, makes its key (row

@@ -172,61 +172,55 @@ __global__ __launch_bounds__(kOneNT) void k_scan_one(Op op, uint32_t n, bool emi
   __shared__ U2 scratch[kOneNT / kWave];
   __shared__ U2 sv[kOneTile];
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-  U2 carry = mk2(0, 0);
-  for (uint32_t base = 0; base < n; base += (uint32_t)kOneTile) {
-    U2 vals[kOneItems];
-    typename ScanAux<Op>::type aux[kOneItems];
+  U2 vals[kOneItems];
+  typename ScanAux<Op>::type aux[kOneItems];
+#pragma unroll
+  for (int e = 0; e < kOneItems; ++e) {
+    const uint32_t i = (uint32_t)e * kOneNT + tid;
+    vals[e] = i < n ? scan_value(op, (uint64_t)i, aux[e]) : mk2(0, 0);
+    sv[i] = vals[e];
+  }
+  __syncthreads();
+  U2 mine[kOneItems];
+  U2 t = mk2(0, 0);
+#pragma unroll
+  for (int e = 0; e < kOneItems; ++e) {
+    mine[e] = sv[tid * kOneItems + e];
+    t = t + mine[e];
+  }
+  U2 inc = t;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint64_t oa = __shfl_up(inc.a, d, kWave), ob = __shfl_up(inc.b, d, kWave);
+    if (lane >= (uint32_t)d) inc = inc + mk2(oa, ob);
+  }
+  if (lane == kWave - 1) scratch[wave] = inc;
+  __syncthreads();
+  U2 excl = inc - t, all = mk2(0, 0);
+  for (uint32_t w = 0; w < (uint32_t)(kOneNT / kWave); ++w) {
+    const U2 x = scratch[w];
+    if (w < wave) excl = excl + x;
+    all = all + x;
+  }
+#pragma unroll
+  for (int e = 0; e < kOneItems; ++e) {
+    sv[tid * kOneItems + e] = excl;
+    excl = excl + mine[e];
+  }
+  __syncthreads();
+  if (emit) {
 #pragma unroll
     for (int e = 0; e < kOneItems; ++e) {
-      const uint32_t i = base + (uint32_t)e * kOneNT + tid;
-      vals[e] = i < n ? scan_value(op, (uint64_t)i, aux[e]) : mk2(0, 0);
-      sv[e * kOneNT + tid] = vals[e];
-    }
-    __syncthreads();
-    U2 mine[kOneItems];
-    U2 t = mk2(0, 0);
-#pragma unroll
-    for (int e = 0; e < kOneItems; ++e) {
-      mine[e] = sv[tid * kOneItems + e];
-      t = t + mine[e];
-    }
-    U2 inc = t;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const uint64_t oa = __shfl_up(inc.a, d, kWave), ob = __shfl_up(inc.b, d, kWave);
-      if (lane >= (uint32_t)d) inc = inc + mk2(oa, ob);
-    }
-    if (lane == kWave - 1) scratch[wave] = inc;
-    __syncthreads();
-    U2 excl = carry + inc - t;
-    for (uint32_t w = 0; w < (uint32_t)(kOneNT / kWave); ++w) {
-      const U2 x = scratch[w];
-      if (w < wave) excl = excl + x;
-      carry = carry + x;
-    }
-#pragma unroll
-    for (int e = 0; e < kOneItems; ++e) {
-      sv[tid * kOneItems + e] = excl;
-      excl = excl + mine[e];
-    }
-    __syncthreads();
-    if (emit) {
-#pragma unroll
-      for (int e = 0; e < kOneItems; ++e) {
-        const uint32_t i = base + (uint32_t)e * kOneNT + tid;
-        if (i < n) {
-          if constexpr (ScanAux<Op>::on)
-            op.emit((uint64_t)i, sv[e * kOneNT + tid], vals[e], aux[e]);
-          else
-            op.emit((uint64_t)i, sv[e * kOneNT + tid], vals[e]);
-        }
+      const uint32_t i = (uint32_t)e * kOneNT + tid;
+      if (i < n) {
+        if constexpr (ScanAux<Op>::on) op.emit((uint64_t)i, sv[i], vals[e], aux[e]);
+        else op.emit((uint64_t)i, sv[i], vals[e]);
       }
     }
-    __syncthreads();
   }
   if (tid == 0) {
-    *total = carry;
-    if (host) *host = carry;
+    *total = all;
+    if (host) *host = all;
   }
 }
 

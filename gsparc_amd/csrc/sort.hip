@@ -8,8 +8,8 @@
 //     LDS in digit order and written out in coalesced digit runs -- keys
 //     first, then values through the same LDS buffer.  Longer digit runs per
 //     tile (bigger tiles) are what make the scatter efficient.
-//   * Two ways to find each tile's global digit offsets:
-//       reduce-then-scan (default): an upsweep writes per-tile digit counts
+//   * Two ways to find each tile's global digit offsets, by size (sort_onesweep):
+//       reduce-then-scan (large sorts): an upsweep writes per-tile digit counts
 //       into a digit-major matrix whose exclusive scan, in memory order, is
 //       every tile's start for every digit; no inter-tile waits.
 //       onesweep: a single kernel per pass with decoupled look-back over
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(NT) void k_onesweep(
 constexpr int kSmallNT = 512, kSmallIPT = 12, kSmallRB = 8;
 template <typename IdxT>
 __global__ __launch_bounds__(kSmallNT) void k_sort_small(LinArgs a, const float* __restrict__ val,
-                                                         uint32_t n, int first_bit,
+                                                         uint32_t n,
                                                          uint64_t* __restrict__ keys,
                                                          float* __restrict__ vals) {
   constexpr int RB = kSmallRB, IPT = kSmallIPT, NT = kSmallNT, R = 1 << RB;
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(kSmallNT) void k_sort_small(LinArgs a, const float*
     o |= s_or[w];
     an &= s_and[w];
   }
-  const uint64_t vary = o & ~an & ~low_mask(first_bit);
+  const uint64_t vary = o & ~an;
   const int lo = vary ? __builtin_ctzll(vary) : 0, hi = vary ? 64 - __builtin_clzll(vary) : 0;
   for (int shift = lo; shift < hi; shift += RB) {
     if (!((vary >> shift) & (R - 1))) continue;  // a digit that all keys share
@@ -499,13 +499,13 @@ void SortWorkspace::prepare(uint64_t n, hipStream_t s) {
 }
 
 bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
-                          uint64_t* keys, float* vals, int lo, hipStream_t s) {
+                          uint64_t* keys, float* vals, hipStream_t s) {
   if (n > (uint64_t)kSmallNT * kSmallIPT || sort_cfg().mode) return false;
   if (idx_bytes == 4)
-    hipLaunchKernelGGL(k_sort_small<uint32_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n, lo,
+    hipLaunchKernelGGL(k_sort_small<uint32_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
                        keys, vals);
   else
-    hipLaunchKernelGGL(k_sort_small<uint64_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n, lo,
+    hipLaunchKernelGGL(k_sort_small<uint64_t>, dim3(1), dim3(kSmallNT), 0, s, a, val, (uint32_t)n,
                        keys, vals);
   return true;
 }
@@ -528,8 +528,8 @@ void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
 
 // vals NULL: the keys alone are moved; vsrc: the values are read from there
 // instead of vals (which the second pass writes).
-// Sorts keys/vals (n <= ws.cap, n < 2^32) on bits [lo, nbits).  With the
-// onesweep algorithm ws.hist must hold the digit histograms of all passes.
+// Sorts keys/vals (n that ws was ensured for, below 2^32) on bits [lo, nbits).  With
+// the onesweep algorithm ws.hist must hold the digit histograms of all passes.
 // Result ends in (keys, vals) when the pass count is even, else in
 // (ws.alt_keys, ws.alt_vals); the returned flag says which (true = alt).
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,

@@ -73,17 +73,18 @@ constexpr uint64_t onesweep_max(int rb) {
   return rb <= 9 ? kOnesweepMax : rb == 10 ? 1ull << 18 : 1ull << 16;
 }
 bool sort_onesweep(uint64_t n, int rb);
-// Linearizes and sorts up to one tile of nonzeros in one launch, on bits [lo, 64);
-// false when there are more.
+// Linearizes and sorts up to one tile of nonzeros in one launch; false when there
+// are more.
 bool sort_linearize_small(const LinArgs& a, int idx_bytes, const float* val, uint64_t n,
-                          uint64_t* keys, float* vals, int lo, hipStream_t s);
+                          uint64_t* keys, float* vals, hipStream_t s);
 // Digit width for a sort over nbits key bits (fewest passes, digits <= 10).
 int choose_radix_bits(int nbits);
 void histogram(const SortWorkspace& ws, const uint64_t* keys, uint64_t n,
                int passes, hipStream_t s, int lo = 0);
-// Sorts (keys, vals), stably, on bits [lo, nbits), ws.hist() holding the histograms of
-// all passes for sizes that sort_onesweep.  Returns true when the sorted data ended in (ws.alt_keys,
-// ws.alt_vals) (odd pass count).
+// Sorts (keys, vals), stably, on bits [lo, nbits), ws.hist() holding the histograms
+// of all passes for sizes that sort_onesweep.  vals NULL: the keys alone are moved;
+// vsrc: the first pass reads the values there.  Returns true when the sorted data
+// ended in (ws.alt_keys, ws.alt_vals) (odd pass count).
 // kt (optional) times every pass under kernel class `cls`.
 bool sort_after_histogram(SortWorkspace& ws, uint64_t* keys, float* vals,
                           uint64_t n, int nbits, hipStream_t s, KTimer* kt = nullptr,
