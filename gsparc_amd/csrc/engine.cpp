@@ -825,12 +825,14 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
     // row accumulator (a tight budget keeps to the product sort, whose parts the
     // chunks are sized for)
     bool rowacc = kyf > 0 && kyf < 32 && prefer_row_acc() && !partition_only;
+    uint64_t max_live = 0, acc_bytes = 0;
     if (rowacc && chunk_cap) {
       uint64_t max_act = 0;
       for (size_t c = 1; c < bounds_a.size(); ++c)
         max_act = std::max(max_act, bounds_a[c] - bounds_a[c - 1]);
-      const uint64_t held = DevicePool::get().live_bytes();
-      rowacc = held + rowacc_bytes(max_rows, max_act, chunk_cap, ranks) + out_per * ir <= budget_;
+      max_live = std::min(max_rows, max_act);
+      acc_bytes = rowacc_bytes(max_rows, max_act, chunk_cap, ranks);
+      rowacc = DevicePool::get().live_bytes() + acc_bytes + out_per * ir <= budget_;
     }
     RowAccArgs ra;
     if (rowacc) {
@@ -867,10 +869,7 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
       bool done = false;
       uint64_t out_n = 0;
       if (rowacc && kA.size() &&
-          DevicePool::get().live_bytes() +
-                  rowacc_bytes(r1c - r0c, bounds_a[c] - bounds_a[c - 1], n, ranks) +
-                  out_per * (ir - P0) >
-              budget_) {
+          DevicePool::get().live_bytes() + acc_bytes + out_per * (ir - P0) > budget_) {
         // an earlier chunk fell back and the chunks are sized for either, not both
         SPTC_HIP(hipStreamSynchronize(s_));
         kA.release();
@@ -884,10 +883,12 @@ sptc_status Engine::contract(const Operand& X, const Operand& Y, sptc_result_s* 
         ra.r0 = r0c;
         ra.a0 = bounds_a[c - 1];
         ra.rows = r1c - r0c;
+        rplan.rows_at_most = max_live;
+        rplan.prods_at_most = chunk_cap;
         done = rowacc_count(ra, n, bounds_a[c] - bounds_a[c - 1], o_.count_only, &rplan,
                             words_->acc, s_, &kt_);
         out_n = rplan.outs;
-        if (!done) rplan = RowAccPlan();
+        if (!done) rplan = RowAccPlan();  // (waited for)
       }
       std::function<void(OutChunk&)> emit;
       if (done) {

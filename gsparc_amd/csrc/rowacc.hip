@@ -1218,12 +1218,10 @@ NearArgs near_args(const RowAccArgs& a, const RowAccPlan& p) {
 }
 
 // A buffer that grows goes back to the pool, where another thread may take it for
-// its own stream: the kernels of the chunk before are waited for first.
+// its own stream: no launch may be under way.
 template <class T>
-void room(DevBuf<T>& b, uint64_t n, hipStream_t s) {
-  if (b.size() >= n) return;
-  if (b.size()) SPTC_HIP(hipStreamSynchronize(s));
-  b.reset(n);
+void room(DevBuf<T>& b, uint64_t n) {
+  if (b.size() < n) b.reset(n);
 }
 
 }  // namespace
@@ -1244,17 +1242,27 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   const bool by_act = owners < a.rows;
   const uint64_t rows = by_act ? owners : a.rows;
   if (nprod >= (1ull << 32)) throw std::length_error("row accumulator chunk");
-  room(p->live_row, rows, s);
-  room(p->live_cnt, rows, s);
-  room(p->live_src, rows, s);
-  room(p->s_live, rows, s);
-  room(p->s_prod, rows, s);
-  room(p->l_live, rows, s);
   // (column spaces too wide to cut into slabs take no long rows)
   const bool slabs = a.K <= 1u << kRowAccMaxBits;
   const uint32_t least = slabs ? min_slabs(a.K) : 1;
   // (items: long rows hold more than 256 products)
-  room(p->tmp, scan_tmp_count(std::max(rows, nprod / 256 * least + nprod / kItemProds)) + 1, s);
+  const uint64_t ntmp =
+      scan_tmp_count(std::max(rows, nprod / 256 * least + nprod / kItemProds)) + 1;
+  if (p->live_row.size() < rows || p->tmp.size() < ntmp) {
+    // the chunk before may still use them; with this chunk's sizes the largest
+    // (the engine says so) this happens once
+    if (p->tmp.size()) SPTC_HIP(hipStreamSynchronize(s));
+    const uint64_t r = std::max(rows, p->rows_at_most);
+    room(p->live_row, r);
+    room(p->live_cnt, r);
+    room(p->live_src, r);
+    room(p->s_live, r);
+    room(p->s_prod, r);
+    room(p->l_live, r);
+    room(p->tmp, std::max(ntmp, scan_tmp_count(std::max(r, p->prods_at_most / 256 * least +
+                                                               p->prods_at_most / kItemProds)) +
+                                    1));
+  }
   const uint64_t heavy = std::max(kHeavyItem, nprod >> 10);
   const uint64_t weight = kHeavyWeight + (nprod >> 6);
   host[1].a = 0;
@@ -1279,11 +1287,31 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   const uint64_t max_items = p->nlong * least + nprod / kItemProds;
   const uint64_t max_split = owners * (least + 1) + nprod / kItemRun;
   if (max_split >= (1ull << 32)) return false;  // 32-bit places in the descriptors
+  // the bitmaps are kept from the count to the sum while they take no more
+  // than a few bytes per product (one write and one read of K / 8 bytes per
+  // row against another gather and LDS atomic per product)
+  const uint64_t max_words = p->nlong * (a.K / 64 + 1) + max_items;
+  p->keep_words = !count_only && max_words * 8 <= 4 * nprod + (1ull << 20);
+  // (all tables, while nothing runs)
+  if (!count_only) {
+    room(p->tcol, p->short_prods);
+    room(p->tval, p->short_prods);
+  }
+  if (p->nlong) {
+    room(p->l_item, p->nlong + 1);
+    room(p->l_split, p->nlong);
+    room(p->l_word, p->nlong);
+    room(p->item, max_items * (kItemBytes / 4));
+    room(p->item_cnt, max_items);
+    room(p->split, max_split);
+    if (p->keep_words) room(p->words, max_words);
+  }
+  const bool new_quant = p->nlong && !p->quant.size();
+  if (new_quant) p->quant.reset(kQuant + 1);
+  room(p->l_near, p->live);
+  room(p->near_pre, p->live);
+  room(p->near, p->live * (kNearBytes / 8));
   if (p->nshort) {
-    if (!count_only) {
-      room(p->tcol, p->short_prods, s);
-      room(p->tval, p->short_prods, s);
-    }
     GroupArgs g{a,
                 p->live_row.get(),
                 p->s_live.get(),
@@ -1303,26 +1331,12 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
     kt->end(tok, SPTC_K_SORT_LOCAL, (count_only ? 8.0 : 16.0) * (double)p->short_prods, s);
   }
   if (p->nlong) {
-    // the bitmaps are kept from the count to the sum while they take no more
-    // than a few bytes per product (one write and one read of K / 8 bytes per
-    // row against another gather and LDS atomic per product)
-    const uint64_t max_words = p->nlong * (a.K / 64 + 1) + max_items;
-    p->keep_words = !count_only && max_words * 8 <= 4 * nprod + (1ull << 20);
-    room(p->l_item, p->nlong + 1, s);
-    room(p->l_split, p->nlong, s);
-    room(p->l_word, p->nlong, s);
-    room(p->item, max_items * (kItemBytes / 4), s);
-    room(p->item_cnt, max_items, s);
-    room(p->split, max_split, s);
-    if (p->keep_words) room(p->words, max_words, s);
     SlabOp slab{a, least, p->l_live.get(), p->live_row.get(), p->nlong, p->l_item.get(),
                 p->l_split.get(), p->l_word.get()};
     run_scan(slab, p->nlong, p->tmp.get(), s, true, host + 2);
-    if (!p->quant.size()) {
-      p->quant.reset(kQuant + 1);
+    if (new_quant)
       hipLaunchKernelGGL(k_ra_quant, dim3(1), dim3(kQuantNT), 0, s, a.ycol, a.ny, a.K,
                          p->quant.get());
-    }
     hipLaunchKernelGGL(k_ra_items, dim3(grid_of(ceil_div(max_items, kBlock), 2048)), dim3(kBlock),
                        0, s, a, p->l_live.get(), p->live_row.get(), p->l_item.get(),
                        p->l_split.get(), p->l_word.get(), p->quant.get(), p->nlong,
@@ -1340,9 +1354,6 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
                          p->item_cnt.get());
     kt->end(tok, SPTC_K_REDUCE, (count_only ? 8.0 : 4.0) * (double)(nprod - p->short_prods), s);
   }
-  room(p->l_near, p->live, s);
-  room(p->near_pre, p->live, s);
-  room(p->near, p->live * (kNearBytes / 8), s);
   OutOp out{a,
             p->live_cnt.get(),
             p->live_row.get(),
@@ -1356,6 +1367,7 @@ bool rowacc_count(const RowAccArgs& a, uint64_t nprod, uint64_t owners, bool cou
   p->near_rows = host[0].b >> 32;
   p->near_outs = host[0].b & 0xFFFFFFFFull;
   if (p->nlong) p->items = host[2].a & 0xFFFFFFFFull;
+  if (!count_only) room(p->item_off, p->items);
   if (count_only && p->near_outs) {
     const uint32_t nt = (uint32_t)ceil_div(p->near_outs, kNearTile);
     const int tok = kt->begin(s);
@@ -1379,7 +1391,6 @@ void rowacc_emit(const RowAccArgs& a, RowAccPlan& p, uint64_t nprod, uint32_t* o
     kt->end(tok, SPTC_K_EXPAND, 24.0 * (double)p.near_outs, s);
   }
   if (p.items) {
-    room(p.item_off, p.items, s);
     const int tok = kt->begin(s);
     ItemOutOp op{p.item_cnt.get(), reinterpret_cast<const Item*>(p.item.get()), p.l_near.get(),
                  p.item_off.get()};

@@ -52,6 +52,8 @@ struct RowAccArgs {
 // summed slab by slab.
 constexpr uint64_t kItemBytes = 32, kNearBytes = 24;
 struct RowAccPlan {
+  // most rows with products and most products of the call's chunks (0: unknown)
+  uint64_t rows_at_most = 0, prods_at_most = 0;
   uint64_t live = 0, nshort = 0, nlong = 0;  // rows
   uint64_t short_prods = 0;
   uint64_t items = 0;                        // long rows' slabs (after count)
