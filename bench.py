@@ -694,7 +694,7 @@ def self_check(X, spec, r):
            "value_sum_closed_form": vs_cf, "emitted_value_sum": emitted,
            "order_violations": bad}
     # positive values: FP32-rounded products sum within u32 of the exact
-    # checksum, compensated FP32 output sums within about 3 u32
+    # checksum, output sums rounded once more within 2 u32
     ok = (r.ir_nnz == ir_cf and abs(r.info.value_sum - vs_cf) <= 2 * u32 * vs_cf
           and abs(emitted - vs_cf) <= 6 * u32 * vs_cf and bad == 0)
     out["ok"] = bool(ok)

@@ -5,10 +5,9 @@
 // columns are d << low .. (d + 1) << low - 1, in expansion order (the pass is
 // stable).  A bucket's columns fit an LDS row, so it is reduced there instead
 // of being sorted on its low bits: each product is added to its column's
-// FP64 slot in product order (products of one
-// column in the same 64-product window are applied lowest lane first), the
-// touched slots are marked in a bitmap and emitted in column order.  The sums
-// are those of the fully sorted path (same values, same order, same steps),
+// FP64 slot in product order (products of one column in the same 64-product
+// window are applied lowest lane first), the touched slots are marked in a bitmap and emitted in column order.  The sums
+// are those of the fully sorted path (same values, added in the same order),
 // so the outputs agree bit for bit.
 //
 // An option (SPTC_BIG_TAIL=buckets): on the NIPS workload it replaces the

@@ -170,7 +170,9 @@ __device__ __forceinline__ T block_excl_scan(T v, T* scratch, T* total) {
 // every path.  A product holds 24 bits, so the FP64 sum is exact while the
 // products of one output span less than 2^29 / count in magnitude: the order
 // of the adds then does not matter, and sums taken in product order
-// (reduce), by LDS atomics (dense rows) or by window agree bit for bit.
+// (reduce), by LDS atomics (dense rows, the row accumulator's long rows) or by
+// window agree bit for bit, on every run.  Otherwise they agree to FP64 rounding,
+// and those by atomics, which have no fixed order, may differ from run to run.
 // (One add and a conversion per product; the compensated FP32 pair that it
 // replaced took seven operations and, like it, an ordered pass to be
 // reproducible.)

@@ -58,7 +58,8 @@ void split_operand(const sptc_coo& t, const Layout& lay, int parts, bool own,
 // convert_and_sort_64), contracted with the X part, and the pair results
 // are merged row by row into one chunk of the output (Y parts hold disjoint,
 // ascending column ranges, so a row's entries are its pieces in part
-// order).  Results are bit-identical to the unpartitioned contraction.
+// order).  Results are the unpartitioned contraction's (bit for bit where the FP64
+// sums are exact, see SumF64).
 sptc_status contract_partitioned(Engine& e, const sptc_coo& X, const sptc_coo& Y,
                                  const Layout& xl, const Layout& yl, OperandSplit& xs,
                                  OperandSplit& ys, sptc_result_s* res);

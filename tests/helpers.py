@@ -134,8 +134,8 @@ def compare_with_oracle(X, Y, cx, cy, res, x_rows=None):
 # ---- closed forms of a contraction (exact index arithmetic in numpy) -------
 
 # FP32 unit roundoff.  With positive values an FP64 sum of FP32-rounded
-# products is within U32 (relative) of the exact sum, and a compensated FP32
-# sum of them within about 3 * U32.
+# products is within U32 (relative) of the exact sum, and that sum rounded to
+# FP32 within 2 * U32.
 U32 = 2.0 ** -24
 
 

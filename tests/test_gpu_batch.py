@@ -1,7 +1,7 @@
 """GPU parity of the batched path (sptc_batch_*): every instance of a batch
 must equal the golden fixtures and, bit for bit, the plain single-call path
-on the same operands -- indices, values, product counts and accumulator
-choice -- across eager replays and hipGraph replays."""
+on the same operands (whose FP64 sums are exact in any order) -- indices, values,
+product counts and accumulator choice -- across eager replays and hipGraph replays."""
 import numpy as np
 import pytest
 

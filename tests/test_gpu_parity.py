@@ -294,8 +294,9 @@ def test_dense_matches_golden(gpu, case):
 
 @pytest.mark.parametrize("seed", range(4))
 def test_dense_equals_esc_bitwise(gpu, seed):
-    """Both accumulators sum each output's products in the same order with the
-    same compensated FP32 steps: identical indices and identical bits."""
+    """Both accumulators give the FP64 sum of each output's products, rounded once.
+    The values here lie within a factor of 500, so those sums are exact in any
+    order: identical indices and identical bits."""
     rng = np.random.default_rng(500 + seed)
     X = random_coo(rng, (400, 300, 50), 80_000, positive=bool(seed % 2))
     Y = random_coo(rng, (50, 60, 90), 60_000, positive=bool(seed % 2))
@@ -323,7 +324,7 @@ def test_dense_above_an_lds_row_is_tiled(gpu):
 def test_duplicate_coordinates_sum_like_the_oracle(gpu):
     """The .tns reader keeps duplicate entries (io_manager.tpp:210-240); ESC
     sums their products like any equal keys; the LDS dense row refuses them
-    (its ordered adds assume distinct columns per owner), so -d 1 runs the
+    (it assumes distinct columns per owner), so -d 1 runs the
     tiled dense accumulator, which adds them like the reference's atomics."""
     rng = np.random.default_rng(10)
     X = random_coo(rng, (30, 20, 10), 1500)

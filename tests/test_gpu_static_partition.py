@@ -4,9 +4,9 @@ Operands whose device footprint exceeds half the memory budget are split
 into free-key ranges (the reference's FindPartitionNum / Partition /
 convert_and_sort_64, tensor_manager.tpp:32-61,633-798) and contracted pair
 by pair (the X x Y partition loop, sptc.cuh:42-81).  The result must be the
-unpartitioned one entry for entry and bit for bit: a row's products come
-from the same X nonzeros in the same order, and each output column from
-exactly one Y part.
+unpartitioned one entry for entry and, since the FP64 sums of these values are
+exact in any order, bit for bit: a row's products come from the same X nonzeros,
+and each output column from exactly one Y part.
 """
 import numpy as np
 import pytest

@@ -88,7 +88,7 @@ def test_order5_wide_self_contraction(gpu):
     assert res.info.ncbits == int(np.ceil(np.log2(3000)))  # rank of <= 3000 tuples
     _check(res, X, X, [1, 2], [1, 2])
     # the dense accumulator cannot apply (column space); ESC and the planned
-    # form give the same result bit for bit
+    # form give the same result bit for bit (values whose FP64 sums are exact)
     plan = sptc.Plan(X, X, [1, 2], [1, 2])
     for a, b in zip(plan.execute().to_host(), res.to_host()):
         np.testing.assert_array_equal(a, b)
