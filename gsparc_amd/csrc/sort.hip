@@ -35,6 +35,7 @@ namespace {
 constexpr uint64_t kFlagAgg = 1ull << 62;
 constexpr uint64_t kFlagPre = 2ull << 62;
 constexpr uint64_t kValMask = (1ull << 48) - 1;
+// Rounds of a look-back wait, each eight loads and a sleep: some 10 s at least.
 constexpr uint32_t kSpinLimit = 1u << 24;
 
 __device__ __forceinline__ uint64_t pack_status(uint64_t flag, uint32_t epoch,
